@@ -157,6 +157,36 @@ inline int prefill_splits(int T, int inner, int outer, int ncu)
     const int s = cap / tiles < nblk / 2 ? cap / tiles : nblk / 2;
     return s > 1 ? s : 1;
 }
+// Which tile a prefill launch takes: 0 for 64 tokens x 128 rows (split over K
+// where that fills idle CUs), 1 or 2 for the wide kernel's 128 tokens x 128 or
+// 256 rows.  The line between them is the estimated time of each, in us, from
+// its block columns and its tiles per CU u = tiles / CUs (c = u rounded up:
+// the busiest CU's tiles).  The coefficients are a least-squares fit of the
+// three kernels timed on MI355X at 640 shapes (1 to 2048 tokens, 256 to 14336
+// rows, 1024 to 12288 columns; relative rms 7-10 %); over the 326 of them
+// without a split the choice is 0.01 % from the fastest on average and never
+// over 1 % slower than 64 x 128.  Examples, us (64 x 128 / 128 x 128 /
+// 128 x 256): 512 x 4096 x 4096 26.6 / 35.2 / 51.5, 192 x 12288 x 4096 44.5 /
+// 34.7 / 51.0, 1024 x 4096 x 4096 48.2 / 39.6 / 52.6, 1024 x 14336 x 4096 154.9
+// / 119.6 / 109.9.
+constexpr int kPrefillWideBM = 128;
+inline double prefill_cost(int tiles, int nblk, int ncu, double fixed, double col, double per_u, double per_c)
+{
+    const double u = (double)tiles / ncu, c = (double)((tiles + ncu - 1) / ncu);
+    return fixed + nblk * (col + per_u * u + per_c * c);
+}
+inline int prefill_wide_rows(int T, int inner, int outer, int ncu)
+{
+    const int nblk = inner / 256, cus = ncu > 0 ? ncu : 1;
+    const int nsplit = prefill_splits(T, inner, outer, ncu);
+    if (nsplit > 1)
+        return 0; // few tiles of either size: K is shared out instead
+    auto tiles = [&](int bm, int bn) { return ((T + bm - 1) / bm) * ((outer + bn - 1) / bn); };
+    const double c0 = prefill_cost(tiles(kPrefillBM, kPrefillBN), nblk, cus, 6.6, -0.37, 0.53, 0.99);
+    const double c1 = prefill_cost(tiles(kPrefillWideBM, 128), nblk, cus, 4.5, 0.20, 0.63, 1.23);
+    const double c2 = prefill_cost(tiles(kPrefillWideBM, 256), nblk, cus, 6.5, -0.10, 1.13, 2.44);
+    return c0 <= c1 && c0 <= c2 ? 0 : c1 <= c2 ? 1 : 2;
+}
 hipError_t launch_prefill_q4k(const void *w, const float *X, void *xh, float *Y, int T,
                               int inner, int outer, hipStream_t s);
 // Its two halves for rows of more than kPrefillF32MaxK columns: X rounded into

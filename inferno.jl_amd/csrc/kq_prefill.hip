@@ -49,6 +49,18 @@ constexpr int PF_BM = kPrefillBM, PF_BN = kPrefillBN; // workgroup tile: tokens 
 // (s = 0), so the non-finite value reaches its outputs.  Rows of at most
 // 8192 values stay in registers between the maximum and the conversion;
 // longer rows are read twice.
+//
+// Order of a row in Xh: its 256-column blocks in order, and inside a block its
+// 32 chunks of 8 values (16 bytes) by (stage g, half h, c), chunk 16 h + 4 g +
+// c at place 8 g + 4 h + c.  The wide kernel below multiplies a block in four
+// stages, lane half h of its matrix products covering columns 128 h + 32 g +
+// 8 c ..: with this order a stage of a token row is 128 contiguous bytes.
+__host__ __device__ constexpr int pf_chunk_place(int chunk)
+{
+    return 8 * ((chunk >> 2) & 3) + 4 * (chunk >> 4) + (chunk & 3);
+}
+// element i (a multiple of 8) of a row -> its element offset in Xh's row
+__device__ __forceinline__ int pf_x_place(int i) { return (i & ~255) + 8 * pf_chunk_place((i & 255) >> 3); }
 constexpr int PF_CVT_REG = 4; // 8-value steps a thread holds: 256 x 8 x 4 = 8192 values
 __global__ __launch_bounds__(256) void k_x_to_f16(const float *__restrict__ X,
                                                   _Float16 *__restrict__ Xh, int *__restrict__ xs,
@@ -116,12 +128,12 @@ __global__ __launch_bounds__(256) void k_x_to_f16(const float *__restrict__ X,
         for (int k = 0; k < PF_CVT_REG; ++k) {
             const int i = 8 * (tid + 256 * k);
             if (i < K)
-                *reinterpret_cast<half8 *>(hrow + i) = cvt8(v[k][0], v[k][1]);
+                *reinterpret_cast<half8 *>(hrow + pf_x_place(i)) = cvt8(v[k][0], v[k][1]);
         }
     } else {
         for (int i = 8 * tid; i < K; i += 8 * 256)
-            *reinterpret_cast<half8 *>(hrow + i) = cvt8(*reinterpret_cast<const float4 *>(row + i),
-                                                        *reinterpret_cast<const float4 *>(row + i + 4));
+            *reinterpret_cast<half8 *>(hrow + pf_x_place(i)) =
+                cvt8(*reinterpret_cast<const float4 *>(row + i), *reinterpret_cast<const float4 *>(row + i + 4));
     }
     if (tid == 0)
         xs[t] = s;
@@ -285,7 +297,8 @@ __device__ __forceinline__ void pf_read(const uint8_t *sa, const uint8_t *blk0, 
     for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const int m = 32 * t + li, c = 8 * j + 2 * s + h;
+            const int m = 32 * t + li;
+            const int c = 16 * (j & 1) + 8 * (s >> 1) + 4 * (j >> 1) + 2 * (s & 1) + h; // pf_chunk_place(8j + 2s + h)
             o.x[s][t] = *reinterpret_cast<const half8 *>(sa + m * PF_ROW_BYTES + 16 * (c ^ (m & 15)));
         }
 }
@@ -547,6 +560,263 @@ __global__ __launch_bounds__(PF_THREADS) void k_prefill_q4k(const uint8_t *__res
     }
 }
 
+// Wide tiles, for products with enough of them to fill the chip: 128 tokens x
+// 128 RU weight rows per workgroup of 4 waves, wave w holding rows 32 RU w ..
+// of the tile against all 128 tokens, over all of K.  Against the 64 x 128
+// tile above this dequantizes each weight once per 128 tokens instead of 64
+// (half the vector work per matrix product), brings 200 KB (RU = 2; RU = 1:
+// 330) from L2 per 256 x 256 x 256 product instead of 400, and needs no
+// partial sums.
+//
+// LDS: two X stages of 64 columns (16 KB each) and one column's weight blocks
+// of each wave's own rows (9 or 5 KB a wave): 68 KB for RU = 2, two workgroups
+// per CU, 52 KB for RU = 1, three.  The workgroups of a CU run at their own
+// pace, so one multiplies while another waits at its barrier.
+//
+// A wave runs K steps of 16 columns: while one step's 4 RU products run, the
+// next step's activations are read from LDS and its weights dequantized
+// (interleave() keeps the two streams mixed).  A stage is 4 steps.  Before the
+// last step's products the wave waits for its copies of the next stage and
+// for its LDS reads and meets the others; the stage's buffer is then free, so
+// the copies of the stage after next go into it, with a whole stage's time to
+// land, and the next stage's first operands are read behind the products.
+// The raw weight bytes of a column go to registers (the first half with the
+// header during the previous column's last stage), which frees the wave's
+// weight buffer for the next column's copies.  Copies past the last stage or
+// column repeat the last one, so the loop has no branches and every wait a
+// constant count.
+//
+// Measured on MI355X (us, the product alone; 64 x 128 tiles before):
+// 2048 x 12288 x 4096 181-186 against 287-305 (1.11-1.14 PFLOP/s), 512 x 14336 x
+// 4096 62-64 against 95, 2048 x 4096 x 4096 69-70 against 98-101, 1024 x 4096 x
+// 4096 40-41 (RU = 1) against 50-52.  The matrix cores are busy 58 % of the
+// cycles at a clock that power holds at 1.6-1.8 GHz: fewer bytes and vector
+// instructions per product raise the clock, reordering does not (priorities,
+// another interleave, tile orders: within 1 %; non-temporal stores of Y 10-25 %
+// slower).
+constexpr int PFW_BM = kPrefillWideBM;
+constexpr int PFW_XSTAGE = PFW_BM * 128; // 64 columns of 128 tokens, fp16
+// 1 KB copies of a wave's 32 RU rows of one block column: 9, or 5 (the last half used)
+__host__ __device__ constexpr int pfw_copies(int ru) { return (32 * ru * 144 + 1023) / 1024; }
+
+template <bool EXACTW, int RU>
+__global__ __launch_bounds__(256, RU == 2 ? 2 : 3) void k_prefill_q4k_wide(
+    const uint8_t *__restrict__ W, const _Float16 *__restrict__ Xh, const int *__restrict__ xs,
+    float *__restrict__ Y, int T, int K, int N, int mtiles, int ntiles)
+{
+    constexpr int WB = pfw_copies(RU), WREG = WB * 1024, TT = PFW_BM / 32, VPM = EXACTW ? 5 : 4;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * PFW_XSTAGE + 4 * WREG];
+
+    const int tiles = mtiles * ntiles;
+    const int lin = prefill_lin((int)blockIdx.x, tiles, 1);
+    if (lin >= tiles)
+        return; // whole workgroup
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, li = lane & 31;
+    const int nk = K / 256;
+    const uint32_t row_bytes = (uint32_t)nk * 144u;
+    const PrefillSplit ps = prefill_split_of(lin, mtiles, ntiles, nk, 1);
+    const int m0 = ps.mt * PFW_BM, n0 = ps.nt * (128 * RU) + 32 * RU * wave; // this wave's first row
+
+    // byte offsets of this wave's copies from Xh / W (stage 0, column 0):
+    // tokens 32 wave .. +31 of the X stage (8 a copy; chunk c of token m at
+    // place c ^ (m / 2 % 8) of its 128 bytes, so that the 16 lanes of a
+    // 128-bit read, one chunk of consecutive tokens, hit distinct banks) and
+    // the wave's own weight rows.  Rows past T or N re-read the last one.
+    uint32_t xo[4], wo[WB];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = 32 * wave + 8 * i + (lane >> 3);
+        const int c = (lane & 7) ^ ((m >> 1) & 7);
+        xo[i] = 2u * (uint32_t)min(m0 + m, T - 1) * (uint32_t)K + 16u * (uint32_t)c;
+    }
+#pragma unroll
+    for (int i = 0; i < WB; ++i) {
+        const int q = min(64 * i + lane, 32 * RU * 9 - 1);
+        const int row = q / 9, piece = q - 9 * row;
+        wo[i] = (uint32_t)min(n0 + row, N - 1) * row_bytes + 16u * (uint32_t)piece;
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    const uint32_t xdst = lds0 + 4096u * wave, wdst = lds0 + 2 * PFW_XSTAGE + (uint32_t)WREG * wave;
+    const uint8_t *Xb = reinterpret_cast<const uint8_t *>(Xh);
+    auto issue_x = [&](int st, int buf) {
+        const uint8_t *b = Xb + (size_t)st * 128;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            pf_copy16(b, xo[i], xdst + PFW_XSTAGE * buf + 1024 * i);
+    };
+    auto issue_w = [&](int kb) {
+        const uint8_t *b = W + (size_t)kb * 144;
+#pragma unroll
+        for (int i = 0; i < WB; ++i)
+            pf_copy16(b, wo[i], wdst + 1024 * i);
+    };
+
+    float16v acc[RU][TT];
+#pragma unroll
+    for (int u = 0; u < RU; ++u)
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[u][t][r] = 0.0f;
+
+    const uint8_t *wl = lds + 2 * PFW_XSTAGE + WREG * wave + 144 * li;
+    const int f = (li >> 1) & 7;
+    const uint8_t *xl[4]; // the lane's chunk of K step c in buffer 0, token li
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        xl[c] = lds + 128 * li + 16 * ((4 * h + c) ^ f);
+
+    // lane (li, h): rows 32 u + li, columns 128 h .. 128 h + 127 of the block (qs
+    // bytes 64 h ..): stage g is sub-block 4 h + g, K step c its bytes 8 c ..
+    uint4 rq[RU][4], hdn[RU];
+    uint32_t sc4[RU], mn4[RU];
+    float d[RU], dmin[RU];
+    auto read_w_lo = [&]() {
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            const uint8_t *b = wl + 32 * 144 * u;
+            const uint4 hd = *reinterpret_cast<const uint4 *>(b);
+            rq[u][0] = *reinterpret_cast<const uint4 *>(b + 16 + 64 * h);
+            rq[u][1] = *reinterpret_cast<const uint4 *>(b + 16 + 64 * h + 16);
+            hdn[u] = hd;
+        }
+    };
+    auto decode_w = [&]() {
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            const uint4 hd = hdn[u];
+            d[u] = h2f(hd.x & 0xffffu);
+            dmin[u] = -h2f(hd.x >> 16);
+            // sub-blocks 4h .. 4h + 3, one per byte (k_scale_min)
+            const uint32_t sl = hd.y & 0x3f3f3f3fu, ml = hd.z & 0x3f3f3f3fu;
+            const uint32_t sh = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
+            const uint32_t mh = ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u);
+            sc4[u] = h ? sh : sl;
+            mn4[u] = h ? mh : ml;
+        }
+    };
+    auto read_w_hi = [&]() {
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            const uint8_t *b = wl + 32 * 144 * u + 48 + 64 * h;
+            rq[u][2] = *reinterpret_cast<const uint4 *>(b);
+            rq[u][3] = *reinterpret_cast<const uint4 *>(b + 16);
+        }
+    };
+    half8 xf[2][TT], wq[2][RU];
+    float ds[RU], dm[RU];
+    auto read_x = [&](int g, int c) { // into xf[c & 1]
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+            xf[c & 1][t] = *reinterpret_cast<const half8 *>(xl[c] + PFW_XSTAGE * (g & 1) + 4096 * t);
+    };
+    auto dequant = [&](int g, int c) { // into wq[c & 1]
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            if (c == 0) {
+                ds[u] = d[u] * ubyte_f(sc4[u], g);
+                dm[u] = dmin[u] * ubyte_f(mn4[u], g);
+            }
+            const uint4 r4 = rq[u][2 * (g >> 1) + (c >> 1)];
+            const uint2 by = (c & 1) ? make_uint2(r4.z, r4.w) : make_uint2(r4.x, r4.y);
+            if constexpr (EXACTW) {
+                wq[c & 1][u] = pf_dequant8_exact(by, (g & 1) != 0, ds[u], dm[u]);
+            } else {
+                const _Float16 s16 = (_Float16)ds[u], m16 = (_Float16)dm[u];
+                wq[c & 1][u] = pf_dequant8(by, (g & 1) != 0, half2v{s16, s16}, half2v{m16, m16});
+            }
+        }
+    };
+    auto mma = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+                acc[u][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[c & 1][u], xf[c & 1][t], acc[u][t], 0, 0, 0);
+    };
+    // mixes a step's LDS reads, products and the next step's dequantization
+    auto interleave = [&]() {
+        __builtin_amdgcn_sched_group_barrier(0x100, TT, 0);
+#pragma unroll
+        for (int i = 0; i < RU * TT; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int nst = 4 * nk;
+    issue_w(0);
+    issue_x(0, 0);
+    issue_x(1, 1);
+    __builtin_amdgcn_s_waitcnt(4 | 0x0070);
+    lds_barrier();
+    read_w_lo();
+    decode_w();
+    read_x(0, 0);
+    dequant(0, 0);
+    for (int kb = 0; kb < nk; ++kb) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (g == 0)
+                read_w_hi();
+            if (g == 3)
+                read_w_lo(); // the next column's
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                read_x(g, c + 1);
+                mma(c);
+                dequant(g, c + 1);
+                interleave();
+            }
+            // the next stage has landed, and every wave holds this one in registers
+            if (g == 1)
+                __builtin_amdgcn_s_waitcnt(WB | 0x0070);
+            else
+                __builtin_amdgcn_s_waitcnt(0x0070);
+            lds_barrier();
+            issue_x(min(4 * kb + g + 2, nst - 1), g & 1);
+            if (g == 0)
+                issue_w(min(kb + 1, nk - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            read_x(g + 1, 0);
+            mma(3);
+            if (g == 3)
+                decode_w();
+            dequant((g + 1) & 3, 0);
+            interleave();
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0070); // the last (unused) copies have landed
+
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+        const int m = m0 + 32 * t + li;
+        if (m >= T)
+            continue;
+        const int sm = -xs[m]; // undo the row's power-of-two scale (exact)
+        float *yrow = Y + (size_t)m * N;
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 v = make_float4(__builtin_ldexpf(acc[u][t][4 * q], sm), __builtin_ldexpf(acc[u][t][4 * q + 1], sm),
+                                             __builtin_ldexpf(acc[u][t][4 * q + 2], sm), __builtin_ldexpf(acc[u][t][4 * q + 3], sm));
+                const int n = n0 + 32 * u + 8 * q + 4 * h;
+                if ((N & 3) == 0) {
+                    if (n < N)
+                        *reinterpret_cast<float4 *>(yrow + n) = v;
+                } else {
+                    if (n < N) yrow[n] = v.x;
+                    if (n + 1 < N) yrow[n + 1] = v.y;
+                    if (n + 2 < N) yrow[n + 2] = v.z;
+                    if (n + 3 < N) yrow[n + 3] = v.w;
+                }
+            }
+    }
+}
+
 // Y += P[0] + P[1] + ... + P[nparts - 1] (n floats each), in that order, so
 // the result does not depend on which split finished first.
 template <bool VEC>
@@ -715,6 +985,21 @@ hipError_t launch_prefill_q4k(const void *w, const float *X, void *xh, float *Y,
     return launch_prefill_gemm(w, xh, Y, T, inner, outer, s);
 }
 
+template <int RU>
+static void launch_prefill_wide(const void *w, const void *xh, const int *xs, float *Y, int T, int inner,
+                                int outer, hipStream_t s)
+{
+    const int mtiles = (T + kPrefillWideBM - 1) / kPrefillWideBM;
+    const int ntiles = (outer + 128 * RU - 1) / (128 * RU);
+    const dim3 grid(prefill_grid(mtiles * ntiles, 1)), block(256);
+    if (inner <= kPrefillExactWMaxK)
+        hipLaunchKernelGGL((k_prefill_q4k_wide<true, RU>), grid, block, 0, s, (const uint8_t *)w,
+                           (const _Float16 *)xh, xs, Y, T, inner, outer, mtiles, ntiles);
+    else
+        hipLaunchKernelGGL((k_prefill_q4k_wide<false, RU>), grid, block, 0, s, (const uint8_t *)w,
+                           (const _Float16 *)xh, xs, Y, T, inner, outer, mtiles, ntiles);
+}
+
 hipError_t launch_prefill_gemm(const void *w, void *xh, float *Y, int T, int inner, int outer,
                                hipStream_t s)
 {
@@ -722,6 +1007,14 @@ hipError_t launch_prefill_gemm(const void *w, void *xh, float *Y, int T, int inn
         return hipErrorInvalidValue;
     int *xs = reinterpret_cast<int *>(static_cast<uint8_t *>(xh) + prefill_scale_offset(T, inner));
     float *P = reinterpret_cast<float *>(static_cast<uint8_t *>(xh) + prefill_part_offset(T, inner));
+    const int ru = prefill_wide_rows(T, inner, outer, device_cus());
+    if (ru) {
+        if (ru == 2)
+            launch_prefill_wide<2>(w, xh, xs, Y, T, inner, outer, s);
+        else
+            launch_prefill_wide<1>(w, xh, xs, Y, T, inner, outer, s);
+        return hipGetLastError();
+    }
     const int mtiles = (T + PF_BM - 1) / PF_BM, ntiles = (outer + PF_BN - 1) / PF_BN;
     const int nsplit = prefill_splits(T, inner, outer, device_cus());
     const dim3 grid(prefill_grid(mtiles * ntiles, nsplit));
