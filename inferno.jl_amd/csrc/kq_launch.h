@@ -60,7 +60,7 @@ inline bool prefill_fits(int T, int inner, int outer)
            (int64_t)outer * (inner / 256) * 144 <= (int64_t)UINT32_MAX &&
            (int64_t)T * outer <= (int64_t)INT32_MAX; // tile counts stay ints
 }
-// Rows of at most this many columns run in the fp32 kernel (k_prefill_q4k_f32).
+// Rows of at most this many columns run on fp32 operands (k_prefill_q4k_split).
 constexpr int kPrefillF32MaxK = 512;
 // Longer rows of at most this many columns take fp16 weights rounded once
 // from their exact values (k_prefill_q4k<true>).
@@ -196,7 +196,19 @@ hipError_t launch_prefill_q4k(const void *w, const float *X, void *xh, float *Y,
 hipError_t launch_prefill_convert(const float *X, void *xh, int T, int inner, hipStream_t s);
 hipError_t launch_prefill_gemm(const void *w, void *xh, float *Y, int T, int inner, int outer,
                                hipStream_t s);
-// The same product on fp32 operands (k_prefill_q4k_f32), any inner; needs
+// Tokens per workgroup tile (64 weight rows) of the product on fp32 operands:
+// 32 or 64, whichever needs less time in rounds of one workgroup per CU, a
+// 32-token tile taking 0.58-0.62 of a 64-token one's time.  Measured on MI355X
+// (us, 32 / 64 tokens): 256 x 2048 x 2048 13.6 / 20.1, 300 x 4096 x 4096 65.2 /
+// 71.5, 200 x 4096 x 4096 43.5 / 40.3, 509 x 2048 x 2048 25.9 / 23.6.
+constexpr int kPrefillSplitMaxK = 1 << 24; // longer rows are computed value by value
+inline int prefill_split_tokens(int T, int outer, int ncu)
+{
+    const int64_t cus = ncu > 0 ? ncu : 1, nt = ((int64_t)outer + 63) / 64;
+    const int64_t r32 = (((int64_t)T + 31) / 32 * nt + cus - 1) / cus, r64 = (((int64_t)T + 63) / 64 * nt + cus - 1) / cus;
+    return 10 * r32 <= 17 * r64 ? 32 : 64;
+}
+// The same product on fp32 operands (k_prefill_q4k_split), any inner; needs
 // T * outer <= INT32_MAX.
 hipError_t launch_prefill_q4k_f32(const void *w, const float *X, float *Y, int T, int inner,
                                   int outer, hipStream_t s);

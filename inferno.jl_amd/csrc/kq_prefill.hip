@@ -10,7 +10,7 @@
 // v_mfma_f32_32x32x16_f16 accumulates in fp32.  A dot product over fp16
 // operands errs by about 2.8e-4 ||w|| ||x|| / sqrt(K) on random data, so short
 // rows need more care: rows of at most 512 columns, and the fp32-operand
-// entry point, run k_prefill_q4k_f32 (below); rows of at most 2048 columns
+// entry point, run k_prefill_q4k_split (below); rows of at most 2048 columns
 // round each weight once from its exact value (k_prefill_q4k<true>) instead
 // of through fp16 sub-block scales.
 //
@@ -28,6 +28,8 @@
 // partial sums meet in LDS and leave as 16-byte stores.
 #include "kq_common.h"
 #include "kq_launch.h"
+
+#include <type_traits>
 
 namespace ihip {
 
@@ -850,104 +852,367 @@ __global__ __launch_bounds__(256) void k_prefill_splits_sum(float *__restrict__ 
     }
 }
 
-// Rows of at most kPrefillF32MaxK columns: an fp32 GEMM on the fp32 matrix
-// cores (v_mfma_f32_32x32x2_f32), with the weights dequantized to fp32 exactly
-// (src/Dequant.jl:364-371) and X read as it is.  With fp16 operands a dot
-// product's rounding error, relative to ||w_row|| ||x||, shrinks only as
-// 1/sqrt(K): over 512 x 2048 outputs of seeded random data the largest
-// error reached 1.7x the row bound 1e-4 ||w_row|| ||x|| at K = 256 and
+// The fp32-operand product: for rows of at most kPrefillF32MaxK columns, and
+// at any length for callers that ask for it (launch_prefill_q4k_f32).  With
+// fp16 operands a dot product's rounding error, relative to ||w_row|| ||x||,
+// shrinks only as 1/sqrt(K): over 512 x 2048 outputs of seeded random data the
+// largest error reached 1.7x the row bound 1e-4 ||w_row|| ||x|| at K = 256 and
 // 0.97-1.05x at K = 512 (0.73 at 768, 0.70 at 1024, 0.30 at 4096), so short
 // rows take this path, whose error is fp32 rounding.
 //
-// Tile: 64 tokens x 64 weight rows per workgroup of 4 waves; wave (rw, tw)
-// owns weight rows 32 rw.. and tokens 32 tw.. .  K goes through LDS 64
-// columns at a time (48 KB, so that two or three workgroups share a CU and
-// one fills its chunk while another multiplies), both operands stored
-// k-major (W[k][row], X[k][token]) with rows of 96 floats, so a matrix-core
-// operand read (32 consecutive rows or tokens at k and at k + 1) hits 64
-// distinct banks.
-constexpr int PF32_KC = 64;   // columns per LDS chunk (two Q4_K sub-blocks): 48 KB of LDS
-constexpr int PF32_LD = 96;   // floats per LDS row
-__global__ __launch_bounds__(256) void k_prefill_q4k_f32(const uint8_t *__restrict__ W,
-                                                         const float *__restrict__ X,
-                                                         float *__restrict__ Y, int T, int K, int N,
-                                                         int mtiles)
-{
-    __shared__ __attribute__((aligned(16))) float Wl[PF32_KC * PF32_LD];
-    __shared__ __attribute__((aligned(16))) float Xl[PF32_KC * PF32_LD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int rw = wave & 1, tw = wave >> 1;
-    const int mt = (int)blockIdx.x % mtiles, nt = (int)blockIdx.x / mtiles;
-    const int m0 = mt * 64, n0 = nt * 64;
-    const int nblk = K / 256;
-    // fill roles: thread t stages row (or token) t / 4, 32 columns 32 (t % 4) ..
-    const int fr = tid >> 2, fp = tid & 3;
-    const uint8_t *wrow = W + (size_t)min(n0 + fr, N - 1) * (size_t)nblk * 144;
-    const float *xrow = X + (size_t)min(m0 + fr, T - 1) * (size_t)K;
+// fp32 products run at a sixteenth of the matrix cores' bf16 rate, so the
+// operands are written as bf16 without losing a bit:
+//  * x = p1 + p2 + p3, its 24 significant bits cut into three bf16 values;
+//  * the weights of a sub-block s as d sc q - dmin m
+//    = (d sc / 2) (2 q - 15) + (7.5 d sc - dmin m), 2 q - 15 an odd integer
+//    of -15 .. 15.  About the middle of the quants' range, so that the two
+//    terms do not cancel where the weights centre on zero.
+// Every bf16 product is exact.  A sub-block's sum over its 32 columns, three
+// v_mfma_f32_32x32x16_bf16 for each 16 of them (smallest parts first),
+// accumulates in fp32 from zero and one fp32 FMA per output scales it into the
+// row's sum; the second term is an fp32 product (v_mfma_f32_32x32x2_f32) of
+// the columns' sums and the mins, two sub-blocks at a time.
+//
+// Tile: 32 TT tokens x 64 weight rows per workgroup of 8 waves, which share K:
+// wave (half, j) takes sub-block pair j of the blocks 2 i + half and
+// accumulates the whole tile, so each value of X is cut up by one wave only
+// and the waves run at their own pace: every wave copies its operands through
+// LDS by itself (two X stages of 32 columns, its 48 bytes of the 64 rows'
+// blocks), with no barrier before the eight partial tiles are added up in
+// LDS, in wave order.  The vector work of a stage (cutting X 5.5 instructions
+// a value, its sums and largest magnitude 1.5, the weights, the scaling) is
+// about 1.5 times its matrix time and bounds it; the two waves of a SIMD
+// overlap them.
+//
+// Measured on MI355X (us a call; the fp32 matrix products this replaced):
+// 509 x 2048 x 2048 22.0 against 58.0, 512 x 4096 x 4096 80.8 against 186, 700 x
+// 4096 x 4096 117 against 262, 100 x 2048 x 2048 12.1 against 55.4, 512 x 256 x
+// 4096 13.7 against 14.9; error against 64 bits at 509 x 2048 x 2048 1.1e-7
+// against 8.2e-7 (fewer roundings: 64 sums of 32 columns instead of 2048).
+//
+// The matrix cores take bf16 subnormals as zeros, and a sub-block's sum could
+// overflow before its scale is applied.  Each token's largest magnitude is
+// found along the way; a tile with a token outside 2^-80 .. 2^118 is computed
+// again on tokens scaled by powers of two, which is exact, and a token that
+// holds an infinity value by value.
+constexpr int PFX_WSTAGE = 64 * 48; // header and the pair's 32 quant bytes of 64 rows
+constexpr int PFX_LD = 72;          // floats per row of a partial tile
+constexpr float kSplitMinX = 0x1p-80f, kSplitMaxX = 0x1p118f;
+__host__ __device__ constexpr int pfx_wave_bytes(int tt) { return 2 * 4096 * tt + PFX_WSTAGE; }
+static_assert(8 * pfx_wave_bytes(2) <= 160 * 1024 - 256, "the eight waves' stages fit the 160 KB of LDS");
+static_assert(PFX_LD * 64 * 4 <= pfx_wave_bytes(2) && PFX_LD * 32 * 4 <= pfx_wave_bytes(1), "and the partial tiles");
 
-    float16v acc;
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// 8 nibbles (the low ones of the 8 bytes, already shifted down) -> 2 q - 15 in
+// bf16.  The e4m3 byte whose low four bits are v is v * 2^-9 for every v of 0
+// .. 15: v = |2 q - 15|, the sign on top.
+__device__ __forceinline__ bf16x8 pfx_quants(uint2 bytes)
+{
+    auto code = [](uint32_t q) {
+        const uint32_t neg = ~q & 0x08080808u;           // q < 8: 2 q - 15 = -(2 (7 - q) + 1)
+        const uint32_t flip = neg - (neg >> 3);          // 7 where q < 8
+        const uint32_t mag = (q ^ flip) & 0x07070707u;   // q - 8 or 7 - q
+        return (mag << 1) | ((neg << 4) | 0x01010101u);
+    };
+    const uint32_t c0 = code(bytes.x), c1 = code(bytes.y);
+    const bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(c0, 512.0f, false);
+    const bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(c0, 512.0f, true);
+    const bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(c1, 512.0f, false);
+    const bf16x2 d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(c1, 512.0f, true);
+    bf16x8 r;
+    r[0] = a[0]; r[1] = a[1]; r[2] = b[0]; r[3] = b[1];
+    r[4] = c[0]; r[5] = c[1]; r[6] = d[0]; r[7] = d[1];
+    return r;
+}
+
+// 8 values of x -> their three bf16 parts (each the top half of what the
+// parts before it leave, which is exact), their sum and largest magnitude.
+__device__ __forceinline__ void pfx_parts(float4 lo, float4 hi, bf16x8 (&p)[3], float &sum, float &big)
+{
+    float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    for (int c = 0; c < 4 * nblk; ++c) {
-        // weights: columns 16 fp .. of chunk c are elements l0 .. l0 + 15 of
-        // sub-block sb = 2 (c % 4) + fp / 2 of block c / 4, element
-        // 64 j + 32 h + l = (d sc) q_l - dmin m with q_l the low (h = 0) or
-        // high nibble of qs[32 j + l] (src/Dequant.jl:364-371)
-        {
-            const uint8_t *blk = wrow + (size_t)(c >> 2) * 144;
-            const int sb = 2 * (c & 3) + (fp >> 1), j = sb >> 1, h = sb & 1, l0 = 16 * (fp & 1);
-            const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
-            const float d = h2f(hd.x & 0xffffu), dmin = h2f(hd.x >> 16);
-            uint32_t sc, m;
-            k_scale_min(hd.y, hd.z, hd.w, sb, sc, m);
-            const float d1 = d * (float)sc, m1 = dmin * (float)m;
-            const uint4 qa = *reinterpret_cast<const uint4 *>(blk + 16 + 32 * j + l0);
-            const uint32_t qw[4] = {qa.x, qa.y, qa.z, qa.w};
+    for (int i = 0; i < 8; i += 2)
+        big = fmaxf(fmaxf(fabsf(v[i]), fabsf(v[i + 1])), big);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const uint32_t q = ((qw[i >> 2] >> (8 * (i & 3))) >> (4 * h)) & 0xfu;
-                Wl[(16 * fp + i) * PF32_LD + fr] = d1 * (float)q - m1;
+    for (int k = 0; k < 3; ++k) {
+        uint32_t d[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t a = __float_as_uint(v[2 * i]), b = __float_as_uint(v[2 * i + 1]);
+            d[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+            v[2 * i] -= __uint_as_float(a & 0xffff0000u);
+            v[2 * i + 1] -= __uint_as_float(b & 0xffff0000u);
+        }
+        p[k] = __builtin_bit_cast(bf16x8, make_uint4(d[0], d[1], d[2], d[3]));
+    }
+}
+
+template <int TT>
+__global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__restrict__ W,
+                                                              const float *__restrict__ X,
+                                                              float *__restrict__ Y, int T, int K, int N,
+                                                              int mtiles, int ntiles, int by_value)
+{
+    constexpr int XC = 4 * TT, XST = 4096 * TT, WAVE = pfx_wave_bytes(TT); // 1 KB copies and bytes of an X stage
+    __shared__ __attribute__((aligned(16))) uint8_t lds[8 * WAVE];
+    __shared__ uint32_t tokmax[32 * TT]; // the tokens' largest |x| (bits)
+
+    const int tiles = mtiles * ntiles;
+    const int lin = prefill_lin((int)blockIdx.x, tiles, 1);
+    if (lin >= tiles)
+        return; // whole workgroup
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, li = lane & 31, j = wave & 3, half = wave >> 2;
+    const int nk = K / 256;
+    const size_t row_bytes = (size_t)nk * 144;
+    const PrefillSplit ps = prefill_split_of(lin, mtiles, ntiles, nk, 1);
+    const int m0 = ps.mt * (32 * TT), n0 = ps.nt * 64;
+    if (tid < 32 * TT)
+        tokmax[tid] = 0u;
+    __syncthreads();
+
+    float16v acc[TT][2];
+    float big[TT];
+    int shift[TT];
+    const int nb = by_value ? 0 : (nk - half + 1) >> 1, ns = 2 * nb; // this wave's blocks and stages
+    auto product = [&](auto scaled) { // scaled: of the tokens times 2^shift
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            big[t] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[t][u][r] = 0.0f;
+        }
+        if (nb <= 0)
+            return;
+        // copies: 8 tokens x 128 bytes each of an X stage, chunk c of token m
+        // at place c ^ (m / 2 % 8) of its 128 bytes (the 16 lanes of a 128-bit
+        // read hit distinct banks), and 64 rows x 3 pieces of the blocks.  The
+        // offsets stay below 2^32: the launcher bounds K.  Rows past T or N
+        // re-read the last one, stages past the last repeat it.
+        uint32_t xo[XC], wo[3];
+#pragma unroll
+        for (int i = 0; i < XC; ++i) {
+            const int m = 8 * i + (lane >> 3), c = (lane & 7) ^ ((m >> 1) & 7);
+            xo[i] = (uint32_t)min(m, T - 1 - m0) * ((uint32_t)K * 4u) + 16u * (uint32_t)c;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int q = 64 * i + lane, row = q / 3, piece = q - 3 * row;
+            wo[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)row_bytes + (piece ? 32u * j + 16u * piece : 0u);
+        }
+        const uint8_t *Xb = reinterpret_cast<const uint8_t *>(X + (size_t)m0 * K + 256 * half + 64 * j);
+        const uint8_t *Wb = W + (size_t)n0 * row_bytes + 144 * half;
+        uint8_t *const mine = lds + WAVE * wave;
+        const uint32_t xdst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mine;
+        const uint32_t wdst = xdst + 2 * XST;
+        auto issue_x = [&](int n) {
+            const int st = min(n, ns - 1);
+            const uint8_t *b = Xb + (size_t)(st >> 1) * 2048 + 128 * (st & 1);
+#pragma unroll
+            for (int i = 0; i < XC; ++i)
+                pf_copy16(b, xo[i], xdst + XST * (n & 1) + 1024 * i);
+        };
+        auto issue_w = [&](int i) {
+            const uint8_t *b = Wb + (size_t)min(i, nb - 1) * 288;
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                pf_copy16(b, wo[k], wdst + 1024 * k);
+        };
+        const uint8_t *xl = mine + 128 * li, *wl = mine + 2 * XST + 48 * li;
+        const int f = (li >> 1) & 7;
+
+        float4 xr[TT][2][2];
+        uint2 qs[2][2];
+        float ds[2][2], ndm[2], xsum[2][TT]; // [row tile or sub-block][..]
+        auto read_x = [&](int s) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        xr[t][c][e] = *reinterpret_cast<const float4 *>(xl + XST * s + 4096 * t +
+                                                                       16 * ((4 * c + 2 * h + e) ^ f));
+        };
+        auto stage = [&](int s) {
+            bf16x8 wq[2][2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const uint2 b = qs[u][c];
+                    wq[u][c] = pfx_quants(s ? make_uint2(b.x >> 4, b.y >> 4) : b);
+                }
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                bf16x8 p[2][3];
+                xsum[s][t] = 0.0f;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    if constexpr (decltype(scaled)::value) {
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            float4 &v = xr[t][c][e];
+                            v = make_float4(__builtin_ldexpf(v.x, shift[t]), __builtin_ldexpf(v.y, shift[t]),
+                                            __builtin_ldexpf(v.z, shift[t]), __builtin_ldexpf(v.w, shift[t]));
+                        }
+                    }
+                    pfx_parts(xr[t][c][0], xr[t][c][1], p[c], xsum[s][t], big[t]);
+                }
+                float16v sub[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) sub[u][r] = 0.0f;
+#pragma unroll
+                for (int k = 2; k >= 0; --k)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c)
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            sub[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[c][k], wq[u][c], sub[u], 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        acc[t][u][r] = fmaf(sub[u][r], ds[u][s], acc[t][u][r]);
+            }
+        };
+
+        issue_w(0);
+        issue_x(0);
+        issue_x(1);
+        for (int i = 0; i < nb; ++i) {
+            __builtin_amdgcn_s_waitcnt(XC | 0x0f70); // all but the next stage's copies have landed
+            asm volatile("" ::: "memory");
+            uint4 hd[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                hd[u] = *reinterpret_cast<const uint4 *>(wl + 32 * 48 * u);
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    qs[u][c] = *reinterpret_cast<const uint2 *>(wl + 32 * 48 * u + 16 + 16 * c + 8 * h);
+            }
+            read_x(0);
+            __builtin_amdgcn_s_waitcnt(0xc07f); // and are in registers: their place is free
+            asm volatile("" ::: "memory");
+            issue_x(2 * i + 2);
+            issue_w(i + 1);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const float d = h2f(hd[u].x & 0xffffu), dmin = h2f(hd[u].x >> 16);
+                float scA, mA, scB, mB;
+                k_scale_min_pair(hd[u].y, hd[u].z, hd[u].w, j, scA, mA, scB, mB);
+                ds[u][0] = 0.5f * d * scA;
+                ds[u][1] = 0.5f * d * scB;
+                // this lane half's sub-block of the pair
+                ndm[u] = fmaf(15.0f, h ? ds[u][1] : ds[u][0], -(dmin * (h ? mB : mA)));
+            }
+            stage(0);
+            __builtin_amdgcn_s_waitcnt((XC + 3) | 0x0f70);
+            asm volatile("" ::: "memory");
+            read_x(1);
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            asm volatile("" ::: "memory");
+            issue_x(2 * i + 3);
+            stage(1);
+            // lane (li, h): token li's sum over the pair's sub-block h
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const auto x2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(xsum[0][t]),
+                                                                 __float_as_uint(xsum[1][t]), false, false);
+                const float both = __uint_as_float((uint32_t)x2[0]) + __uint_as_float((uint32_t)x2[1]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(both, ndm[u], acc[t][u], 0, 0, 0);
             }
         }
-        // activations: token fr, columns 64 c + 16 fp ..
-        {
-            const float4 *xs = reinterpret_cast<const float4 *>(xrow + (size_t)c * PF32_KC + 16 * fp);
+        __builtin_amdgcn_s_waitcnt(0x0070); // the last (unused) copies have landed
+    };
+    product(std::false_type{});
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 v = xs[i];
-                Xl[(16 * fp + 4 * i + 0) * PF32_LD + fr] = v.x;
-                Xl[(16 * fp + 4 * i + 1) * PF32_LD + fr] = v.y;
-                Xl[(16 * fp + 4 * i + 2) * PF32_LD + fr] = v.z;
-                Xl[(16 * fp + 4 * i + 3) * PF32_LD + fr] = v.w;
-            }
-        }
-        __syncthreads();
-        // A = weights (lane l: row l % 32 at k + l / 32), B = activations
-        // (token l % 32 at k + l / 32)
-        const float *wa = Wl + (lane >> 5) * PF32_LD + 32 * rw + (lane & 31);
-        const float *xb = Xl + (lane >> 5) * PF32_LD + 32 * tw + (lane & 31);
-#pragma unroll 8
-        for (int k = 0; k < PF32_KC; k += 2)
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[k * PF32_LD], xb[k * PF32_LD], acc, 0, 0, 0);
+    for (int t = 0; t < TT; ++t)
+        atomicMax(&tokmax[32 * t + li], __float_as_uint(big[t]));
+    __syncthreads();
+    // a token's power of two: its largest magnitude to [0.5, 1)
+    auto shift_of = [&](int m) {
+        const float b = __uint_as_float(tokmax[m]);
+        return b > 0.0f && b < __builtin_inff() ? -__builtin_amdgcn_frexp_expf(b) : 0;
+    };
+    bool out_of_range = false;
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+        const float b = __uint_as_float(tokmax[32 * t + li]);
+        out_of_range |= (b > 0.0f && b < kSplitMinX) || (b >= kSplitMaxX && b < __builtin_inff());
+        shift[t] = shift_of(32 * t + li);
+    }
+    const bool again = __ballot(out_of_range) != 0; // the same in every wave
+    if (again) {
+        product(std::true_type{});
         __syncthreads();
     }
-    // lane l, register r: weight row 32 rw + 8 (r / 4) + 4 (l / 32) + r % 4,
-    // token 32 tw + l % 32
-    const int m = m0 + 32 * tw + (lane & 31);
-    if (m >= T)
-        return;
-    float *yrow = Y + (size_t)m * (size_t)N;
+    // lane (li, h), register r of acc[t][u]: token 32 t + 8 (r / 4) + 4 h + r % 4, row 32 u + li
+    float *const P = reinterpret_cast<float *>(lds);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int n = n0 + 32 * rw + 8 * q + 4 * (lane >> 5);
-        const float4 v = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-        if ((N & 3) == 0 && n + 3 < N) {
-            *reinterpret_cast<float4 *>(yrow + n) = v;
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                P[(32 * TT * wave + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3)) * PFX_LD + 32 * u + li] = acc[t][u][r];
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < TT; ++p) {
+        const int ml = 32 * p + (tid >> 4), nl = 4 * (tid & 15), m = m0 + ml, n = n0 + nl;
+        if (m >= T || n >= N)
+            continue;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (!by_value && tokmax[ml] < 0x7f800000u) {
+            const int sm = again ? -shift_of(ml) : 0;
+#pragma unroll
+            for (int w = 0; w < 8; ++w) {
+                const float4 q = *reinterpret_cast<const float4 *>(P + (32 * TT * w + ml) * PFX_LD + nl);
+                v.x += q.x;
+                v.y += q.y;
+                v.z += q.z;
+                v.w += q.w;
+            }
+            v = make_float4(__builtin_ldexpf(v.x, sm), __builtin_ldexpf(v.y, sm), __builtin_ldexpf(v.z, sm),
+                            __builtin_ldexpf(v.w, sm));
         } else {
-            if (n < N) yrow[n] = v.x;
-            if (n + 1 < N) yrow[n + 1] = v.y;
-            if (n + 2 < N) yrow[n + 2] = v.z;
-            if (n + 3 < N) yrow[n + 3] = v.w;
+            // weight element 64 jj + 32 hh + l of a block is (d sc) q_l - dmin m
+            // with q_l the low (hh = 0) or high nibble of qs[32 jj + l]
+            // (src/Dequant.jl:364-371)
+            float a[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int e = 0; e < 4 && n + e < N; ++e)
+                for (int kb = 0; kb < nk; ++kb) {
+                    const uint8_t *blk = W + (size_t)(n + e) * row_bytes + (size_t)kb * 144;
+                    const float *xv = X + (size_t)m * K + 256 * (size_t)kb;
+                    const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
+                    const float d = h2f(hd.x & 0xffffu), dmin = h2f(hd.x >> 16);
+                    for (int k = 0; k < 256; ++k) {
+                        uint32_t sc, mn;
+                        k_scale_min(hd.y, hd.z, hd.w, k >> 5, sc, mn);
+                        const uint32_t q = (blk[16 + 32 * (k >> 6) + (k & 31)] >> (4 * ((k >> 5) & 1))) & 15u;
+                        a[e] = fmaf(d * (float)sc * (float)q - dmin * (float)mn, xv[k], a[e]);
+                    }
+                }
+            v = make_float4(a[0], a[1], a[2], a[3]);
+        }
+        float *y = Y + (size_t)m * (size_t)N + n;
+        if ((N & 3) == 0) {
+            *reinterpret_cast<float4 *>(y) = v;
+        } else {
+            y[0] = v.x;
+            if (n + 1 < N) y[1] = v.y;
+            if (n + 2 < N) y[2] = v.z;
+            if (n + 3 < N) y[3] = v.w;
         }
     }
 }
@@ -957,9 +1222,17 @@ hipError_t launch_prefill_q4k_f32(const void *w, const float *X, float *Y, int T
 {
     if (T <= 0 || outer <= 0 || inner <= 0 || inner % 256 || (int64_t)T * outer > (int64_t)INT32_MAX)
         return hipErrorInvalidValue;
-    const int mtiles = (T + 63) / 64, ntiles = (outer + 63) / 64;
-    hipLaunchKernelGGL(k_prefill_q4k_f32, dim3((unsigned)(mtiles * ntiles)), dim3(256), 0, s,
-                       (const uint8_t *)w, X, Y, T, inner, outer, mtiles);
+    const int tt = prefill_split_tokens(T, outer, device_cus()) / 32;
+    const int mtiles = (T + 32 * tt - 1) / (32 * tt), ntiles = (outer + 63) / 64;
+    // 64 rows of X, and 64 rows of W, are addressed by 32-bit byte offsets
+    const int by_value = inner > kPrefillSplitMaxK;
+    const dim3 grid(prefill_grid(mtiles * ntiles, 1)), block(512);
+    if (tt == 1)
+        hipLaunchKernelGGL(k_prefill_q4k_split<1>, grid, block, 0, s, (const uint8_t *)w, X, Y, T, inner, outer,
+                           mtiles, ntiles, by_value);
+    else
+        hipLaunchKernelGGL(k_prefill_q4k_split<2>, grid, block, 0, s, (const uint8_t *)w, X, Y, T, inner, outer,
+                           mtiles, ntiles, by_value);
     return hipGetLastError();
 }
 

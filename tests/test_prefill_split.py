@@ -1,0 +1,93 @@
+"""The product on fp32 operands (k_prefill_q4k_split: X cut into three bf16
+parts, K shared by the eight waves of a workgroup) against float64 at the edges
+of its tiles and of its share of K, and with values at the ends of fp32's range.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from inferno_hip import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _product(w, X, outer, inner):
+    import torch
+    from inferno_hip import device as D
+    Y = D.prefill_q4_k_f32(D.DeviceWeight(torch.from_numpy(w).cuda(), synth.Q4_K, inner, outer),
+                           torch.from_numpy(X).cuda())
+    return Y.cpu().numpy().astype(np.float64)
+
+
+def _check(w, X, outer, inner, what):
+    wf = oracle.dequant(synth.Q4_K, w, inner * outer).reshape(outer, inner).astype(np.float64)
+    xf = X.astype(np.float64)
+    # fp32 rounding stays under a tenth of the row bound 1e-4 ||w_row|| ||x||
+    # (K terms of 2^-24 each, random signs: 2^-24 sqrt(K) / sqrt(K) of the norms
+    # times the six roundings of a sub-block); one step of fp32's
+    # subnormals for results below its range
+    tol = 1e-5 * np.linalg.norm(wf, axis=1)[None, :] * np.linalg.norm(xf, axis=1)[:, None] + 2.0 ** -149
+    ratio = np.max(np.abs(_product(w, X, outer, inner) - xf @ wf.T) / tol)
+    print(f"{what}: max err/tol = {ratio:.3e}", flush=True)
+    assert ratio <= 1.0
+
+
+# tokens around the 32- and 64-token tiles, rows around 64 and off 4 (scalar
+# stores), one to nine block columns (the wave halves' uneven shares, none for one)
+@pytest.mark.parametrize("T,outer,inner", [(1, 1, 256), (31, 63, 512), (33, 65, 768), (32, 4096, 256),
+                                           (63, 130, 2304), (65, 8193, 512), (129, 4095, 1280), (257, 4100, 256)])
+def test_tile_edges(T, outer, inner):
+    print(f"split prefill T={T} {outer}x{inner}", flush=True)
+    rng = synth.rng_for(0x5B17 + T)
+    w = synth.weight(rng, synth.Q4_K, outer, inner)
+    X = (rng.standard_normal((T, inner)) * np.exp2(rng.integers(-20, 21, T))[:, None]).astype(np.float32)
+    _check(w, X, outer, inner, f"{T}x{outer}x{inner}")
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -140, 2.0 ** -120, 2.0 ** -100, 2.0 ** 100, 2.0 ** 116, 2.0 ** 119])
+def test_ends_of_the_range(scale):
+    """Tokens whose bf16 parts would be subnormal or whose sub-block sums would
+    overflow (their tiles are computed on scaled tokens)."""
+    print(f"split prefill scale={scale}", flush=True)
+    rng = synth.rng_for(0x5B18)
+    T, outer, inner = 40, 70, 512
+    w = synth.weight(rng, synth.Q4_K, outer, inner)
+    X = (rng.uniform(-1, 1, (T, inner)) * scale).astype(np.float32)
+    X[3] = rng.standard_normal(inner)  # an ordinary token in the same tile
+    _check(w, X, outer, inner, f"scale {scale}")
+
+
+def test_non_finite_activations_reach_their_tokens_only():
+    rng = synth.rng_for(0x5B19)
+    T, outer, inner = 70, 64, 512
+    w = synth.weight(rng, synth.Q4_K, outer, inner)
+    X = rng.standard_normal((T, inner)).astype(np.float32)
+    bad = X.copy()
+    bad[5, 100], bad[66, 300] = np.nan, np.inf
+    bad.view(np.uint32)[7, 9] = 0x7F800001  # a NaN whose upper half is an infinity's
+    Y, Z = _product(w, X, outer, inner), _product(w, bad, outer, inner)
+    wf = oracle.dequant(synth.Q4_K, w, inner * outer).reshape(outer, inner)
+    assert np.isnan(Z[5]).all() and np.isnan(Z[7]).all()
+    col = wf[:, 300]
+    assert np.array_equal(np.isposinf(Z[66]), col > 0) and np.array_equal(np.isneginf(Z[66]), col < 0)
+    keep = [t for t in range(T) if t not in (5, 7, 66)]
+    np.testing.assert_allclose(Z[keep], Y[keep], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("bias", [0.0, 3.0])
+def test_error_is_no_larger_than_fp32_products_in_order(bias):
+    """Against the fp32 sum of fp32 products in column order, activations with
+    and without a common offset."""
+    rng = synth.rng_for(0x5B1A)
+    T, outer, inner = 64, 256, 2048
+    w = synth.weight(rng, synth.Q4_K, outer, inner)
+    X = (rng.standard_normal((T, inner)) + bias).astype(np.float32)
+    wf = oracle.dequant(synth.Q4_K, w, inner * outer).reshape(outer, inner).astype(np.float32)
+    exact = X.astype(np.float64) @ wf.T.astype(np.float64)
+    serial = np.zeros((T, outer), np.float32)
+    for k in range(inner):
+        serial += X[:, k:k + 1] * wf[None, :, k]
+    here = np.linalg.norm(_product(w, X, outer, inner) - exact)
+    there = np.linalg.norm(serial - exact)
+    print(f"bias {bias}: {here / np.linalg.norm(exact):.2e}, fp32 in order {there / np.linalg.norm(exact):.2e}", flush=True)
+    assert here <= there
