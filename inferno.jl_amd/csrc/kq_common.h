@@ -60,6 +60,12 @@ __device__ __forceinline__ float dpp_add(float v)
     return v + __int_as_float(moved);
 }
 
+template <int CTRL>
+__device__ __forceinline__ int dpp_add_i32(int v)
+{
+    return v + __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+}
+
 // Sum over the 64 lanes of a wavefront; every lane gets the total.  DPP lane
 // moves (no LDS traffic): pairs, quads, half-rows and rows of 16 by
 // quad_perm / row_half_mirror / row_mirror, then row_bcast:15 and
@@ -135,6 +141,15 @@ __device__ __forceinline__ void lds_copy16(const void *src, uint32_t lds)
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :
                  : "v"(src), "s"(lds)
+                 : "memory", "m0");
+}
+
+// The same from a wave-uniform base plus the lane's 32-bit byte offset.
+__device__ __forceinline__ void lds_copy16_at(const void *base, uint32_t off, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(off), "s"(base), "s"(lds)
                  : "memory", "m0");
 }
 

@@ -16,10 +16,12 @@
 // `dmin*m` term of Q4_K/Q5_K and the weight offsets of Q6_K / Q8_0 / IQ4_NL
 // are taken off through per-sub-block sums of x that all rows share.
 //
-//   * Q4_K / Q5_K ("wide" kernels, k_gemv_kwide / k_gemv_kpers): blocks are
-//     16-byte multiples, so lanes load straight from HBM with 128-bit loads.
-//     A wave covers 16 blocks (4096 columns) of R rows per pass: lane =
-//     (block, sub-block pair), 64 weights per lane per row.
+//   * Q4_K / Q5_K rows that fill 16 blocks ("wide" kernels, k_gemv_kwide /
+//     k_gemv_kpers): blocks are 16-byte multiples, so lanes load straight from
+//     HBM with 128-bit loads.  A wave covers 16 blocks (4096 columns) of R rows
+//     per pass: lane = (block, sub-block pair), 64 weights per lane per row.
+//   * Other Q4_K / Q5_K rows and Q6_K (k_gemv_mdig): four rows x four blocks a
+//     step, the integer products on the matrix cores.
 //   * Q6_K (210 B), Q8_0 (34 B) and IQ4_NL (18 B) blocks are not 16-byte
 //     aligned, but 8 of them are.  k_gemv_sdig streams each wave's rows
 //     through a private LDS ring filled by gfx950's direct-to-LDS 128-bit
@@ -368,9 +370,6 @@ __device__ __forceinline__ float kdig_dot(const KBytes &B, int j, const XDig &X)
 //     1/sqrt(mean(x^2) + eps) at the end, so the norm costs no extra pass.
 //   plain: y[r] = resid[r] + (W x)[r], the residual add of
 //     src/ModelCPU.jl:913-920 (resid may be y itself).
-//
-// The body is shared with k_gemv_kwide_norm (a plain GEMV whose input is the
-// normed x) through kwide_body, which takes NORM and RESID directly.
 template <int FMT, int R, bool GATEUP, bool NORM, bool RESID, int NWV>
 __device__ __forceinline__ void kwide_body(const uint8_t *__restrict__ W, const uint8_t *__restrict__ W2,
                                            const float *__restrict__ x, float *y, int outer, int nblk,
@@ -498,17 +497,437 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kwide(const uint8_t *__restri
                                                                    resid, epi);
 }
 
-// y = W (rmsnorm(x) .* nw) for one weight: the gate/up pass's folded norm
-// (x .* nw staged, the row sums scaled by 1/sqrt(mean(x^2) + eps)) in front of
-// a plain GEMV, e.g. the grouped wq/wk/wv behind a layer's input norm
-// (src/ModelCPU.jl:903, 789-791).
-template <int FMT, int R, int NWV>
-__global__ __launch_bounds__(NWV * 64) void k_gemv_kwide_norm(const uint8_t *__restrict__ W,
-                                                         const float *__restrict__ x, float *y,
-                                                         int outer, int nblk,
-                                                         const float *__restrict__ nw, float eps)
+// ------------------------------------------------------------------------
+// Q4_K / Q5_K on the matrix cores (k_gemv_mdig)
+// ------------------------------------------------------------------------
+
+// v_mfma_i32_4x4x4_16b_i8 forms sixteen independent 4 x 4 products over four
+// bytes each: lane 4 b + r gives byte row r of A_b and byte column r of B_b and
+// gets column r of A_b B_b.  With the digit planes of four elements of x as
+// the rows of A_b and four weights of four matrix rows as the columns of
+// B_b, a lane gets its four weights times all three planes in one instruction
+// outside the vector unit, where the wide kernels issue three v_dot4 (48 of
+// their 120 vector instructions per 64 weights), and it keeps a third of the
+// activations: one plane.
+//
+// Lane geometry: lane = 4 b + r covers sub-block pair b & 3 of block b >> 2 of
+// the step's four blocks (1024 columns), in row r of a group of four rows:
+// a row's bytes of a step are 576 or 704 contiguous bytes, any row length
+// leaves at most three blocks of its last step idle (16-block passes left up
+// to 15), and one sum over the lanes serves four rows.
+//
+// Digits: X = 65536 b2 + 256 b1 + b0 as above, rounded to nearest instead of
+// truncated (half the error), and with b0 and b1 signed too (the i8 product
+// takes no unsigned bytes): the bytes of X + 0x808080, each less 128.  The
+// sub-block sums are exact.
+//
+// The weights come through a private ring of LDS slots per wave, filled by
+// direct-to-LDS copies: a quad of lanes wants four rows, and register loads in
+// that order touch four cache lines per quad (measured at 4096 x 4096 Q4_K:
+// 5.6 us against 4.1).
+//
+// LDS, per step: four planes of 64 + 1 16-byte words: word 4 b + i of plane t
+// holds digit plane i (0..2; 3 unused) of the lane's elements 16 t .. 16 t + 15,
+// so that a wave reads 1 KB in lane order; the 65th word spreads the staging
+// writes over the banks.  Then 16 bytes for each b: Q4_K / Q5_K {sum A, sum B,
+// exponent A, exponent B} of the pair, Q6_K 2^(e - 22) of its four groups.
+constexpr int kMdPlaneDw = 65 * 4, kMdStepDw = 4 * kMdPlaneDw;
+constexpr int kMdUnits = 512; // units (four rows x one step) per workgroup
+// Bytes of a block; 16-byte pieces of a row's step (Q6_K: from the 16-byte
+// unit its first byte lies in, at an even phase of 0 .. 14); pieces between two
+// rows in a ring slot (one more: 13 of 16 lanes' 128-bit reads then hit
+// distinct banks, 8 without); 1 KB copies of a slot.
+template <int FMT>
+struct MdFmt;
+template <>
+struct MdFmt<kQ4_K> {
+    static constexpr int BYTES = 144, PIECES = 36, PITCH = 37, COPIES = 3;
+};
+template <>
+struct MdFmt<kQ5_K> {
+    static constexpr int BYTES = 176, PIECES = 44, PITCH = 45, COPIES = 3;
+};
+template <>
+struct MdFmt<kQ6_K> {
+    static constexpr int BYTES = 210, PIECES = 54, PITCH = 55, COPIES = 4;
+};
+
+// Digits of one float4 of x (number f of the row); 8 consecutive threads hold
+// one sub-block of 32 elements.
+template <int FMT>
+__device__ __forceinline__ void md_stage4(float4 v, int f, uint32_t *dig, float4 *pinfo)
 {
-    kwide_body<FMT, R, false, true, false, NWV>(W, nullptr, x, y, outer, nblk, nw, eps, nullptr, 0);
+    uint32_t m = abs_bits_max(v);
+    m = dpp_max_u32<0xb1, 0xf>(m);
+    m = dpp_max_u32<0x4e, 0xf>(m);
+    m = dpp_max_u32<0x141, 0xf>(m);
+    const bool finite = m < 0x7f800000u;
+    // not below -127, where 2^(e - 22) is the smallest subnormal and every
+    // fp32 value a whole multiple of it
+    const int e = finite ? max(__builtin_amdgcn_frexp_expf(__uint_as_float(m)), -127) : 0;
+    const int sh = 22 - e;
+    auto fixed = [&](float a) { return finite ? (int)__builtin_rintf(__builtin_ldexpf(a, sh)) : 0; };
+    const int X0 = fixed(v.x), X1 = fixed(v.y), X2 = fixed(v.z), X3 = fixed(v.w);
+    uint32_t d0, d1, d2;
+    dig_pack(X0 + 0x808080, X1 + 0x808080, X2 + 0x808080, X3 + 0x808080, d0, d1, d2);
+    // the lane position and the dword of its planes that element 4 f is: pair f
+    // / 16 and f % 16, or (Q6_K: element 128 h + 32 c + 16 l + 4 k of a block is
+    // element 16 c + 4 k of lane position 2 h + l)
+    const int b = FMT == kQ6_K ? ((f >> 6) & 3) * 4 + ((f >> 5) & 1) * 2 + ((f >> 2) & 1) : (f >> 4) & 15;
+    const int t4 = FMT == kQ6_K ? (f >> 3) & 3 : (f >> 2) & 3;
+    uint32_t *p = dig + (f >> 8) * kMdStepDw + t4 * kMdPlaneDw + b * 16 + (f & 3);
+    p[0] = d0 ^ 0x80808080u;
+    p[4] = d1 ^ 0x80808080u;
+    p[8] = d2 ^ 0x80808080u;
+    if constexpr (FMT == kQ6_K) {
+        if ((f & 3) == 0)
+            reinterpret_cast<float *>(pinfo + (f >> 8) * 16 + b)[t4] = finite ? __builtin_ldexpf(1.0f, e - 22) : __builtin_nanf("");
+    } else {
+        // the sum of the rounded values, so that a weight's two terms see the
+        // same x: the rounding of x then meets d sc q - dmin m, not d sc q alone
+        int t = (X0 + X1) + (X2 + X3);
+        t = dpp_add_i32<0xb1>(t);
+        t = dpp_add_i32<0x4e>(t);
+        t = dpp_add_i32<0x141>(t);
+        if ((f & 7) == 0) {
+            float *q = reinterpret_cast<float *>(pinfo + (f >> 4)) + ((f >> 3) & 1);
+            q[0] = finite ? __builtin_ldexpf((float)t, e - 22) : __builtin_nanf("");
+            q[2] = __int_as_float(e);
+        }
+    }
+}
+
+// A lane's share of its row, as kdig_dot: the two sub-blocks of pair j.
+template <int FMT>
+__device__ __forceinline__ float mdig_dot(const KBytes &B, int j, const uint4 (&X)[4], float4 info)
+{
+    typedef int int4v __attribute__((ext_vector_type(4)));
+    const uint32_t qw[8] = {B.q0.x, B.q0.y, B.q0.z, B.q0.w, B.q1.x, B.q1.y, B.q1.z, B.q1.w};
+    const uint32_t e[8] = {B.e0.x, B.e0.y, B.e0.z, B.e0.w, B.e1.x, B.e1.y, B.e1.z, B.e1.w};
+    const uint32_t xd[16] = {X[0].x, X[0].y, X[0].z, X[0].w, X[1].x, X[1].y, X[1].z, X[1].w,
+                             X[2].x, X[2].y, X[2].z, X[2].w, X[3].x, X[3].y, X[3].z, X[3].w};
+    int4v a = {0, 0, 0, 0}, c = {0, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        uint32_t lo = qw[t] & 0x0f0f0f0fu;
+        uint32_t hi = (qw[t] >> 4) & 0x0f0f0f0fu;
+        if constexpr (FMT == kQ5_K) {
+            const uint32_t w = e[t] >> (2 * j);
+            lo |= (w & 0x01010101u) << 4;
+            hi |= (w & 0x02020202u) << 3;
+        }
+        a = __builtin_amdgcn_mfma_i32_4x4x4i8((int)xd[t], (int)lo, a, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_i32_4x4x4i8((int)xd[8 + t], (int)hi, c, 0, 0, 0);
+    }
+    // 256 S2 + S1 stays below 2^24 (dig_combine)
+    const float vA = fmaf((float)((a[2] << 8) + a[1]), 256.0f, (float)a[0]);
+    const float vB = fmaf((float)((c[2] << 8) + c[1]), 256.0f, (float)c[0]);
+    const float d = h2f(B.h.x & 0xffffu), dmin = h2f(B.h.x >> 16);
+    float scA, mA, scB, mB;
+    k_scale_min_pair(B.h.y, B.h.z, B.h.w, j, scA, mA, scB, mB);
+    const float pos = __builtin_ldexpf(scA * vA, __float_as_int(info.z) - 22) +
+                      __builtin_ldexpf(scB * vB, __float_as_int(info.w) - 22);
+    const float neg = fmaf(mA, info.x, mB * info.y);
+    return fmaf(d, pos, -(dmin * neg));
+}
+
+// The same for Q6_K: lane position b = 4 block + 2 h + l, elements 128 h + 32 c
+// + 16 l + (0..15) of the block for c = 0..3 (src/Dequant.jl:521-548: the low or
+// high nibbles of ql[64 h + 32 (c & 1) + 16 l ..] with bits 2 c, 2 c + 1 of qh[32 h
+// + 16 l ..], scale 8 h + 2 c + l).  The block starts sh = 0 or 2 bytes into a
+// dword of LDS.  The quants' offset of 32 comes off on the matrix cores too.
+__device__ __forceinline__ float mdig_dot_q6(const uint8_t *blk, uint32_t sh, int h, int l, const uint4 (&X)[4],
+                                             float4 info)
+{
+    typedef int int4v __attribute__((ext_vector_type(4)));
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(blk); // aligned down: byte i is at i + sh
+    auto read4 = [&](int dw, uint32_t (&o)[4]) {
+        uint32_t w[5];
+#pragma unroll
+        for (int i = 0; i < 5; ++i) w[i] = p[dw + i];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], sh);
+    };
+    uint32_t q0[4], q1[4], qh[4];
+    read4(16 * h + 4 * l, q0);
+    read4(16 * h + 8 + 4 * l, q1);
+    read4(32 + 8 * h + 4 * l, qh);
+    const uint32_t s0 = p[48 + 2 * h], s1 = p[49 + 2 * h], s2 = p[50 + 2 * h], dw = p[52];
+    const uint32_t sa = __builtin_amdgcn_alignbyte(s1, s0, sh) >> (8 * l); // scales c = 0, 1 in bytes 0, 2
+    const uint32_t sb = __builtin_amdgcn_alignbyte(s2, s1, sh) >> (8 * l);
+    const float d = h2f(sh ? dw >> 16 : dw & 0xffffu);
+    const uint32_t xd[4][4] = {{X[0].x, X[0].y, X[0].z, X[0].w}, {X[1].x, X[1].y, X[1].z, X[1].w},
+                               {X[2].x, X[2].y, X[2].z, X[2].w}, {X[3].x, X[3].y, X[3].z, X[3].w}};
+    int4v a[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) a[c] = int4v{0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t w[4] = {(q0[k] & 0x0f0f0f0fu) | ((qh[k] << 4) & 0x30303030u),
+                               (q1[k] & 0x0f0f0f0fu) | ((qh[k] << 2) & 0x30303030u),
+                               ((q0[k] >> 4) & 0x0f0f0f0fu) | (qh[k] & 0x30303030u),
+                               ((q1[k] >> 4) & 0x0f0f0f0fu) | ((qh[k] >> 2) & 0x30303030u)};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            a[c] = __builtin_amdgcn_mfma_i32_4x4x4i8((int)xd[c][k], (int)0xe0e0e0e0u, a[c], 0, 0, 0); // -32
+            a[c] = __builtin_amdgcn_mfma_i32_4x4x4i8((int)xd[c][k], (int)w[c], a[c], 0, 0, 0);
+        }
+    }
+    // 16 products: |256 S2 + S1| < 2^24
+    auto term = [&](const int4v &v, int sc, float m) {
+        const float t = fmaf((float)((v[2] << 8) + v[1]), 256.0f, (float)v[0]);
+        return (float)sc * t * m;
+    };
+    const float t01 = term(a[0], (int8_t)sa, info.x) + term(a[1], (int8_t)(sa >> 16), info.y);
+    const float t23 = term(a[2], (int8_t)sb, info.z) + term(a[3], (int8_t)(sb >> 16), info.w);
+    return d * (t01 + t23);
+}
+
+// Plain GEMV, with the residual epilogue (RESID) or the folded input norm
+// (NORM), or fused gate/up + SwiGLU (GATEUP), as the wide kernels.
+//
+// A workgroup takes gpw consecutive groups of four rows; a unit is one step of
+// a group (GATEUP: of its gate rows or of its up rows), and wave w walks units
+// w, w + NWV, ..., D units' weights in its ring.  The units' row sums wait in
+// LDS for one barrier at the end, where a thread per row adds them in order:
+// the sum does not depend on the launch.  x (and nw) come through the ring's
+// last slots first.
+template <int FMT, bool GATEUP, bool NORM, bool RESID, int NWV, int D, int MAXS>
+__global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restrict__ W,
+                                                        const uint8_t *__restrict__ W2,
+                                                        const float *__restrict__ x, float *y, int outer,
+                                                        int nblk, int gpw, uint32_t inv, const float *__restrict__ nw,
+                                                        float eps, const float *resid, int epi)
+{
+    using F = MdFmt<FMT>;
+    constexpr int NM = GATEUP ? 2 : 1, NT = NWV * 64, PP = F::PIECES, LP = F::PITCH, NC = F::COPIES;
+    constexpr int SLOT = 1024 * NC;
+    constexpr int NX = (MAXS * 256 + NT - 1) / NT; // float4 of x per thread
+    // float4 of x per thread that the ring holds at a time (with nw: both)
+    constexpr int XC = NX < D * NC / (NORM ? 2 : 1) ? NX : D * NC / (NORM ? 2 : 1);
+    static_assert(4 * LP <= 64 * NC && D <= 3, "a unit is NC copies");
+    __shared__ __attribute__((aligned(16))) uint8_t ring[NWV * D * SLOT];
+    __shared__ __attribute__((aligned(16))) uint32_t dig[MAXS * kMdStepDw];
+    __shared__ __attribute__((aligned(16))) float4 pinfo[MAXS * 16];
+    __shared__ float part[kMdUnits * 4];
+    __shared__ float ssw[NWV];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = lane >> 2, r = lane & 3, bq = b >> 2, j = b & 3;
+    const int inner = nblk * 256;
+    const uint32_t row_bytes = (uint32_t)nblk * F::BYTES;
+    const int nstep = (nblk + 3) >> 2;
+    const int ngroups = (outer + 3) >> 2;
+    const int G0 = (int)blockIdx.x * gpw, ng = min(gpw, ngroups - G0);
+    const int units = ng * NM * nstep;
+    const int n = wave < units ? (units - wave - 1) / NWV + 1 : 0; // this wave's
+    // quotients by nstep of numbers up to 16: inv = ceil(65536 / nstep)
+    auto div_steps = [&](int a) { return (int)(((uint32_t)a * inv) >> 16); };
+    const int qn = div_steps(NWV), rn = NWV - qn * nstep;
+
+    // the residual of the thread's first row, ahead of everything else
+    float rv = 0.0f;
+    if constexpr (RESID)
+        rv = resid[min(4 * G0 + tid, outer - 1)];
+
+    uint8_t *const mine = ring + wave * (D * SLOT);
+    const uint32_t mine_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mine;
+
+    // x, then nw: a wave copies what its own threads convert, 1 KB a copy, at
+    // most XC copies of each at a time
+    const int nx = (inner / 4 - 64 * wave + NT - 1) / NT; // its copies of x
+    const int xc = min(nx, XC), raw_slots = ((NORM ? 2 : 1) * xc + NC - 1) / NC;
+    const int pre = max(0, min(n, D - raw_slots)); // units issued before x is there
+    const uint32_t raw = (uint32_t)(D - raw_slots) * SLOT;
+    auto issue_x = [&](int k0) {
+#pragma unroll
+        for (int k = 0; k < XC; ++k)
+            if (k0 + k < nx) {
+                lds_copy16_at(x + 4 * NT * (k0 + k), 16u * (uint32_t)tid, mine_lds + raw + 1024 * k);
+                if constexpr (NORM)
+                    lds_copy16_at(nw + 4 * NT * (k0 + k), 16u * (uint32_t)tid, mine_lds + raw + 1024 * (xc + k));
+            }
+    };
+    issue_x(0);
+
+    // unit u of the workgroup: rows 4 (G0 + g).. of matrix m, step s, with
+    // u = (g NM + m) nstep + s
+    struct Cur {
+        int vg, s;
+    };
+    const int g0 = div_steps(wave);
+    Cur lc = {g0, wave - g0 * nstep}, uc = lc;
+    auto advance = [&](Cur &c) {
+        c.vg += qn;
+        c.s += rn;
+        if (c.s >= nstep) {
+            c.s -= nstep;
+            ++c.vg;
+        }
+    };
+    uint32_t ro[NC], po[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int q = 64 * i + lane, row = min(q / LP, 3);
+        ro[i] = __umul24((uint32_t)row, row_bytes);
+        po[i] = 16u * (uint32_t)min(q - row * LP, PP - 1);
+    }
+    int islot = 0;
+    auto issue = [&]() {
+        const int row0 = 4 * (G0 + (GATEUP ? lc.vg >> 1 : lc.vg));
+        const uint8_t *base = (GATEUP && (lc.vg & 1) ? W2 : W) + (size_t)row0 * row_bytes + (size_t)lc.s * (4 * F::BYTES);
+        // rows past the last, and blocks past the row: the last one again
+        const uint32_t rmax = (uint32_t)(min(outer - row0, 4) - 1) * row_bytes;
+        const uint32_t nbytes = (uint32_t)min(nblk - 4 * lc.s, 4) * F::BYTES;
+        const uint32_t phase = FMT == kQ6_K ? (uint32_t)(uintptr_t)base & 15u : 0u;
+        base -= phase;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            uint32_t o = min(ro[i], rmax);
+            if constexpr (FMT == kQ6_K) { // from the 16-byte unit of the row's first byte
+                o += phase;
+                o = (o & ~15u) + min(po[i], ((o & 15u) + nbytes - 1u) & ~15u);
+            } else {
+                o += min(po[i], nbytes - 16u);
+            }
+            lds_copy16_at(base, o, mine_lds + SLOT * islot + 1024 * i);
+        }
+        islot = islot == D - 1 ? 0 : islot + 1;
+        advance(lc);
+    };
+    for (int i = 0; i < pre; ++i)
+        issue();
+    auto wait_units = [&](int later) { // all copies but those of the last `later` units
+        if (later >= 3)
+            __builtin_amdgcn_s_waitcnt((3 * NC) | 0x0f70);
+        else if (later == 2)
+            __builtin_amdgcn_s_waitcnt((2 * NC) | 0x0f70);
+        else if (later == 1)
+            __builtin_amdgcn_s_waitcnt(NC | 0x0f70);
+        else
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+        asm volatile("" ::: "memory");
+    };
+    wait_units(pre);
+    float ssq = 0.0f;
+#pragma unroll
+    for (int k0 = 0; k0 < NX; k0 += XC) {
+        if (k0 > 0) { // then no slot holds weights yet
+            if (k0 >= nx)
+                break;
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            asm volatile("" ::: "memory");
+            issue_x(k0);
+            wait_units(0);
+        }
+#pragma unroll
+        for (int k = 0; k < XC; ++k)
+            if (k0 + k < nx) {
+                float4 v = *reinterpret_cast<const float4 *>(mine + raw + 1024 * k + 16 * lane);
+                if constexpr (NORM) {
+                    const float4 w = *reinterpret_cast<const float4 *>(mine + raw + 1024 * (xc + k) + 16 * lane);
+                    ssq = fmaf(v.x, v.x, ssq);
+                    ssq = fmaf(v.y, v.y, ssq);
+                    ssq = fmaf(v.z, v.z, ssq);
+                    ssq = fmaf(v.w, v.w, ssq);
+                    v = make_float4(v.x * w.x, v.y * w.y, v.z * w.z, v.w * w.w);
+                }
+                md_stage4<FMT>(v, tid + NT * (k0 + k), dig, pinfo);
+            }
+    }
+    if constexpr (NORM) {
+        const float t = wave_sum(ssq);
+        if (lane == 0)
+            ssw[wave] = t;
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f); // the raw values are read, the digits written
+    asm volatile("" ::: "memory");
+    for (int i = pre; i < min(n, D); ++i)
+        issue();
+    lds_barrier();
+
+    int slot = 0;
+    for (int i = 0; i < n; ++i) {
+        wait_units(min(D, n - i) - 1);
+        const uint8_t *row = mine + SLOT * slot + r * (LP * 16);
+        slot = slot == D - 1 ? 0 : slot + 1;
+        uint4 X[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            X[t] = *reinterpret_cast<const uint4 *>(dig + uc.s * kMdStepDw + t * kMdPlaneDw + 4 * lane);
+        const float4 info = pinfo[16 * uc.s + b];
+        float c;
+        if constexpr (FMT == kQ6_K) {
+            const int vg = GATEUP ? uc.vg >> 1 : uc.vg, row0 = 4 * (G0 + vg);
+            const uint32_t at = (uint32_t)(uintptr_t)(GATEUP && (uc.vg & 1) ? W2 : W) +
+                                (uint32_t)(row0 + min(r, outer - 1 - row0)) * row_bytes + (uint32_t)uc.s * (4 * F::BYTES);
+            // blocks past the row's end read stale bytes of the slot, unused
+            const uint32_t byte = (at & 15u) + (uint32_t)bq * F::BYTES;
+            c = mdig_dot_q6(row + (byte & ~3u), byte & 2u, j >> 1, j & 1, X, info);
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            asm volatile("" ::: "memory");
+            if (i + D < n)
+                issue();
+        } else {
+            KBytes B;
+            kbytes_load<FMT>(row + bq * F::BYTES, j, B);
+            __builtin_amdgcn_s_waitcnt(0xc07f); // in registers: the slot is free
+            asm volatile("" ::: "memory");
+            if (i + D < n)
+                issue();
+            c = mdig_dot<FMT>(B, j, X, info);
+        }
+        // over the lanes of row r: 16 lanes' four, then the four rows of lanes
+        float v = 4 * uc.s + bq < nblk ? c : 0.0f;
+        v = dpp_add<0x128, 0xf>(v); // row_ror:8
+        v = dpp_add<0x124, 0xf>(v); // row_ror:4
+        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float((uint32_t)h[0]) + __uint_as_float((uint32_t)h[1]);
+        const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float((uint32_t)q[0]) + __uint_as_float((uint32_t)q[1]);
+        if (lane < 4)
+            part[(wave + NWV * i) * 4 + lane] = v;
+        advance(uc);
+    }
+    __syncthreads();
+
+    float scale = 1.0f;
+    if constexpr (NORM) {
+        float tot = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NWV; ++i)
+            tot += ssw[i];
+        scale = 1.0f / sqrtf(tot / (float)inner + eps);
+    }
+    for (int t = tid; t < 4 * ng; t += NT) {
+        const int row = 4 * G0 + t;
+        if (row >= outer)
+            break;
+        float v[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const float *p = part + ((t >> 2) * NM + m) * nstep * 4 + (t & 3);
+            float a = 0.0f;
+#pragma unroll
+            for (int s0 = 0; s0 < MAXS; s0 += 4) {
+                if (s0 >= nstep)
+                    break;
+                float q[4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) q[s] = p[4 * min(s0 + s, nstep - 1)];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) a += s0 + s < nstep ? q[s] : 0.0f;
+            }
+            v[m] = a * scale;
+        }
+        if constexpr (GATEUP)
+            y[row] = (v[0] / (1.0f + expf(-v[0]))) * v[NM - 1]; // src/ModelCPU.jl:492-503
+        else if constexpr (RESID)
+            y[row] = epi_apply(t == tid ? rv : resid[row], v[0], epi);
+        else
+            y[row] = v[0];
+    }
 }
 
 // Persistent form of the digit kernel for matrices of many rows and at most
@@ -655,190 +1074,6 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kpers(const uint8_t *__restri
     __shared__ float ssw[NWV];
     kpers_run<FMT, R, GATEUP, GATEUP && EXT, !GATEUP && EXT, NWV, NB>(W, W2, x, y, outer, nblk, nw, eps,
                                                                       resid, epi, xbuf, xsum, xexp, ssw);
-}
-
-// The persistent kernel with the folded norm on a single weight,
-// y = W (rmsnorm(x) .* nw) (as k_gemv_kwide_norm, for rows of at most 16
-// blocks past the per-workgroup kernel's row count).
-template <int FMT, int R, int NWV, int NB>
-__global__ __launch_bounds__(NWV * 64) void k_gemv_kpers_norm(const uint8_t *__restrict__ W,
-                                                         const float *__restrict__ x, float *y,
-                                                         int outer, int nblk,
-                                                         const float *__restrict__ nw, float eps)
-{
-    __shared__ __attribute__((aligned(16))) uint32_t xbuf[3 * kDigPlaneDw];
-    __shared__ __attribute__((aligned(16))) float xsum[128];
-    __shared__ __attribute__((aligned(8))) int xexp[128];
-    __shared__ float ssw[NWV];
-    kpers_run<FMT, R, false, true, false, NWV, NB>(W, nullptr, x, y, outer, nblk, nw, eps, nullptr, 0,
-                                                   xbuf, xsum, xexp, ssw);
-}
-
-// Persistent form for rows of more than 16 blocks (2..MP passes of 4096
-// columns).  One workgroup per CU stages x's digits for every pass once, in
-// LDS (x loads of all passes issued together, clamped to the last pass so
-// none is predicated).  Each wave then walks items (row group, pass) --
-// groups grid-stride, a group's passes in order -- through NB register
-// buffers, so the next items' weights are in flight while one is reduced
-// and a row's short last pass costs its own bytes rather than a whole
-// pass's latency.  Lanes accumulate across a group's passes and the row sum
-// is taken after its last pass: the same arithmetic in the same order as
-// k_gemv_kwide's serial passes, so the outputs are bit-identical.
-template <int FMT, int R, bool GATEUP, bool EXT, int NWV, int NB, int MP>
-__global__ __launch_bounds__(NWV * 64) void k_gemv_kpm(const uint8_t *__restrict__ W,
-                                                       const uint8_t *__restrict__ W2,
-                                                       const float *__restrict__ x,
-                                                       float *y, int outer, int nblk,
-                                                       const float *__restrict__ nw, float eps,
-                                                       const float *resid, int epi)
-{
-    using F = KFmt<FMT>;
-    constexpr int NM = GATEUP ? 2 : 1;
-    constexpr bool NORM = GATEUP && EXT, RESID = !GATEUP && EXT;
-    constexpr int NT = NWV * 64, NXV = xnv(NT);
-    __shared__ __attribute__((aligned(16))) uint32_t xbuf[MP * 3 * kDigPlaneDw];
-    __shared__ __attribute__((aligned(16))) float xsum[MP * 128];
-    __shared__ __attribute__((aligned(8))) int xexp[MP * 128];
-    __shared__ float ssw[NWV];
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b = lane >> 2, j = lane & 3;
-    const int inner = nblk * 256;
-    const int npass = (nblk + 15) >> 4; // 2..MP (the launcher checks)
-    const size_t row_bytes = (size_t)nblk * F::BYTES;
-    const int ngroups = (outer + R - 1) / R;
-    const int stride = gridDim.x * NWV;
-    const int g0 = blockIdx.x * NWV + wave;
-    // this wave's items: groups g0, g0 + stride, ... each with npass passes
-    const int nitems = g0 < ngroups ? ((ngroups - 1 - g0) / stride + 1) * npass : 0;
-
-    auto load = [&](KBytes (&B)[NM][R], float (&RV)[R], int t) {
-        const int k = t / npass, p = t - k * npass; // wave-uniform
-        const int gi = min(g0 + k * stride, ngroups - 1);
-        const int blk = p * 16 + (b < min(16, nblk - p * 16) ? b : 0);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int row = min(gi * R + r, outer - 1);
-            if constexpr (RESID)
-                RV[r] = resid[row]; // wave-uniform: a scalar load
-#pragma unroll
-            for (int m = 0; m < NM; ++m)
-                kbytes_load<FMT>((m == 0 ? W : W2) + (size_t)row * row_bytes + (size_t)blk * F::BYTES,
-                                 j, B[m][r]);
-        }
-    };
-
-    // x of every pass (MP passes of loads, the ones past npass repeating the
-    // last), then the first NB items' weights, then the digits into LDS
-    float4 xv[MP][NXV];
-#pragma unroll
-    for (int p = 0; p < MP; ++p)
-        x_load_pass<NT>(x, min(p, npass - 1) * 4096, inner, xv[p]);
-    float ssq = 0.0f;
-    if constexpr (NORM) {
-#pragma unroll
-        for (int p = 0; p < MP; ++p) {
-            float4 wv[NXV];
-            x_load_pass<NT>(nw, min(p, npass - 1) * 4096, inner, wv);
-            if (p < npass) { // wave-uniform; the loads above are not under it
-#pragma unroll
-                for (int k = 0; k < NXV; ++k) {
-                    ssq = fmaf(xv[p][k].x, xv[p][k].x, ssq);
-                    ssq = fmaf(xv[p][k].y, xv[p][k].y, ssq);
-                    ssq = fmaf(xv[p][k].z, xv[p][k].z, ssq);
-                    ssq = fmaf(xv[p][k].w, xv[p][k].w, ssq);
-                    xv[p][k] = make_float4(xv[p][k].x * wv[k].x, xv[p][k].y * wv[k].y,
-                                           xv[p][k].z * wv[k].z, xv[p][k].w * wv[k].w);
-                }
-            }
-        }
-    }
-    KBytes B[NB][NM][R];
-    float RV[NB][R];
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-        load(B[q], RV[q], q);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int p = 0; p < MP; ++p)
-        if (p < npass)
-            x_stage_dig<NT>(xbuf + p * 3 * kDigPlaneDw, xsum + p * 128, xexp + p * 128, xv[p]);
-    float scale = 1.0f;
-    if constexpr (NORM) {
-        const float t = wave_sum(ssq);
-        if (lane == 0)
-            ssw[wave] = t;
-        __syncthreads();
-        float tot = 0.0f;
-#pragma unroll
-        for (int i = 0; i < NWV; ++i)
-            tot += ssw[i];
-        scale = 1.0f / sqrtf(tot / (float)inner + eps);
-    } else {
-        __syncthreads();
-    }
-
-    float acc[NM][R];
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[m][r] = 0.0f;
-
-    auto reduce = [&](const KBytes (&Bq)[NM][R], const float (&RVq)[R], int t) {
-        const int k = t / npass, p = t - k * npass; // wave-uniform
-        const int gi = g0 + k * stride;
-        const bool active = b < min(16, nblk - p * 16);
-        XDig X;
-        x_from_lds_dig(xbuf + p * 3 * kDigPlaneDw, xsum + p * 128, xexp + p * 128, b, j, X);
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                const float c = kdig_dot<FMT>(Bq[m][r], j, X);
-                acc[m][r] += active ? c : 0.0f;
-            }
-        if (p == npass - 1) { // the group's last pass: its rows are done
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int row = gi * R + r;
-                float v[NM];
-#pragma unroll
-                for (int m = 0; m < NM; ++m) {
-                    v[m] = wave_sum(acc[m][r]) * scale;
-                    acc[m][r] = 0.0f;
-                }
-                float o = v[0];
-                if constexpr (GATEUP)
-                    o = (v[0] / (1.0f + expf(-v[0]))) * v[1]; // src/ModelCPU.jl:492-503
-                // every lane holds the row's value: an unpredicated store (a
-                // row past `outer` rewrites row outer - 1 with its own value)
-                y[min(row, outer - 1)] = RESID ? epi_apply(RVq[r], o, epi) : o;
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    // steady state: every buffer is refilled with an item that exists
-    int t = 0;
-    for (; t + (2 * NB - 1) < nitems; t += NB) { // wave-uniform
-#pragma unroll
-        for (int q = 0; q < NB; ++q) {
-            reduce(B[q], RV[q], t + q);
-            load(B[q], RV[q], t + q + NB);
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-        if (t + q < nitems)
-            reduce(B[q], RV[q], t + q);
-        if (t + q + NB < nitems)
-            load(B[q], RV[q], t + q + NB);
-    }
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-        if (t + q + NB < nitems)
-            reduce(B[q], RV[q], t + q + NB);
 }
 
 // ------------------------------------------------------------------------
@@ -1539,17 +1774,11 @@ int device_cus()
     return ncu;
 }
 
-// Rows of 17..64 blocks whose 8-wave workgroups (two rows per wave for the
-// GEMV, one gate/up row pair for the fused gate/up) would not divide evenly
-// over the CUs take the persistent multi-pass kernel; the fused gate/up only
-// with more row pairs than one per wave of one workgroup per CU (5120 ->
-// 1280 5.5 us serial against 5.9, 8192 -> 1024 6.1 against 6.4; 5120 ->
-// 13824 20.6-21.2 against 26.0-26.4).
-static bool kwide_takes_kpm(int nblk, int outer, bool gateup)
+// IQ4_NL rows of 17..64 256-column units whose two-row, 8-wave workgroups
+// would not divide evenly over the CUs.
+static bool kwide_uneven(int nblk, int outer)
 {
-    const int R = gateup ? 1 : 2;
-    return nblk > 16 && nblk <= 4 * 16 && ((outer + 8 * R - 1) / (8 * R)) % device_cus() != 0 &&
-           (!gateup || (outer + 7) / 8 > device_cus());
+    return nblk > 16 && nblk <= 4 * 16 && ((outer + 15) / 16) % device_cus() != 0;
 }
 
 // Rows of at most 16 blocks with at least four 8-wave row groups per wave
@@ -1559,32 +1788,76 @@ static bool kwide_takes_kpers(int nblk, int outer) { return nblk <= 16 && outer 
 // No more one-row workgroups of 8 waves than CUs: one row per wave.
 static bool kwide_one_row(int outer) { return (outer + 7) / 8 <= device_cus(); }
 
-// k_gemv_kpm with the smallest pass capacity that holds the row.
-template <int FMT, bool GATEUP, bool EXT>
-static void launch_kpm(int npass, int grid, const uint8_t *W, const uint8_t *W2, const float *x,
-                       float *y, int outer, int nblk, const float *nw, float eps, const float *resid,
-                       int epi, hipStream_t s)
+// Rows of at most 64 blocks on the matrix cores: waves and ring depth by the
+// row's steps (Q6_K: its 4 KB slots leave 8 waves beside the digits of more
+// than 12 steps).
+struct MdPlan {
+    int nw, d, maxs;
+};
+constexpr MdPlan mdig_plan(int type, int nblk)
 {
-    constexpr int NWV = 8, NB = 2;
-    if (npass <= 2)
-        hipLaunchKernelGGL((k_gemv_kpm<FMT, 1, GATEUP, EXT, NWV, NB, 2>), dim3(grid), dim3(NWV * 64), 0, s,
-                           W, W2, x, y, outer, nblk, nw, eps, resid, epi);
-    else
-        hipLaunchKernelGGL((k_gemv_kpm<FMT, 1, GATEUP, EXT, NWV, NB, 4>), dim3(grid), dim3(NWV * 64), 0, s,
-                           W, W2, x, y, outer, nblk, nw, eps, resid, epi);
+    if (nblk <= 16)
+        return {8, 3, 4};
+    if (type == kQ6_K)
+        return nblk <= 48 ? MdPlan{12, 2, 12} : MdPlan{8, 2, 16};
+    return {12, 2, 16};
+}
+// Which rows take it, by format, length and (gate/up) kind only: a row's sum is
+// the same whatever launch it is in, and the two kernels' differ.  The wide
+// kernels spread a row's blocks over 16 lane positions, this one over 4 a
+// step, and it starts later (x goes through LDS twice).  So the wide kernels
+// keep the Q4_K / Q5_K rows that fill their lanes, and the short Q4_K ones.
+// Measured on MI355X (us, graph replays over weights in HBM, wide / this):
+// Q4_K 2560 x 9728 8.6 / 6.3, 5120 x 5120 7.8 / 5.6, 4096 x 14336 10.6 / 9.9,
+// 4096 x 4096 4.1 / 4.6, 12288 x 4096 7.4 / 7.8, 3584 x 2560 3.45 / 3.73; Q5_K
+// 4096 x 2048 4.1 / 3.5, 9728 x 2560 7.4 / 6.5, 4096 x 4096 4.8 / 5.1; gate/up
+// Q4_K 6144 x 2048 7.2 / 5.7, 13824 x 5120 20.6 / 17.2, 10240 x 3584 11.0 / 10.5,
+// 12288 x 4096 12.8 / 13.0; Q5_K 9728 x 2560 12.3 / 9.7, 12288 x 4096 15.8 / 15.5;
+// the folded norm Q4_K 6144 x 4096 6.6 / 6.0.  Q6_K (streamed / this) 4096 x
+// 12288 12.4 / 11.7, 2560 x 9728 12.1 / 7.9, 5120 x 13824 26.9 / 15.9, 1024 x 4096
+// 4.9 / 3.6, 12288 x 4096 11.2 / 11.5.
+constexpr int kMdMaxBlocks = 64;
+constexpr bool mdig_takes(int type, int nblk, bool gateup)
+{
+    if (nblk > kMdMaxBlocks)
+        return false;
+    if (type == kQ6_K || nblk > 16)
+        return true;
+    if (gateup)
+        return type == kQ5_K || nblk <= 14;
+    return type == kQ5_K && nblk <= 12;
+}
+template <int FMT, bool GATEUP, bool NORM, bool RESID>
+static void launch_mdig(const uint8_t *W, const uint8_t *W2, const float *x, float *y, int nblk, int outer,
+                        const float *nw, float eps, const float *resid, int epi, hipStream_t s)
+{
+    const int nstep = (nblk + 3) / 4, ngroups = (outer + 3) / 4;
+    const int gpw = std::min((ngroups + device_cus() - 1) / device_cus(), kMdUnits / (nstep * (GATEUP ? 2 : 1)));
+    const dim3 grid((ngroups + gpw - 1) / gpw);
+    const uint32_t inv = (65536u + nstep - 1) / nstep;
+    const MdPlan p = mdig_plan(FMT, nblk);
+    if (p.maxs == 4)
+        hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 8, 3, 4>), grid, dim3(8 * 64), 0, s, W, W2, x, y,
+                           outer, nblk, gpw, inv, nw, eps, resid, epi);
+    else if constexpr (FMT == kQ6_K) {
+        if (p.maxs == 12)
+            hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 12, 2, 12>), grid, dim3(12 * 64), 0, s, W, W2, x,
+                               y, outer, nblk, gpw, inv, nw, eps, resid, epi);
+        else
+            hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 8, 2, 16>), grid, dim3(8 * 64), 0, s, W, W2, x, y,
+                               outer, nblk, gpw, inv, nw, eps, resid, epi);
+    } else
+        hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 12, 2, 16>), grid, dim3(12 * 64), 0, s, W, W2, x, y,
+                           outer, nblk, gpw, inv, nw, eps, resid, epi);
 }
 
-// Q4_K / Q5_K: 8-wave workgroups; two rows per wave for the GEMV, one gate and
-// one up row per wave for the fused gate/up (measured on MI355X at 4096 x 4096
-// and 2 x 12288 x 4096).  Rows of at most 4096 columns with at least four row
-// groups per wave over one workgroup per CU take the persistent kernel (2 x
-// 12288 x 4096 gate/up 12.7 us against 13.9 us; at 4096 x 4096 one row group
-// per wave is all there is and the plain kernel is faster).  Rows of 17..64
-// blocks take the persistent multi-pass kernel when the serial kernel's
-// workgroups do not divide evenly over the CUs (5120 x 5120 7.8-8.8 us
-// against 8.5-8.6, 5120 x 13824 13.9-15.1 against 16.2-16.4, 13824 x 5120
-// 14.6-14.9 against 15.4-15.6); at 4096 rows the serial kernel's one
-// workgroup per CU is faster (4096 x 11008 9.7-10.0 us against 10.7-11.2).
+// Rows that k_gemv_mdig does not take: 8-wave workgroups; two rows per wave
+// for the GEMV, one gate and one up row per wave for the fused gate/up
+// (measured on MI355X at 4096 x 4096 and 2 x 12288 x 4096).  Rows of at most
+// 4096 columns with at least four row groups per wave over one workgroup per
+// CU take the persistent kernel (2 x 12288 x 4096 gate/up 12.7 us against
+// 13.9 us; at 4096 x 4096 one row group per wave is all there is and the plain
+// kernel is faster).
 template <int FMT, bool GATEUP>
 static hipError_t launch_kwide(const void *w, const void *w2, const float *x, float *y,
                                int inner, int outer, hipStream_t s, const float *nw = nullptr,
@@ -1594,23 +1867,26 @@ static hipError_t launch_kwide(const void *w, const void *w2, const float *x, fl
     const int nblk = inner / 256;
     const bool ext = GATEUP ? nw != nullptr : resid != nullptr;
     const uint8_t *W = (const uint8_t *)w, *W2 = (const uint8_t *)w2;
-    if (kwide_takes_kpers(nblk, outer)) {
+    if constexpr (FMT == kQ4_K || FMT == kQ5_K) {
+        if (mdig_takes(FMT, nblk, GATEUP)) {
+            if (ext)
+                launch_mdig<FMT, GATEUP, GATEUP, !GATEUP>(W, W2, x, y, nblk, outer, nw, eps, resid, epi, s);
+            else
+                launch_mdig<FMT, GATEUP, false, false>(W, W2, x, y, nblk, outer, nw, eps, resid, epi, s);
+            return hipGetLastError();
+        }
+    }
+    constexpr bool kPers = !(GATEUP && FMT == kQ5_K); // those rows are all taken above
+    if (kPers && kwide_takes_kpers(nblk, outer)) {
         const int grid = std::max(1, std::min(device_cus(), (outer + NWV - 1) / NWV));
-        if (ext)
+        if constexpr (!kPers)
+            return hipErrorInvalidValue;
+        else if (ext)
             hipLaunchKernelGGL((k_gemv_kpers<FMT, 1, GATEUP, true, NWV, NB>), dim3(grid), dim3(NWV * 64),
                                0, s, W, W2, x, y, outer, nblk, nw, eps, resid, epi);
         else
             hipLaunchKernelGGL((k_gemv_kpers<FMT, 1, GATEUP, false, NWV, NB>), dim3(grid), dim3(NWV * 64),
                                0, s, W, W2, x, y, outer, nblk, nw, eps, resid, epi);
-    } else if (FMT != kIQ4_NL && FMT != kQ8_0 && kwide_takes_kpm(nblk, outer, GATEUP)) {
-        if constexpr (FMT != kIQ4_NL && FMT != kQ8_0) {
-            const int grid = std::max(1, std::min(device_cus(), (outer + NWV - 1) / NWV));
-            const int npass = (nblk + 15) / 16;
-            if (ext)
-                launch_kpm<FMT, GATEUP, true>(npass, grid, W, W2, x, y, outer, nblk, nw, eps, resid, epi, s);
-            else
-                launch_kpm<FMT, GATEUP, false>(npass, grid, W, W2, x, y, outer, nblk, nw, eps, resid, epi, s);
-        }
     } else if (!GATEUP && kwide_one_row(outer)) {
         // no more one-row workgroups than CUs: one row per wave, all of them
         // at once (2048 x 2048 2.8-3.1 us against 3.5-3.6 with two rows per
@@ -1701,7 +1977,15 @@ hipError_t launch_gemv(int type, const void *w, const float *x, float *y, int in
     switch (type) {
     case kQ4_K: return launch_kwide<kQ4_K, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi);
     case kQ5_K: return launch_kwide<kQ5_K, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi);
-    case kQ6_K: return launch_sdig<kQ6_K, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
+    case kQ6_K:
+        if (mdig_takes(type, inner / 256, false)) {
+            if (resid)
+                launch_mdig<kQ6_K, false, false, true>((const uint8_t *)w, nullptr, x, y, inner / 256, outer, nullptr, 0.0f, resid, epi, s);
+            else
+                launch_mdig<kQ6_K, false, false, false>((const uint8_t *)w, nullptr, x, y, inner / 256, outer, nullptr, 0.0f, nullptr, epi, s);
+            return hipGetLastError();
+        }
+        return launch_sdig<kQ6_K, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     case kQ8_0:
         // rows of one pass (at most 4096 columns in whole 256-column units)
         // on the wide lane layout, measured against the streamed kernel in one
@@ -1714,10 +1998,9 @@ hipError_t launch_gemv(int type, const void *w, const float *x, float *y, int in
                    : launch_sdig<kQ8_0, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     case kIQ4_NL:
         // rows of whole 256-column units take the wide kernels' lane layout,
-        // except where the persistent multi-pass kernel would run (its IQ4_NL
-        // dot from LDS digits measured slower than the streamed kernel:
-        // 5120 x 5120 10.9 us against 10.3)
-        return inner % 256 == 0 && !kwide_takes_kpm(inner / 256, outer, false)
+        // except several passes on an uneven grid (5120 x 5120: the streamed
+        // kernel 10.3 us)
+        return inner % 256 == 0 && !kwide_uneven(inner / 256, outer)
                    ? launch_kwide<kIQ4_NL, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi)
                    : launch_sdig<kIQ4_NL, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     default: return hipErrorInvalidValue;
@@ -1729,34 +2012,15 @@ bool gemv_norm_fusable(int type, int inner, int)
     return (type == kQ4_K || type == kQ5_K) && inner % 256 == 0 && inner / 256 <= 16;
 }
 
-template <int FMT>
-static void launch_kwide_norm(const void *w, const float *x, const float *nw, float eps, float *y,
-                              int inner, int outer, hipStream_t s)
-{
-    constexpr int NWV = 8;
-    const int nblk = inner / 256;
-    const uint8_t *W = (const uint8_t *)w;
-    if (kwide_takes_kpers(nblk, outer))
-        hipLaunchKernelGGL((k_gemv_kpers_norm<FMT, 1, NWV, 2>),
-                           dim3(std::max(1, std::min(device_cus(), (outer + NWV - 1) / NWV))),
-                           dim3(NWV * 64), 0, s, W, x, y, outer, nblk, nw, eps);
-    else if (kwide_one_row(outer))
-        hipLaunchKernelGGL((k_gemv_kwide_norm<FMT, 1, NWV>), dim3((outer + NWV - 1) / NWV), dim3(NWV * 64),
-                           0, s, W, x, y, outer, nblk, nw, eps);
-    else
-        hipLaunchKernelGGL((k_gemv_kwide_norm<FMT, 2, NWV>), dim3((outer + 2 * NWV - 1) / (2 * NWV)),
-                           dim3(NWV * 64), 0, s, W, x, y, outer, nblk, nw, eps);
-}
-
 hipError_t launch_gemv_norm(int type, const void *w, const float *x, const float *nw, float eps,
                             float *y, int inner, int outer, hipStream_t s)
 {
     if (!gemv_norm_fusable(type, inner, outer))
         return hipErrorNotSupported;
     if (type == kQ4_K)
-        launch_kwide_norm<kQ4_K>(w, x, nw, eps, y, inner, outer, s);
+        launch_mdig<kQ4_K, false, true, false>((const uint8_t *)w, nullptr, x, y, inner / 256, outer, nw, eps, nullptr, 0, s);
     else
-        launch_kwide_norm<kQ5_K>(w, x, nw, eps, y, inner, outer, s);
+        launch_mdig<kQ5_K, false, true, false>((const uint8_t *)w, nullptr, x, y, inner / 256, outer, nw, eps, nullptr, 0, s);
     return hipGetLastError();
 }
 
