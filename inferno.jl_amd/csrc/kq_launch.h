@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace ihip {
 
 // kq_gemv.hip
@@ -175,17 +177,46 @@ inline double prefill_cost(int tiles, int nblk, int ncu, double fixed, double co
     const double u = (double)tiles / ncu, c = (double)((tiles + ncu - 1) / ncu);
     return fixed + nblk * (col + per_u * u + per_c * c);
 }
-inline int prefill_wide_rows(int T, int inner, int outer, int ncu)
+struct PrefillCosts {
+    double narrow, wide1, wide2; // 64 x 128 (with its splits), 128 x 128, 128 x 256
+};
+inline PrefillCosts prefill_costs(int T, int inner, int outer, int ncu)
 {
     const int nblk = inner / 256, cus = ncu > 0 ? ncu : 1;
-    const int nsplit = prefill_splits(T, inner, outer, ncu);
-    if (nsplit > 1)
-        return 0; // few tiles of either size: K is shared out instead
     auto tiles = [&](int bm, int bn) { return ((T + bm - 1) / bm) * ((outer + bn - 1) / bn); };
-    const double c0 = prefill_cost(tiles(kPrefillBM, kPrefillBN), nblk, cus, 6.6, -0.37, 0.53, 0.99);
-    const double c1 = prefill_cost(tiles(kPrefillWideBM, 128), nblk, cus, 4.5, 0.20, 0.63, 1.23);
-    const double c2 = prefill_cost(tiles(kPrefillWideBM, 256), nblk, cus, 6.5, -0.10, 1.13, 2.44);
-    return c0 <= c1 && c0 <= c2 ? 0 : c1 <= c2 ? 1 : 2;
+    const int nsplit = prefill_splits(T, inner, outer, ncu);
+    PrefillCosts c;
+    c.narrow = prefill_cost(tiles(kPrefillBM, kPrefillBN), nblk, cus, 6.6, -0.37, 0.53, 0.99);
+    if (nsplit > 1) // the split's share of the columns, then its planes' traffic and the summing launch
+        c.narrow = 8.17 + (double)nblk / nsplit * (0.70 + 0.63 * tiles(kPrefillBM, kPrefillBN) * nsplit / cus) +
+                   1.07e-6 * T * outer * nsplit;
+    c.wide1 = prefill_cost(tiles(kPrefillWideBM, 128), nblk, cus, 4.5, 0.20, 0.63, 1.23);
+    c.wide2 = prefill_cost(tiles(kPrefillWideBM, 256), nblk, cus, 6.5, -0.10, 1.13, 2.44);
+    return c;
+}
+inline int prefill_wide_rows(int T, int inner, int outer, int ncu)
+{
+    if (prefill_splits(T, inner, outer, ncu) > 1)
+        return 0; // few tiles of either size: K is shared out instead
+    const PrefillCosts c = prefill_costs(T, inner, outer, ncu);
+    return c.narrow <= c.wide1 && c.narrow <= c.wide2 ? 0 : c.wide1 <= c.wide2 ? 1 : 2;
+}
+// Whether it takes the 32-token x 64-row tiles whose waves share K instead
+// (k_prefill_q4k_thin): by the same estimate, fitted to 105 shapes of 8 to 1024
+// tokens timed in graph replays (relative rms 9 %; the split 64 x 128 tile 5 %).
+// Over them the choice is never over 2 % slower than without this kernel,
+// 1.13 times as fast on average and 0.2 % from the faster of the two.
+constexpr int kPrefillThinBM = 32, kPrefillThinBN = 64;
+inline bool prefill_thin(int T, int inner, int outer, int ncu)
+{
+    const int nblk = inner / 256, cus = ncu > 0 ? ncu : 1;
+    const int64_t tiles = ((int64_t)T + kPrefillThinBM - 1) / kPrefillThinBM * (((int64_t)outer + kPrefillThinBN - 1) / kPrefillThinBN);
+    if (tiles > 16 * (int64_t)cus)
+        return false; // a product of many tiles
+    const double thin = prefill_cost((int)tiles, nblk, cus, 3.55, -0.154 + 0.1 * std::min(T, 32) / 32, 0.074, 0.577);
+    const int ru = prefill_wide_rows(T, inner, outer, ncu);
+    const PrefillCosts c = prefill_costs(T, inner, outer, ncu);
+    return thin < (ru == 0 ? c.narrow : ru == 1 ? c.wide1 : c.wide2);
 }
 hipError_t launch_prefill_q4k(const void *w, const float *X, void *xh, float *Y, int T,
                               int inner, int outer, hipStream_t s);

@@ -819,6 +819,215 @@ __global__ __launch_bounds__(256, RU == 2 ? 2 : 3) void k_prefill_q4k_wide(
     }
 }
 
+// Small products: 32 tokens x 64 weight rows per workgroup of 8 waves that share
+// K.  Wave (half, j) takes sub-block pair j of the block columns 2 i + half and
+// accumulates the whole tile, so every activation and every weight byte of
+// the tile is read and dequantized by one wave only, each wave copies its own
+// operands through LDS and waits for nothing but them, and a weight of few
+// rows still has eight waves at work on each tile.  A step's operands go to
+// registers before its products, which frees the wave's LDS for the next
+// step's copies; two workgroups share a CU (57 KB).  The eight partial tiles
+// are added up in LDS in a fixed order: waves w and w + 4, then 0..3.
+//
+// Bound by the copies (a 48-byte piece of a weight row touches three or four
+// cache lines a quad of lanes): wider tiles (64 to 128 tokens, 128 rows) copy
+// less but leave CUs idle, and were slower wherever this kernel is taken.
+// Measured on MI355X (us, graph replays, the 64 x 128 tile / this): 8 x 1024 x
+// 2048 (tokens x columns x rows) 8.9 / 5.3, 256 x 1024 x 2048 10.8 / 6.2, 8 x 2560
+// x 9728 11.7 / 7.7, 77 x 2560 x 9728 16.2 / 14.7, 128 x 4096 x 4096 15.4 / 11.8, 512
+// x 2048 x 512 11.0 / 8.1.
+constexpr int PFT_BM = kPrefillThinBM, PFT_BN = kPrefillThinBN, PFT_RU = PFT_BN / 32;
+constexpr int PFT_X = 4096, PFT_WAVE = PFT_X + 48 * PFT_BN; // bytes of a wave's step: 64 columns of X, the rows' pieces
+constexpr int PFT_LD = PFT_BN + 4;                          // floats between two tokens of a partial tile
+static_assert(PFT_BM == 32 && 8 * PFT_WAVE >= 4 * 4 * PFT_BM * PFT_LD, "four partial tiles fit the waves' LDS");
+
+template <bool EXACTW>
+__global__ __launch_bounds__(512, 2) void k_prefill_q4k_thin(const uint8_t *__restrict__ W,
+                                                             const _Float16 *__restrict__ Xh,
+                                                             const int *__restrict__ xs, float *__restrict__ Y,
+                                                             int T, int K, int N, int mtiles, int ntiles)
+{
+    constexpr int RU = PFT_RU, XC = 4, WC = 3 * PFT_BN / 64; // 1 KB copies of a step
+    constexpr int LD = PFT_LD;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[8 * PFT_WAVE];
+
+    const int tiles = mtiles * ntiles;
+    const int lin = prefill_lin((int)blockIdx.x, tiles, 1);
+    if (lin >= tiles)
+        return; // whole workgroup
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, li = lane & 31, j = wave & 3, half = wave >> 2;
+    const int nk = K / 256;
+    const uint32_t row_bytes = (uint32_t)nk * 144u;
+    const PrefillSplit ps = prefill_split_of(lin, mtiles, ntiles, nk, 1);
+    const int m0 = ps.mt * PFT_BM, n0 = ps.nt * PFT_BN;
+
+    float16v acc[RU];
+#pragma unroll
+    for (int u = 0; u < RU; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[u][r] = 0.0f;
+
+    const int nb = (nk - half + 1) >> 1; // this wave's steps
+    if (nb > 0) {
+        // copies: 8 tokens x 8 chunks each of the pair's 64 columns (chunk e of
+        // token m at place e ^ (m / 2 % 8) of its 128 bytes, for the banks),
+        // and header and 32 quant bytes of every row.  Rows past T or N re-read
+        // the last one, steps past the last repeat it.
+        uint32_t xo[XC], wo[WC];
+#pragma unroll
+        for (int i = 0; i < XC; ++i) {
+            const int m = 8 * i + (lane >> 3), e = (lane & 7) ^ ((m >> 1) & 7);
+            xo[i] = 2u * (uint32_t)min(m0 + m, T - 1) * (uint32_t)K + 16u * (uint32_t)pf_chunk_place(8 * j + e);
+        }
+#pragma unroll
+        for (int i = 0; i < WC; ++i) {
+            const int q = 64 * i + lane, row = q / 3, piece = q - 3 * row;
+            wo[i] = (uint32_t)min(n0 + row, N - 1) * row_bytes + (piece ? 32u * j + 16u * piece : 0u);
+        }
+        uint8_t *const mine = lds + PFT_WAVE * wave;
+        const uint32_t xdst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mine;
+        const uint8_t *Xb = reinterpret_cast<const uint8_t *>(Xh) + 512 * half, *Wb = W + 144 * half;
+        auto issue = [&](int i) {
+            const int st = min(i, nb - 1);
+            const uint8_t *x = Xb + (size_t)st * 1024, *w = Wb + (size_t)st * 288;
+#pragma unroll
+            for (int k = 0; k < WC; ++k)
+                pf_copy16(w, wo[k], xdst + PFT_X + 1024 * k);
+#pragma unroll
+            for (int k = 0; k < XC; ++k)
+                pf_copy16(x, xo[k], xdst + 1024 * k);
+        };
+        const uint8_t *xl = mine + 128 * li, *wl = mine + PFT_X + 48 * li;
+        const int f = (li >> 1) & 7;
+        issue(0);
+        for (int i = 0; i < nb; ++i) {
+            __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0): this step's copies
+            asm volatile("" ::: "memory");
+            half8 x[4];
+            uint2 q[RU][2];
+            uint4 hd[RU / 2]; // of the row tiles 2 v + h
+#pragma unroll
+            for (int v = 0; v < RU / 2; ++v)
+                hd[v] = *reinterpret_cast<const uint4 *>(wl + 32 * 48 * (2 * v + h));
+#pragma unroll
+            for (int u = 0; u < RU; ++u)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    q[u][c] = *reinterpret_cast<const uint2 *>(wl + 32 * 48 * u + 16 + 16 * c + 8 * h);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                x[s] = *reinterpret_cast<const half8 *>(xl + 16 * ((2 * s + h) ^ f));
+            __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): in registers
+            asm volatile("" ::: "memory");
+            issue(i + 1);
+            // scale and min of sub-blocks 2j, 2j + 1: each lane half decodes its
+            // row tiles' and the halves exchange them (pf_mma)
+            float dsf[EXACTW ? RU : 1][2], dmf[EXACTW ? RU : 1][2];
+            half2v ds[RU], dm[RU];
+#pragma unroll
+            for (int v = 0; v < RU / 2; ++v) {
+                const float d = h2f(hd[v].x & 0xffffu), dmin = h2f(hd[v].x >> 16);
+                float scA, mA, scB, mB;
+                k_scale_min_pair(hd[v].y, hd[v].z, hd[v].w, j, scA, mA, scB, mB);
+                auto both = [](float a) {
+                    return __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+                };
+                if constexpr (EXACTW) {
+                    const auto xa = both(d * scA), xb = both(d * scB), ya = both(-(dmin * mA)), yb = both(-(dmin * mB));
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        dsf[2 * v + k][0] = __uint_as_float((uint32_t)xa[k]);
+                        dsf[2 * v + k][1] = __uint_as_float((uint32_t)xb[k]);
+                        dmf[2 * v + k][0] = __uint_as_float((uint32_t)ya[k]);
+                        dmf[2 * v + k][1] = __uint_as_float((uint32_t)yb[k]);
+                    }
+                } else {
+                    const half2v s2 = {(_Float16)(d * scA), (_Float16)(d * scB)};
+                    const half2v m2 = {(_Float16)(-(dmin * mA)), (_Float16)(-(dmin * mB))};
+                    const auto xa = both(__builtin_bit_cast(float, s2)), ya = both(__builtin_bit_cast(float, m2));
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        ds[2 * v + k] = __builtin_bit_cast(half2v, (uint32_t)xa[k]);
+                        dm[2 * v + k] = __builtin_bit_cast(half2v, (uint32_t)ya[k]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int u = 0; u < RU; ++u) {
+                    half8 wq;
+                    if constexpr (EXACTW)
+                        wq = pf_dequant8_exact(q[u][s & 1], s >= 2, dsf[u][s >> 1], dmf[u][s >> 1]);
+                    else {
+                        const _Float16 a = ds[u][s >> 1], b = dm[u][s >> 1];
+                        wq = pf_dequant8(q[u][s & 1], s >= 2, half2v{a, a}, half2v{b, b});
+                    }
+                    acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq, x[s], acc[u], 0, 0, 0);
+                }
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70); // the last (unused) copies have landed
+    }
+    __syncthreads();
+
+    // lane (li, h), register 4 q + r of acc[u]: token li, row 32 u + 8 q + 4 h + r
+    float *const P = reinterpret_cast<float *>(lds);
+    auto place = [&](int w, int u, int q) {
+        return reinterpret_cast<float4 *>(P + (PFT_BM * w + li) * LD + 32 * u + 8 * q + 4 * h);
+    };
+    auto put = [&](int w) {
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *place(w, u, q) = make_float4(acc[u][4 * q], acc[u][4 * q + 1], acc[u][4 * q + 2], acc[u][4 * q + 3]);
+    };
+    if (wave >= 4)
+        put(wave - 4);
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 p = *place(wave, u, q);
+                acc[u][4 * q] += p.x;
+                acc[u][4 * q + 1] += p.y;
+                acc[u][4 * q + 2] += p.z;
+                acc[u][4 * q + 3] += p.w;
+            }
+        put(wave);
+    }
+    __syncthreads();
+    // 16 threads a token, four rows each
+    const int ml = tid >> 4, nl = 4 * (tid & 15), m = m0 + ml, n = n0 + nl;
+    if (m >= T || n >= N)
+        return;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float4 p = *reinterpret_cast<const float4 *>(P + (PFT_BM * w + ml) * LD + nl);
+        v.x += p.x;
+        v.y += p.y;
+        v.z += p.z;
+        v.w += p.w;
+    }
+    const int sm = -xs[m]; // undo the row's power-of-two scale (exact)
+    v = make_float4(__builtin_ldexpf(v.x, sm), __builtin_ldexpf(v.y, sm), __builtin_ldexpf(v.z, sm),
+                    __builtin_ldexpf(v.w, sm));
+    float *y = Y + (size_t)m * N + n;
+    if ((N & 3) == 0) {
+        *reinterpret_cast<float4 *>(y) = v;
+    } else {
+        y[0] = v.x;
+        if (n + 1 < N) y[1] = v.y;
+        if (n + 2 < N) y[2] = v.z;
+        if (n + 3 < N) y[3] = v.w;
+    }
+}
+
 // Y += P[0] + P[1] + ... + P[nparts - 1] (n floats each), in that order, so
 // the result does not depend on which split finished first.
 template <bool VEC>
@@ -1280,6 +1489,17 @@ hipError_t launch_prefill_gemm(const void *w, void *xh, float *Y, int T, int inn
         return hipErrorInvalidValue;
     int *xs = reinterpret_cast<int *>(static_cast<uint8_t *>(xh) + prefill_scale_offset(T, inner));
     float *P = reinterpret_cast<float *>(static_cast<uint8_t *>(xh) + prefill_part_offset(T, inner));
+    if (prefill_thin(T, inner, outer, device_cus())) {
+        const int mt = (T + PFT_BM - 1) / PFT_BM, nt = (outer + PFT_BN - 1) / PFT_BN;
+        const dim3 grid(prefill_grid(mt * nt, 1)), block(512);
+        if (inner <= kPrefillExactWMaxK)
+            hipLaunchKernelGGL(k_prefill_q4k_thin<true>, grid, block, 0, s, (const uint8_t *)w, (const _Float16 *)xh,
+                               (const int *)xs, Y, T, inner, outer, mt, nt);
+        else
+            hipLaunchKernelGGL(k_prefill_q4k_thin<false>, grid, block, 0, s, (const uint8_t *)w, (const _Float16 *)xh,
+                               (const int *)xs, Y, T, inner, outer, mt, nt);
+        return hipGetLastError();
+    }
     const int ru = prefill_wide_rows(T, inner, outer, device_cus());
     if (ru) {
         if (ru == 2)

@@ -7,3 +7,8 @@ extern "C" int prefill_wide_rows_of(int T, int inner, int outer, int ncu)
 {
     return ihip::prefill_wide_rows(T, inner, outer, ncu);
 }
+
+extern "C" int prefill_thin_of(int T, int inner, int outer, int ncu)
+{
+    return ihip::prefill_thin(T, inner, outer, ncu);
+}

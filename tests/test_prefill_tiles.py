@@ -1,7 +1,8 @@
 """Tile choice of the prefill GEMM: the wide kernel's 128-token tiles for products
-with enough of them to fill the chip, 64 tokens x 128 rows otherwise
-(prefill_wide_rows, inferno.jl_amd/csrc/kq_launch.h), and the wide kernel
-against a float64 product at the edges of its tiles.
+with enough of them to fill the chip (prefill_wide_rows,
+inferno.jl_amd/csrc/kq_launch.h), 32-token x 64-row tiles whose waves share K
+for small ones (prefill_thin), 64 tokens x 128 rows otherwise, and both kernels
+against a float64 product at the edges of their tiles.
 """
 import ctypes as C
 from pathlib import Path
@@ -23,6 +24,22 @@ def wide_rows():
     f = C.CDLL(str(LIB)).prefill_wide_rows_of
     f.argtypes, f.restype = [C.c_int] * 4, C.c_int
     return lambda T, outer, inner, ncu=256: f(T, inner, outer, ncu)
+
+
+@pytest.fixture(scope="module")
+def thin(wide_rows):
+    f = C.CDLL(str(LIB)).prefill_thin_of
+    f.argtypes, f.restype = [C.c_int] * 4, C.c_int
+    return lambda T, outer, inner, ncu=256: bool(f(T, inner, outer, ncu))
+
+
+def test_thin_choice(thin):
+    assert thin(8, 9728, 2560) and thin(77, 9728, 2560) and thin(128, 4096, 4096) and thin(512, 2048, 1024)
+    assert not thin(512, 4096, 4096)       # one 64 x 128 tile per CU
+    assert not thin(2048, 12288, 4096)
+    assert not thin(64, 4096, 12288)       # long rows: split over workgroups
+    assert not thin(1, 1 << 24, 1024)
+    assert isinstance(thin(8, 512, 1024, 1), bool)
 
 
 def test_tile_choice(wide_rows):
@@ -47,10 +64,26 @@ WIDE = ((641, 8193, 768, 1), (1151, 4099, 1024, 1), (1000, 4096, 2048, 1), (193,
 def test_wide_tiles_match_float64(wide_rows, T, outer, inner, ru):
     """Within 1e-4 * ||w_row|| * ||x|| of the float64 product, as every prefill
     launch on seeded random data."""
+    assert wide_rows(T, outer, inner) == ru
+    _match_float64("wide", T, outer, inner)
+
+
+# one token and one row, tiles one short and one over, rows off 4; 3 to 16
+# block columns (uneven shares of the wave halves), both weight roundings
+THIN = ((1, 1, 768), (31, 63, 1024), (33, 65, 1280), (65, 4097, 2048), (32, 4096, 2304), (95, 4098, 2816), (300, 1030, 4096))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,outer,inner", THIN)
+def test_thin_tiles_match_float64(thin, T, outer, inner):
+    assert thin(T, outer, inner)
+    _match_float64("thin", T, outer, inner)
+
+
+def _match_float64(what, T, outer, inner):
     import torch
     from inferno_hip import device as D
-    assert wide_rows(T, outer, inner) == ru
-    print(f"wide prefill T={T} {outer}x{inner}", flush=True)
+    print(f"{what} prefill T={T} {outer}x{inner}", flush=True)
     rng = synth.rng_for(0x71DE + T)
     w = synth.weight(rng, synth.Q4_K, outer, inner)
     X = (rng.standard_normal((T, inner)) * np.exp2(rng.integers(-20, 21, T))[:, None]).astype(np.float32)
@@ -61,5 +94,5 @@ def test_wide_tiles_match_float64(wide_rows, T, outer, inner, ru):
     ref = xf @ wf.t().contiguous()
     tol = 1e-4 * xf.norm(dim=1)[:, None] * wf.norm(dim=1)[None, :]
     ratio = ((Y.double() - ref).abs() / tol).max().item()
-    print(f"wide prefill max err/tol = {ratio:.3e}", flush=True)
+    print(f"{what} prefill max err/tol = {ratio:.3e}", flush=True)
     assert ratio <= 1.0
