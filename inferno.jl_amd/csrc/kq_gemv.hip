@@ -20,13 +20,13 @@
 //     k_gemv_kpers): blocks are 16-byte multiples, so lanes load straight from
 //     HBM with 128-bit loads.  A wave covers 16 blocks (4096 columns) of R rows
 //     per pass: lane = (block, sub-block pair), 64 weights per lane per row.
-//   * Other Q4_K / Q5_K rows and Q6_K (k_gemv_mdig): four rows x four blocks a
-//     step, the integer products on the matrix cores.
-//   * Q6_K (210 B), Q8_0 (34 B) and IQ4_NL (18 B) blocks are not 16-byte
-//     aligned, but 8 of them are.  k_gemv_sdig streams each wave's rows
-//     through a private LDS ring filled by gfx950's direct-to-LDS 128-bit
-//     copies (no registers, no workgroup barrier), then re-slices blocks
-//     from LDS.
+//   * All other rows of at most 16384 columns (k_gemv_mdig): four rows x 1024
+//     columns a step through a private LDS ring per wave, filled by gfx950's
+//     direct-to-LDS 128-bit copies, the integer products on the matrix cores.
+//   * The lm_head with its argmax, and longer rows of Q6_K (210 B), Q8_0 (34 B)
+//     and IQ4_NL (18 B), whose blocks are not 16-byte aligned (8 of them are):
+//     k_gemv_sdig streams each wave's rows through a ring of the same kind
+//     and re-slices blocks from LDS.
 //   * Greedy argmax (lm_head) is fused into the streamed kernel's epilogue:
 //     each workgroup writes one (value, index) partial to its own slot and a
 //     one-workgroup kernel reduces the partials, so no two workgroups touch
@@ -35,6 +35,7 @@
 #include "inferno_hip.h"
 
 #include <algorithm>
+#include <type_traits>
 #include "kq_common.h"
 #include "kq_launch.h"
 #include "kq_sdig_plan.h"
@@ -530,26 +531,40 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kwide(const uint8_t *__restri
 // holds digit plane i (0..2; 3 unused) of the lane's elements 16 t .. 16 t + 15,
 // so that a wave reads 1 KB in lane order; the 65th word spreads the staging
 // writes over the banks.  Then 16 bytes for each b: Q4_K / Q5_K {sum A, sum B,
-// exponent A, exponent B} of the pair, Q6_K 2^(e - 22) of its four groups.
+// exponent A, exponent B} of the pair, Q6_K 2^(e - 22) of its four groups, Q8_0
+// and IQ4_NL 2^(e - 22) of its two blocks.
 constexpr int kMdPlaneDw = 65 * 4, kMdStepDw = 4 * kMdPlaneDw;
 constexpr int kMdUnits = 512; // units (four rows x one step) per workgroup
-// Bytes of a block; 16-byte pieces of a row's step (Q6_K: from the 16-byte
-// unit its first byte lies in, at an even phase of 0 .. 14); pieces between two
-// rows in a ring slot (one more: 13 of 16 lanes' 128-bit reads then hit
+// Bytes of a block and blocks of a step; 16-byte pieces of a row's step (PHASED:
+// from the 16-byte unit its first byte lies in, at an even phase of 0 .. 14);
+// pieces between two rows in a ring slot (one more: 13 of 16 lanes' 128-bit reads then hit
 // distinct banks, 8 without); 1 KB copies of a slot.
 template <int FMT>
 struct MdFmt;
 template <>
 struct MdFmt<kQ4_K> {
-    static constexpr int BYTES = 144, PIECES = 36, PITCH = 37, COPIES = 3;
+    static constexpr int BYTES = 144, BLOCKS = 4, PIECES = 36, PITCH = 37, COPIES = 3;
+    static constexpr bool PHASED = false;
 };
 template <>
 struct MdFmt<kQ5_K> {
-    static constexpr int BYTES = 176, PIECES = 44, PITCH = 45, COPIES = 3;
+    static constexpr int BYTES = 176, BLOCKS = 4, PIECES = 44, PITCH = 45, COPIES = 3;
+    static constexpr bool PHASED = false;
 };
 template <>
 struct MdFmt<kQ6_K> {
-    static constexpr int BYTES = 210, PIECES = 54, PITCH = 55, COPIES = 4;
+    static constexpr int BYTES = 210, BLOCKS = 4, PIECES = 54, PITCH = 55, COPIES = 4;
+    static constexpr bool PHASED = true;
+};
+template <>
+struct MdFmt<kQ8_0> {
+    static constexpr int BYTES = 34, BLOCKS = 32, PIECES = 69, PITCH = 70, COPIES = 5;
+    static constexpr bool PHASED = true;
+};
+template <>
+struct MdFmt<kIQ4_NL> {
+    static constexpr int BYTES = 18, BLOCKS = 32, PIECES = 37, PITCH = 38, COPIES = 3;
+    static constexpr bool PHASED = true;
 };
 
 // Digits of one float4 of x (number f of the row); 8 consecutive threads hold
@@ -582,6 +597,9 @@ __device__ __forceinline__ void md_stage4(float4 v, int f, uint32_t *dig, float4
     if constexpr (FMT == kQ6_K) {
         if ((f & 3) == 0)
             reinterpret_cast<float *>(pinfo + (f >> 8) * 16 + b)[t4] = finite ? __builtin_ldexpf(1.0f, e - 22) : __builtin_nanf("");
+    } else if constexpr (FMT == kQ8_0 || FMT == kIQ4_NL) {
+        if ((f & 7) == 0)
+            reinterpret_cast<float *>(pinfo + (f >> 4))[(f >> 3) & 1] = finite ? __builtin_ldexpf(1.0f, e - 22) : __builtin_nanf("");
     } else {
         // the sum of the rounded values, so that a weight's two terms see the
         // same x: the rounding of x then meets d sc q - dmin m, not d sc q alone
@@ -683,6 +701,47 @@ __device__ __forceinline__ float mdig_dot_q6(const uint8_t *blk, uint32_t sh, in
     return d * (t01 + t23);
 }
 
+// The same for two blocks of 32 (Q8_0, IQ4_NL) from byte `byte` (even) of the
+// row in LDS, block A then B: an fp16 scale and 32 signed bytes, or 16 bytes of
+// grid indices whose low nibbles are elements 0..15 and high ones 16..31.  b_in:
+// block B is part of the row.
+template <int FMT>
+__device__ __forceinline__ float mdig_dot_b32(const uint8_t *row, uint32_t byte, const uint4 (&X)[4], float4 info,
+                                              bool b_in)
+{
+    typedef int int4v __attribute__((ext_vector_type(4)));
+    constexpr int NQ = FMT == kQ8_0 ? 8 : 4; // dwords of quants in a block
+    const uint32_t xd[16] = {X[0].x, X[0].y, X[0].z, X[0].w, X[1].x, X[1].y, X[1].z, X[1].w,
+                             X[2].x, X[2].y, X[2].z, X[2].w, X[3].x, X[3].y, X[3].z, X[3].w};
+    float t[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t at = byte + (uint32_t)(k * MdFmt<FMT>::BYTES);
+        const float d = h2f(*reinterpret_cast<const uint16_t *>(row + at));
+        const uint32_t *p = reinterpret_cast<const uint32_t *>(row + ((at + 2u) & ~3u));
+        uint32_t w[NQ + 1];
+#pragma unroll
+        for (int i = 0; i <= NQ; ++i) w[i] = p[i];
+        int4v a = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const uint32_t q = __builtin_amdgcn_alignbyte(w[i + 1], w[i], (at + 2u) & 3u);
+            if constexpr (FMT == kQ8_0) {
+                a = __builtin_amdgcn_mfma_i32_4x4x4i8((int)xd[8 * k + i], (int)q, a, 0, 0, 0);
+            } else {
+                uint32_t lo, hi; // grid + 128
+                iq4nl_lookup2(q, lo, hi);
+                a = __builtin_amdgcn_mfma_i32_4x4x4i8((int)xd[8 * k + i], (int)(lo ^ 0x80808080u), a, 0, 0, 0);
+                a = __builtin_amdgcn_mfma_i32_4x4x4i8((int)xd[8 * k + 4 + i], (int)(hi ^ 0x80808080u), a, 0, 0, 0);
+            }
+        }
+        // 8-bit weights: 256 S2 can pass 2^24, so the planes fold in fp32
+        const float v = fmaf(fmaf((float)a[2], 256.0f, (float)a[1]), 256.0f, (float)a[0]);
+        t[k] = d * v * (k ? info.y : info.x);
+    }
+    return t[0] + (b_in ? t[1] : 0.0f);
+}
+
 // Plain GEMV, with the residual epilogue (RESID) or the folded input norm
 // (NORM), or fused gate/up + SwiGLU (GATEUP), as the wide kernels.
 //
@@ -715,9 +774,10 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = lane >> 2, r = lane & 3, bq = b >> 2, j = b & 3;
-    const int inner = nblk * 256;
+    constexpr int BPS = F::BLOCKS;
+    const int inner = nblk * (1024 / BPS);
     const uint32_t row_bytes = (uint32_t)nblk * F::BYTES;
-    const int nstep = (nblk + 3) >> 2;
+    const int nstep = (nblk + BPS - 1) / BPS;
     const int ngroups = (outer + 3) >> 2;
     const int G0 = (int)blockIdx.x * gpw, ng = min(gpw, ngroups - G0);
     const int units = ng * NM * nstep;
@@ -744,9 +804,11 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
 #pragma unroll
         for (int k = 0; k < XC; ++k)
             if (k0 + k < nx) {
-                lds_copy16_at(x + 4 * NT * (k0 + k), 16u * (uint32_t)tid, mine_lds + raw + 1024 * k);
+                // threads past the row (rows of no whole 256 columns) copy its end
+                const uint32_t o = (uint32_t)min(16 * tid, 4 * inner - 16 - 16 * NT * (k0 + k));
+                lds_copy16_at(x + 4 * NT * (k0 + k), o, mine_lds + raw + 1024 * k);
                 if constexpr (NORM)
-                    lds_copy16_at(nw + 4 * NT * (k0 + k), 16u * (uint32_t)tid, mine_lds + raw + 1024 * (xc + k));
+                    lds_copy16_at(nw + 4 * NT * (k0 + k), o, mine_lds + raw + 1024 * (xc + k));
             }
     };
     issue_x(0);
@@ -776,16 +838,16 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
     int islot = 0;
     auto issue = [&]() {
         const int row0 = 4 * (G0 + (GATEUP ? lc.vg >> 1 : lc.vg));
-        const uint8_t *base = (GATEUP && (lc.vg & 1) ? W2 : W) + (size_t)row0 * row_bytes + (size_t)lc.s * (4 * F::BYTES);
+        const uint8_t *base = (GATEUP && (lc.vg & 1) ? W2 : W) + (size_t)row0 * row_bytes + (size_t)lc.s * (BPS * F::BYTES);
         // rows past the last, and blocks past the row: the last one again
         const uint32_t rmax = (uint32_t)(min(outer - row0, 4) - 1) * row_bytes;
-        const uint32_t nbytes = (uint32_t)min(nblk - 4 * lc.s, 4) * F::BYTES;
-        const uint32_t phase = FMT == kQ6_K ? (uint32_t)(uintptr_t)base & 15u : 0u;
+        const uint32_t nbytes = (uint32_t)min(nblk - BPS * lc.s, BPS) * F::BYTES;
+        const uint32_t phase = F::PHASED ? (uint32_t)(uintptr_t)base & 15u : 0u;
         base -= phase;
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
             uint32_t o = min(ro[i], rmax);
-            if constexpr (FMT == kQ6_K) { // from the 16-byte unit of the row's first byte
+            if constexpr (F::PHASED) { // from the 16-byte unit of the row's first byte
                 o += phase;
                 o = (o & ~15u) + min(po[i], ((o & 15u) + nbytes - 1u) & ~15u);
             } else {
@@ -825,6 +887,8 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
         for (int k = 0; k < XC; ++k)
             if (k0 + k < nx) {
                 float4 v = *reinterpret_cast<const float4 *>(mine + raw + 1024 * k + 16 * lane);
+                if (BPS == 32 && 4 * (tid + NT * (k0 + k)) >= inner)
+                    v = make_float4(0.f, 0.f, 0.f, 0.f);
                 if constexpr (NORM) {
                     const float4 w = *reinterpret_cast<const float4 *>(mine + raw + 1024 * (xc + k) + 16 * lane);
                     ssq = fmaf(v.x, v.x, ssq);
@@ -858,13 +922,18 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
             X[t] = *reinterpret_cast<const uint4 *>(dig + uc.s * kMdStepDw + t * kMdPlaneDw + 4 * lane);
         const float4 info = pinfo[16 * uc.s + b];
         float c;
-        if constexpr (FMT == kQ6_K) {
+        const bool active = BPS * uc.s + (BPS == 32 ? 2 * b : bq) < nblk;
+        if constexpr (F::PHASED) {
             const int vg = GATEUP ? uc.vg >> 1 : uc.vg, row0 = 4 * (G0 + vg);
             const uint32_t at = (uint32_t)(uintptr_t)(GATEUP && (uc.vg & 1) ? W2 : W) +
-                                (uint32_t)(row0 + min(r, outer - 1 - row0)) * row_bytes + (uint32_t)uc.s * (4 * F::BYTES);
+                                (uint32_t)(row0 + min(r, outer - 1 - row0)) * row_bytes + (uint32_t)uc.s * (BPS * F::BYTES);
             // blocks past the row's end read stale bytes of the slot, unused
-            const uint32_t byte = (at & 15u) + (uint32_t)bq * F::BYTES;
-            c = mdig_dot_q6(row + (byte & ~3u), byte & 2u, j >> 1, j & 1, X, info);
+            if constexpr (FMT == kQ6_K) {
+                const uint32_t byte = (at & 15u) + (uint32_t)bq * F::BYTES;
+                c = mdig_dot_q6(row + (byte & ~3u), byte & 2u, j >> 1, j & 1, X, info);
+            } else {
+                c = mdig_dot_b32<FMT>(row, (at & 15u) + (uint32_t)(2 * b) * F::BYTES, X, info, BPS * uc.s + 2 * b + 1 < nblk);
+            }
             __builtin_amdgcn_s_waitcnt(0xc07f);
             asm volatile("" ::: "memory");
             if (i + D < n)
@@ -879,7 +948,7 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
             c = mdig_dot<FMT>(B, j, X, info);
         }
         // over the lanes of row r: 16 lanes' four, then the four rows of lanes
-        float v = 4 * uc.s + bq < nblk ? c : 0.0f;
+        float v = active ? c : 0.0f;
         v = dpp_add<0x128, 0xf>(v); // row_ror:8
         v = dpp_add<0x124, 0xf>(v); // row_ror:4
         const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -1774,13 +1843,6 @@ int device_cus()
     return ncu;
 }
 
-// IQ4_NL rows of 17..64 256-column units whose two-row, 8-wave workgroups
-// would not divide evenly over the CUs.
-static bool kwide_uneven(int nblk, int outer)
-{
-    return nblk > 16 && nblk <= 4 * 16 && ((outer + 15) / 16) % device_cus() != 0;
-}
-
 // Rows of at most 16 blocks with at least four 8-wave row groups per wave
 // over one workgroup per CU take the persistent kernel.
 static bool kwide_takes_kpers(int nblk, int outer) { return nblk <= 16 && outer >= 4 * 8 * 256; }
@@ -1788,19 +1850,19 @@ static bool kwide_takes_kpers(int nblk, int outer) { return nblk <= 16 && outer 
 // No more one-row workgroups of 8 waves than CUs: one row per wave.
 static bool kwide_one_row(int outer) { return (outer + 7) / 8 <= device_cus(); }
 
-// Rows of at most 64 blocks on the matrix cores: waves and ring depth by the
-// row's steps (Q6_K: its 4 KB slots leave 8 waves beside the digits of more
-// than 12 steps).
+// Rows of at most 16 steps of 1024 columns on the matrix cores: waves and ring
+// depth by the row's steps and the format's slot (3 to 5 KB a wave and slot,
+// beside 4 KB of digits a step).
 struct MdPlan {
     int nw, d, maxs;
 };
-constexpr MdPlan mdig_plan(int type, int nblk)
+constexpr MdPlan mdig_plan(int type, int nstep)
 {
-    if (nblk <= 16)
+    if (nstep <= 4)
         return {8, 3, 4};
-    if (type == kQ6_K)
-        return nblk <= 48 ? MdPlan{12, 2, 12} : MdPlan{8, 2, 16};
-    return {12, 2, 16};
+    if (type == kQ6_K && nstep <= 12)
+        return {12, 2, 12};
+    return type == kQ6_K || type == kQ8_0 ? MdPlan{8, 2, 16} : MdPlan{12, 2, 16};
 }
 // Which rows take it, by format, length and (gate/up) kind only: a row's sum is
 // the same whatever launch it is in, and the two kernels' differ.  The wide
@@ -1815,8 +1877,9 @@ constexpr MdPlan mdig_plan(int type, int nblk)
 // 12288 x 4096 12.8 / 13.0; Q5_K 9728 x 2560 12.3 / 9.7, 12288 x 4096 15.8 / 15.5;
 // the folded norm Q4_K 6144 x 4096 6.6 / 6.0.  Q6_K (streamed / this) 4096 x
 // 12288 12.4 / 11.7, 2560 x 9728 12.1 / 7.9, 5120 x 13824 26.9 / 15.9, 1024 x 4096
-// 4.9 / 3.6, 12288 x 4096 11.2 / 11.5.
-constexpr int kMdMaxBlocks = 64;
+// 4.9 / 3.6, 12288 x 4096 11.2 / 11.5; Q8_0 5003 x 2720 8.4 / 5.8, 2560 x 9728 11.2 /
+// 8.3; IQ4_NL 5120 x 5120 10.7 / 6.8, 5003 x 2720 8.8 / 5.1, 20000 x 6144 24.3 / 17.7.
+constexpr int kMdMaxSteps = 16, kMdMaxBlocks = 4 * kMdMaxSteps;
 constexpr bool mdig_takes(int type, int nblk, bool gateup)
 {
     if (nblk > kMdMaxBlocks)
@@ -1831,24 +1894,35 @@ template <int FMT, bool GATEUP, bool NORM, bool RESID>
 static void launch_mdig(const uint8_t *W, const uint8_t *W2, const float *x, float *y, int nblk, int outer,
                         const float *nw, float eps, const float *resid, int epi, hipStream_t s)
 {
-    const int nstep = (nblk + 3) / 4, ngroups = (outer + 3) / 4;
+    constexpr int BPS = MdFmt<FMT>::BLOCKS;
+    const int nstep = (nblk + BPS - 1) / BPS, ngroups = (outer + 3) / 4;
     const int gpw = std::min((ngroups + device_cus() - 1) / device_cus(), kMdUnits / (nstep * (GATEUP ? 2 : 1)));
     const dim3 grid((ngroups + gpw - 1) / gpw);
     const uint32_t inv = (65536u + nstep - 1) / nstep;
-    const MdPlan p = mdig_plan(FMT, nblk);
+    constexpr MdPlan p16 = mdig_plan(FMT, 16), p12 = mdig_plan(FMT, 12);
+    auto launch = [&](auto nwv, auto d, auto maxs) {
+        hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, nwv.value, d.value, maxs.value>), grid,
+                           dim3(nwv.value * 64), 0, s, W, W2, x, y, outer, nblk, gpw, inv, nw, eps, resid, epi);
+    };
+    using std::integral_constant;
+    const MdPlan p = mdig_plan(FMT, nstep);
     if (p.maxs == 4)
-        hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 8, 3, 4>), grid, dim3(8 * 64), 0, s, W, W2, x, y,
-                           outer, nblk, gpw, inv, nw, eps, resid, epi);
-    else if constexpr (FMT == kQ6_K) {
-        if (p.maxs == 12)
-            hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 12, 2, 12>), grid, dim3(12 * 64), 0, s, W, W2, x,
-                               y, outer, nblk, gpw, inv, nw, eps, resid, epi);
-        else
-            hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 8, 2, 16>), grid, dim3(8 * 64), 0, s, W, W2, x, y,
-                               outer, nblk, gpw, inv, nw, eps, resid, epi);
-    } else
-        hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, 12, 2, 16>), grid, dim3(12 * 64), 0, s, W, W2, x, y,
-                           outer, nblk, gpw, inv, nw, eps, resid, epi);
+        launch(integral_constant<int, 8>{}, integral_constant<int, 3>{}, integral_constant<int, 4>{});
+    else if (p.maxs == p12.maxs)
+        launch(integral_constant<int, p12.nw>{}, integral_constant<int, p12.d>{}, integral_constant<int, p12.maxs>{});
+    else
+        launch(integral_constant<int, p16.nw>{}, integral_constant<int, p16.d>{}, integral_constant<int, p16.maxs>{});
+}
+
+template <int FMT>
+static hipError_t launch_mdig_b32(const void *w, const float *x, float *y, int inner, int outer, const float *resid,
+                                  int epi, hipStream_t s)
+{
+    if (resid)
+        launch_mdig<FMT, false, false, true>((const uint8_t *)w, nullptr, x, y, inner / 32, outer, nullptr, 0.0f, resid, epi, s);
+    else
+        launch_mdig<FMT, false, false, false>((const uint8_t *)w, nullptr, x, y, inner / 32, outer, nullptr, 0.0f, nullptr, epi, s);
+    return hipGetLastError();
 }
 
 // Rows that k_gemv_mdig does not take: 8-wave workgroups; two rows per wave
@@ -1963,7 +2037,12 @@ static hipError_t launch_sdig(const void *w, const float *x, float *y, int inner
     if (p.d != 2 && !(p.d == 3 && p.nw == 8))
         return hipErrorInvalidValue; // no such instantiation
     switch (p.nw) {
-    case 8: launch_sdig_nw<FMT, ARGMAX, 8>(w, x, y, nblk, outer, p, parts, s, resid, epi); break;
+    case 8:
+        if constexpr (ARGMAX) // short rows without the argmax run in k_gemv_mdig
+            launch_sdig_nw<FMT, ARGMAX, 8>(w, x, y, nblk, outer, p, parts, s, resid, epi);
+        else
+            return hipErrorInvalidValue;
+        break;
     case 12: launch_sdig_nw<FMT, ARGMAX, 12>(w, x, y, nblk, outer, p, parts, s, resid, epi); break;
     case 16: launch_sdig_nw<FMT, ARGMAX, 16>(w, x, y, nblk, outer, p, parts, s, resid, epi); break;
     default: return hipErrorInvalidValue;
@@ -1987,22 +2066,22 @@ hipError_t launch_gemv(int type, const void *w, const float *x, float *y, int in
         }
         return launch_sdig<kQ6_K, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     case kQ8_0:
-        // rows of one pass (at most 4096 columns in whole 256-column units)
-        // on the wide lane layout, measured against the streamed kernel in one
-        // process: 151936 x 2048 60-62 us against 67.5, 5120 x 3072 6.6 against
-        // 8.2, 8192 x 4096 8.9 against 9.4, 4096 x 2048 4.6 against 4.8,
-        // 4096 x 4096 6.1-6.2 against 6.1-6.3; rows of several passes stay on
-        // the streamed kernel (4096 x 14336 16.2 against 17.7)
-        return inner % 256 == 0 && inner <= 4096
-                   ? launch_kwide<kQ8_0, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi)
-                   : launch_sdig<kQ8_0, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
+        // rows of one pass (at most 4096 columns in whole 256-column units) on
+        // the wide lane layout: 4096 x 4096 5.9 us against k_gemv_mdig's 6.1,
+        // 2048 x 2048 3.0 / 3.3, 9728 x 2560 8.0 / 7.6
+        if (inner % 256 == 0 && inner <= 4096)
+            return launch_kwide<kQ8_0, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi);
+        if (inner <= 1024 * kMdMaxSteps)
+            return launch_mdig_b32<kQ8_0>(w, x, y, inner, outer, resid, epi, s);
+        return launch_sdig<kQ8_0, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     case kIQ4_NL:
-        // rows of whole 256-column units take the wide kernels' lane layout,
-        // except several passes on an uneven grid (5120 x 5120: the streamed
-        // kernel 10.3 us)
-        return inner % 256 == 0 && !kwide_uneven(inner / 256, outer)
-                   ? launch_kwide<kIQ4_NL, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi)
-                   : launch_sdig<kIQ4_NL, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
+        // the wide lane layout where it is all but full (4096 x 4096 5.0 us
+        // against k_gemv_mdig's 5.4), and for rows too long for the others
+        if (inner % 256 == 0 && ((inner > 3584 && inner <= 4096) || inner > 1024 * kMdMaxSteps))
+            return launch_kwide<kIQ4_NL, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi);
+        if (inner <= 1024 * kMdMaxSteps)
+            return launch_mdig_b32<kIQ4_NL>(w, x, y, inner, outer, resid, epi, s);
+        return launch_sdig<kIQ4_NL, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     default: return hipErrorInvalidValue;
     }
 }

@@ -12,7 +12,7 @@ from inferno_hip import synth
 
 pytestmark = pytest.mark.gpu
 
-TYPES = (synth.Q4_K, synth.Q5_K, synth.Q6_K)
+TYPES = (synth.Q4_K, synth.Q5_K, synth.Q6_K, synth.Q8_0, synth.IQ4_NL)
 
 
 def _gemv(t, w, x, outer, inner, resid=None):
