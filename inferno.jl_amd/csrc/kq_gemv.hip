@@ -80,12 +80,12 @@ __device__ __forceinline__ void x_load_pass(const float *__restrict__ x, int col
 // (v_dot4_{u32_u8,i32_i8}: four byte products and the accumulate in one
 // instruction) when x is written as an integer.  Each 32-element sub-block of
 // x is scaled by 2^(22-e), e the binary exponent of the sub-block's largest
-// |x| (|x| < 2^e), and truncated to an integer X with |X| < 2^22: the error of
-// x ~ X * 2^(e-22) is below 2^(e-22) <= |x|max * 2^-21.  The sub-block's
+// |x| (|x| < 2^e), and rounded to an integer X with |X| <= 2^22: the error of
+// x ~ X * 2^(e-22) is at most 2^(e-23) <= |x|max * 2^-22.  The sub-block's
 // |x|max is at most its own 2-norm, so the error vector of 32 values has a
-// norm below sqrt(32) * 2^-21 times theirs, and over any number of sub-blocks
-// ||x - X 2^(e-22)||_2 < sqrt(32) * 2^-21 * ||x||_2: a dot product is off by
-// less than 2.7e-6 * ||w||_2 ||x||_2 whatever its length and data (the row
+// norm below sqrt(32) * 2^-22 times theirs, and over any number of sub-blocks
+// ||x - X 2^(e-22)||_2 < sqrt(32) * 2^-22 * ||x||_2: a dot product is off by
+// less than 1.4e-6 * ||w||_2 ||x||_2 whatever its length and data (the row
 // bound is 1e-4; about 1e-7 for random data).  X is split into three byte digits,
 // X = 65536 * b2 + 256 * b1 + b0 (b0, b1 unsigned, b2 signed); the products
 // q * b are exact integers, so the per-sub-block sums are exact and
@@ -117,16 +117,16 @@ __device__ __forceinline__ void dig_pack(int X0, int X1, int X2, int X3, uint32_
     d2 = __builtin_amdgcn_perm(q23, q01, 0x05040100u);
 }
 
-// Digits of four elements that share exponent e (finite == false: zeros).
-__device__ __forceinline__ void dig_four(float4 v, int e, bool finite, uint32_t &d0, uint32_t &d1,
-                                         uint32_t &d2)
+// Digits of four elements that share exponent e (finite == false: zeros), and
+// the sum of the four integers.
+__device__ __forceinline__ int dig_four(float4 v, int e, bool finite, uint32_t &d0, uint32_t &d1,
+                                        uint32_t &d2)
 {
     const int sh = 22 - e;
-    const int X0 = finite ? (int)__builtin_ldexpf(v.x, sh) : 0;
-    const int X1 = finite ? (int)__builtin_ldexpf(v.y, sh) : 0;
-    const int X2 = finite ? (int)__builtin_ldexpf(v.z, sh) : 0;
-    const int X3 = finite ? (int)__builtin_ldexpf(v.w, sh) : 0;
+    auto fixed = [&](float a) { return finite ? (int)__builtin_rintf(__builtin_ldexpf(a, sh)) : 0; };
+    const int X0 = fixed(v.x), X1 = fixed(v.y), X2 = fixed(v.z), X3 = fixed(v.w);
     dig_pack(X0, X1, X2, X3, d0, d1, d2);
+    return (X0 + X1) + (X2 + X3);
 }
 
 // |x| bits of four elements, maxed: NaN > +Inf > every finite value.
@@ -152,25 +152,26 @@ __device__ __forceinline__ void x_stage_dig(uint32_t *pl, float *xsum, int *xexp
         if (tid + NT * k >= 1024)
             continue; // past the pass; wave-uniform (NT and 1024 are multiples of 64)
         const float4 v = xv[k];
-        float t = (v.x + v.y) + (v.z + v.w);
         uint32_t m = abs_bits_max(v);
-        t = dpp_add<0xb1, 0xf>(t);
         m = dpp_max_u32<0xb1, 0xf>(m);
-        t = dpp_add<0x4e, 0xf>(t);
         m = dpp_max_u32<0x4e, 0xf>(m);
-        t = dpp_add<0x141, 0xf>(t);
         m = dpp_max_u32<0x141, 0xf>(m);
         const bool finite = m < 0x7f800000u;
         const int e = finite ? __builtin_amdgcn_frexp_expf(__uint_as_float(m)) : 0;
         uint32_t d0, d1, d2;
-        dig_four(v, e, finite, d0, d1, d2);
+        // the sum of the rounded values, so that a weight's two terms (d sc q
+        // and dmin m) see the same x
+        int t = dig_four(v, e, finite, d0, d1, d2);
+        t = dpp_add_i32<0xb1>(t);
+        t = dpp_add_i32<0x4e>(t);
+        t = dpp_add_i32<0x141>(t);
         const int g = dpad(tid + NT * k);
         pl[g] = d0;
         pl[kDigPlaneDw + g] = d1;
         pl[2 * kDigPlaneDw + g] = d2;
         if ((tid & 7) == 0) {
             const int sb = (tid + NT * k) >> 3;
-            xsum[sb] = finite ? t : __builtin_nanf("");
+            xsum[sb] = finite ? __builtin_ldexpf((float)t, e - 22) : __builtin_nanf("");
             xexp[sb] = e;
         }
     }
