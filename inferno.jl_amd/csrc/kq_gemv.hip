@@ -518,10 +518,9 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kwide(const uint8_t *__restri
 // leaves at most three blocks of its last step idle (16-block passes left up
 // to 15), and one sum over the lanes serves four rows.
 //
-// Digits: X = 65536 b2 + 256 b1 + b0 as above, rounded to nearest instead of
-// truncated (half the error), and with b0 and b1 signed too (the i8 product
-// takes no unsigned bytes): the bytes of X + 0x808080, each less 128.  The
-// sub-block sums are exact.
+// Digits: X = 65536 b2 + 256 b1 + b0 as above, but with b0 and b1 signed too
+// (the i8 product takes no unsigned bytes): the bytes of X + 0x808080, each
+// less 128.  The sub-block sums are exact.
 //
 // The weights come through a private ring of LDS slots per wave, filled by
 // direct-to-LDS copies: a quad of lanes wants four rows, and register loads in

@@ -13,9 +13,8 @@ namespace ihip {
 // residual add, or the SwiGLU of an unfused gate/up pair); resid may be y.
 hipError_t launch_gemv(int type, const void *w, const float *x, float *y, int inner, int outer,
                        hipStream_t s, const float *resid = nullptr, int epi = 0);
-// y = W (rmsnorm(x) .* nw) in one launch (the wide kernels' folded norm, per
-// workgroup or persistent by row count) for Q4_K / Q5_K rows of at most 16
-// blocks; hipErrorNotSupported otherwise.
+// y = W (rmsnorm(x) .* nw) in one launch (k_gemv_mdig's folded norm) for Q4_K /
+// Q5_K rows of at most 16 blocks; hipErrorNotSupported otherwise.
 bool gemv_norm_fusable(int type, int inner, int outer);
 hipError_t launch_gemv_norm(int type, const void *w, const float *x, const float *nw, float eps,
                             float *y, int inner, int outer, hipStream_t s);
@@ -249,7 +248,8 @@ hipError_t launch_quantize_q8k(const float *x, void *y, int64_t k, hipStream_t s
 hipError_t launch_gemv_q8k(int type, const void *w, const void *q8, float *out, int inner,
                            int outer, hipStream_t s);
 // x as fp32, quantized to Q8_K inside the launch where the kernel takes the
-// shape (Q4_K / Q5_K, at most 32768 columns, 16-byte aligned w and x); q8out
+// shape (Q4_K / Q5_K, at most 32768 columns; Q6_K of at most 6144 columns and
+// one round of rows; 16-byte aligned w and x); q8out
 // (optional) receives the Q8_K blocks; otherwise x is quantized into q8out or,
 // without it, into q8tmp (inner / 256 blocks) first.
 hipError_t launch_gemv_q8k_x(int type, const void *w, const float *x, void *q8out, void *q8tmp,
