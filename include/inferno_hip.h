@@ -362,10 +362,15 @@ int ihip_gemv_q8k_dev(int ggml_type, const void *w, const void *q8, float *out, 
                       int outer, ihip_stream stream);
 /* The same with x as fp32, quantized to Q8_K as ihip_quantize_row_q8_k_dev
  * does -- the reference's q{4,5,6}_k_gemv (src/kernels/quant_kernels.c:602-650)
- * as one device call.  Q4_K / Q5_K rows of at most 32768 columns with a
- * 16-byte aligned x run as one launch, and q8 (when not NULL) receives the
- * Q8_K blocks of x; other cases quantize x into q8 first, which they then
- * require (inner/256 * IHIP_Q8_K_BYTES, 4-byte aligned). */
+ * as one device call.  With a 16-byte aligned x, Q4_K / Q5_K rows of at most
+ * 32768 columns run as one launch, q8 may be NULL, and q8 (when not NULL)
+ * receives the Q8_K blocks of x.  Everything else requires q8 (inner/256 *
+ * IHIP_Q8_K_BYTES, 4-byte aligned) and leaves the blocks of x in it: Q6_K
+ * rows of at most 6144 columns, up to 16 rows per compute unit, with a 16-byte
+ * aligned w and x run as one launch too, the rest quantizes x into q8 first.
+ * So does every call whose out overlaps x: all of x has been read when the
+ * first row of out is written (without q8 it is IHIP_ERR_INVALID).  q8 and out
+ * must not overlap. */
 int ihip_gemv_q8k_x_dev(int ggml_type, const void *w, const float *x, float *out, void *q8,
                         int inner, int outer, ihip_stream stream);
 

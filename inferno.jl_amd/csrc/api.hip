@@ -1381,12 +1381,24 @@ int ihip_gemv_q8k_x_dev(int ggml_type, const void *w, const float *x, float *out
     if (((uintptr_t)w & wa) || ((uintptr_t)x & 3u) || ((uintptr_t)q8 & 3u) || ((uintptr_t)out & 3u))
         return fail(IHIP_ERR_INVALID, "w must be %d-byte aligned, x, q8 and out 4-byte aligned",
                     (int)wa + 1);
+    // The kernels that quantize x themselves read all of it in every workgroup
+    // while rows of out (and q8) are written: buffers that share a byte take the
+    // quantizing launch first, which has read x before a row is written.
+    const size_t xb = 4 * (size_t)inner, ob = 4 * (size_t)outer, qb = q8 ? q8k_bytes(inner) : 0;
+    const bool apart = !overlap(x, xb, out, ob) && !overlap(q8, qb, x, xb) && !overlap(q8, qb, out, ob);
     const bool one_launch = (ggml_type == kQ4_K || ggml_type == kQ5_K) && inner <= 32768 &&
                             ((uintptr_t)x & 15u) == 0;
     if (!one_launch && !q8)
         return fail(IHIP_ERR_INVALID, "this shape or type quantizes x into q8 first: pass q8 "
                                       "(inner/256 Q8_K blocks)");
-    hipError_t e = launch_gemv_q8k_x(ggml_type, w, x, q8, nullptr, out, inner, outer, (hipStream_t)stream);
+    if (!apart && !q8)
+        return fail(IHIP_ERR_INVALID, "x overlaps out: pass q8 (inner/256 Q8_K blocks), which x is "
+                                      "quantized into first");
+    hipError_t e;
+    if (apart)
+        e = launch_gemv_q8k_x(ggml_type, w, x, q8, nullptr, out, inner, outer, (hipStream_t)stream);
+    else if ((e = launch_quantize_q8k(x, q8, inner, (hipStream_t)stream)) == hipSuccess)
+        e = launch_gemv_q8k(ggml_type, w, q8, out, inner, outer, (hipStream_t)stream);
     if (e != hipSuccess)
         return fail(IHIP_ERR_HIP, "q8k gemv launch failed: %s", hipGetErrorString(e));
     return IHIP_OK;

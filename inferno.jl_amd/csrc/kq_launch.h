@@ -251,7 +251,8 @@ hipError_t launch_gemv_q8k(int type, const void *w, const void *q8, float *out, 
 // shape (Q4_K / Q5_K, at most 32768 columns; Q6_K of at most 6144 columns and
 // one round of rows; 16-byte aligned w and x); q8out
 // (optional) receives the Q8_K blocks; otherwise x is quantized into q8out or,
-// without it, into q8tmp (inner / 256 blocks) first.
+// without it, into q8tmp (inner / 256 blocks) first.  x, out and q8out must
+// not overlap: the one launch reads x while it writes the others.
 hipError_t launch_gemv_q8k_x(int type, const void *w, const float *x, void *q8out, void *q8tmp,
                              float *out, int inner, int outer, hipStream_t s);
 

@@ -313,7 +313,7 @@ def gemv_q8k_x(w: DeviceWeight, x: torch.Tensor, out: torch.Tensor = None, q8: t
     """out = W x in the reference C path's numerics with x given as fp32 (the
     reference's q{4,5,6}_k_gemv, src/kernels/quant_kernels.c:602-650): x is
     quantized to Q8_K inside the call; q8, when given (inner/256 * 292 bytes),
-    receives the blocks."""
+    receives the blocks (Q6_K, and an out that overlaps x, require it)."""
     if out is None:
         out = torch.empty(w.outer, dtype=torch.float32, device=x.device)
     check(lib().ihip_gemv_q8k_x_dev(w.ggml_type, _ptr(w.data), _ptr(x, torch.float32, "x"),

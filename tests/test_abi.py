@@ -127,6 +127,21 @@ def test_gemv_operands_that_race_are_refused():
     assert b"must not overlap" in L.ihip_last_error()
 
 
+def test_int8_gemv_in_place_needs_q8():
+    """The int8-activation GEMV that quantizes x in its own launch reads x in
+    every workgroup while rows of out are written: without q8 to quantize into
+    first, x overlapping out is refused for every type."""
+    import ctypes as C
+    from inferno_hip import _lib
+    L = _lib.lib()
+    w, x = C.c_void_p(1 << 20), C.c_void_p(1 << 24)
+    for t in (12, 13, 14):
+        for shift in (0, -4 * 60, 4 * 255):  # out starts with x, ends inside it, starts on its last value
+            out = C.c_void_p((1 << 24) + shift)
+            assert L.ihip_gemv_q8k_x_dev(t, w, x, out, None, 256, 64, None) == _lib.IHIP_ERR_INVALID, (t, shift)
+            assert (b"x overlaps out" if t != 14 else b"pass q8") in L.ihip_last_error()
+
+
 def test_weight_bytes_follow_the_block_layouts():
     """ihip_weight_bytes (the offsets of a weight group's members) against the
     block sizes of the formats (src/QuantsCPU.jl:22-26); no device

@@ -240,3 +240,39 @@ def test_q8k_argument_errors():
     w = D.DeviceWeight(dev(np.zeros(34 * 8, np.uint8)), synth.Q8_0, 256, 1)
     with pytest.raises(IHIPArgumentError):
         D.gemv_q8k(w, q8)
+
+
+@pytest.mark.parametrize("t", K_TYPES)
+@pytest.mark.parametrize("outer,inner,shift", [(4096, 4096, 0), (1024, 4096, 2048), (4096, 1024, -3000), (257, 6144, 6000), (5, 256, 0)])
+def test_gemv_q8k_x_in_place(t, outer, inner, shift):
+    """out over x (out starts `shift` floats into x): x is quantized before the
+    first row is written."""
+    from inferno_hip import device as D
+    say(f"gemv_q8k_x type {t} {outer}x{inner} out at x + {shift}")
+    rng = synth.rng_for(0x1A + outer + inner)
+    w, x = synth.weight(rng, t, outer, inner), synth.activations(rng, inner)
+    want, blocks = oracle.gemv_q8k(t, w, x, inner, outer), oracle.quantize_row_q8k(x)
+    a = max(0, -shift)
+    buf = torch.zeros(max(a + inner, a + shift + outer), device="cuda")
+    xd, out = buf[a:a + inner], buf[a + shift:a + shift + outer]
+    q8 = torch.zeros(blocks.size, dtype=torch.uint8, device="cuda")
+    for _ in range(3):
+        xd.copy_(dev(x))
+        D.gemv_q8k_x(D.DeviceWeight(dev(w), t, inner, outer), xd, out, q8)
+        assert same_bits(out.cpu().numpy(), want)
+        assert np.array_equal(q8.cpu().numpy(), blocks)
+
+
+@pytest.mark.parametrize("t", K_TYPES)
+def test_gemv_q8k_x_blocks_over_x(t):
+    """q8 over the one block of x it is made from."""
+    from inferno_hip import device as D
+    say(f"gemv_q8k_x type {t} q8 over x")
+    rng = synth.rng_for(0x1B)
+    outer, inner = 1000, 256
+    w, x = synth.weight(rng, t, outer, inner), synth.activations(rng, inner)
+    xd = dev(x)
+    q8 = xd.view(torch.uint8)[:292]
+    out = D.gemv_q8k_x(D.DeviceWeight(dev(w), t, inner, outer), xd, None, q8)
+    assert same_bits(out.cpu().numpy(), oracle.gemv_q8k(t, w, x, inner, outer))
+    assert np.array_equal(q8.cpu().numpy(), oracle.quantize_row_q8k(x))
