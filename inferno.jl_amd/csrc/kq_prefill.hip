@@ -1099,14 +1099,16 @@ __global__ __launch_bounds__(256) void k_prefill_splits_sum(float *__restrict__ 
 // 4096 13.7 against 14.9; error against 64 bits at 509 x 2048 x 2048 1.1e-7
 // against 8.2e-7 (fewer roundings: 64 sums of 32 columns instead of 2048).
 //
-// The matrix cores take bf16 subnormals as zeros, and a sub-block's sum could
-// overflow before its scale is applied.  Each token's largest magnitude is
-// found along the way; a tile with a token outside 2^-80 .. 2^118 is computed
-// again on tokens scaled by powers of two, which is exact, and a token that
-// holds an infinity value by value.
+// The matrix cores take bf16 subnormals as zeros, and sums could overflow
+// before a scale is applied or before the two terms cancel.  Each token's
+// largest magnitude is found along the way; a tile with a token outside 2^-80 ..
+// 2^76 is computed again on tokens scaled by powers of two, which is exact
+// (below 2^76 no partial sum reaches 2^127: a scale times a quant is below
+// 2^26, a row shorter than 2^24), and a token that holds an infinity value by
+// value.
 constexpr int PFX_WSTAGE = 64 * 48; // header and the pair's 32 quant bytes of 64 rows
 constexpr int PFX_LD = 72;          // floats per row of a partial tile
-constexpr float kSplitMinX = 0x1p-80f, kSplitMaxX = 0x1p118f;
+constexpr float kSplitMinX = 0x1p-80f, kSplitMaxX = 0x1p76f;
 __host__ __device__ constexpr int pfx_wave_bytes(int tt) { return 2 * 4096 * tt + PFX_WSTAGE; }
 static_assert(8 * pfx_wave_bytes(2) <= 160 * 1024 - 256, "the eight waves' stages fit the 160 KB of LDS");
 static_assert(PFX_LD * 64 * 4 <= pfx_wave_bytes(2) && PFX_LD * 32 * 4 <= pfx_wave_bytes(1), "and the partial tiles");

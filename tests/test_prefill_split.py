@@ -91,3 +91,20 @@ def test_error_is_no_larger_than_fp32_products_in_order(bias):
     there = np.linalg.norm(serial - exact)
     print(f"bias {bias}: {here / np.linalg.norm(exact):.2e}, fp32 in order {there / np.linalg.norm(exact):.2e}", flush=True)
     assert here <= there
+
+
+@pytest.mark.parametrize("top", [2.0 ** 75, 2.0 ** 90, 2.0 ** 117])
+def test_terms_that_cancel_do_not_overflow(top):
+    """Weights of zero beside a large scale (quants 0, scale 63, d = 1): the two
+    terms they are split into are 472 times the activations and cancel."""
+    print(f"split prefill cancelling terms, x to {top}", flush=True)
+    rng = synth.rng_for(0x5B1B)
+    T, outer, inner = 33, 65, 512
+    w = np.zeros((outer, inner // 256, 144), np.uint8)
+    w[:, :, 0:2] = np.frombuffer(np.float16(1).tobytes(), np.uint8)  # d = 1, dmin = 0
+    w[:, :, 4:8], w[:, :, 12:16] = 0xFF, 0x0F  # the eight scales 63, the mins 0
+    w[:, :, 8:12] = 0
+    w[:, :, 16::32] = 1  # one weight of 63 in each 64
+    w = w.reshape(-1)
+    X = (rng.uniform(0.5, 1, (T, inner)) * top).astype(np.float32)
+    _check(w, X, outer, inner, f"cancelling terms, x to {top}")
