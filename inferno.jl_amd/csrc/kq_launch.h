@@ -231,7 +231,7 @@ hipError_t launch_prefill_gemm(const void *w, void *xh, float *Y, int T, int inn
 // 32-token tile taking 0.58-0.62 of a 64-token one's time.  Measured on MI355X
 // (us, 32 / 64 tokens): 256 x 2048 x 2048 13.6 / 20.1, 300 x 4096 x 4096 65.2 /
 // 71.5, 200 x 4096 x 4096 43.5 / 40.3, 509 x 2048 x 2048 25.9 / 23.6.
-constexpr int kPrefillSplitMaxK = 1 << 24; // longer rows are computed value by value
+constexpr int kPrefillSplitMaxK = 1 << 24; // 64 rows of X or W of this length are within 32-bit byte offsets
 inline int prefill_split_tokens(int T, int outer, int ncu)
 {
     const int64_t cus = ncu > 0 ? ncu : 1, nt = ((int64_t)outer + 63) / 64;

@@ -1103,14 +1103,22 @@ __global__ __launch_bounds__(256) void k_prefill_splits_sum(float *__restrict__ 
 // before a scale is applied or before the two terms cancel.  Each token's
 // largest magnitude is found along the way; a tile with a token outside 2^-80 ..
 // 2^76 is computed again on tokens scaled by powers of two, which is exact
-// (below 2^76 no partial sum reaches 2^127: a scale times a quant is below
-// 2^26, a row shorter than 2^24), and a token that holds an infinity value by
-// value.
+// (below 2^76 no partial sum reaches 2^127: a scale and a quant are below 2^26,
+// a row shorter than 2^24).  A token that holds an infinity has infinite or
+// NaN outputs, which only the signs decide: +Inf where every infinity meets a
+// weight of its own sign, -Inf where every one meets the other, NaN otherwise.
+// A tile with such a token runs once more on the signs of the weights (1, 0,
+// -1) and of the infinities (other values 0): its sums, whole numbers, are the
+// number of the token's infinities, minus that, or neither.
+// Measured (us a call; fp32 matrix products): 509 x 2048 x 2048 24.7 without an
+// infinity, 42 with one, 44 with one in every token (62); 512 x 4096 x 4096 83,
+// 148, 162 (210); 512 x 256 x 4096 14.5, 23.3, 24.3 (16.9).
 constexpr int PFX_WSTAGE = 64 * 48; // header and the pair's 32 quant bytes of 64 rows
 constexpr int PFX_LD = 72;          // floats per row of a partial tile
 constexpr float kSplitMinX = 0x1p-80f, kSplitMaxX = 0x1p76f;
+enum { kSplitPlain, kSplitScaled, kSplitSigns }; // what a pass over the tile multiplies
 __host__ __device__ constexpr int pfx_wave_bytes(int tt) { return 2 * 4096 * tt + PFX_WSTAGE; }
-static_assert(8 * pfx_wave_bytes(2) <= 160 * 1024 - 256, "the eight waves' stages fit the 160 KB of LDS");
+static_assert(8 * pfx_wave_bytes(2) <= 160 * 1024 - 512, "the eight waves' stages fit the 160 KB of LDS");
 static_assert(PFX_LD * 64 * 4 <= pfx_wave_bytes(2) && PFX_LD * 32 * 4 <= pfx_wave_bytes(1), "and the partial tiles");
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -1161,15 +1169,65 @@ __device__ __forceinline__ void pfx_parts(float4 lo, float4 hi, bf16x8 (&p)[3], 
     }
 }
 
-template <int TT>
+// Signs of the weights d1 q - m1 of the same nibbles (NaN for NaN) in bf16.
+// d1 q and m1 are exact in fp32, so the difference has the sign of the weight.
+__device__ __forceinline__ bf16x8 pfx_signs(uint2 bytes, float d1, float m1)
+{
+    uint32_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t s[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const uint32_t q = ((i < 2 ? bytes.x : bytes.y) >> (16 * (i & 1) + 8 * k)) & 15u;
+            const float v = d1 * (float)q - m1;
+            s[k] = __float_as_uint(v > 0.0f ? 1.0f : v < 0.0f ? -1.0f : v);
+        }
+        d[i] = __builtin_amdgcn_perm(s[1], s[0], 0x07060302u);
+    }
+    return __builtin_bit_cast(bf16x8, make_uint4(d[0], d[1], d[2], d[3]));
+}
+
+// 8 values of x -> 1 or -1 for the infinities among them, NaN for NaN, 0 for
+// the rest; counts the infinities.
+__device__ __forceinline__ bf16x8 pfx_infinities(float4 lo, float4 hi, int &count)
+{
+    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    uint32_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t s[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float x = v[2 * i + k];
+            const bool inf = fabsf(x) == __builtin_inff();
+            count += inf ? 1 : 0;
+            s[k] = __float_as_uint(inf ? copysignf(1.0f, x) : x != x ? __builtin_nanf("") : 0.0f);
+        }
+        d[i] = __builtin_amdgcn_perm(s[1], s[0], 0x07060302u);
+    }
+    return __builtin_bit_cast(bf16x8, make_uint4(d[0], d[1], d[2], d[3]));
+}
+
+// FAR: rows past kPrefillSplitMaxK columns, whose bytes 64 rows (32 tokens)
+// away need 64-bit offsets.
+template <int TT, bool FAR>
 __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__restrict__ W,
                                                               const float *__restrict__ X,
                                                               float *__restrict__ Y, int T, int K, int N,
-                                                              int mtiles, int ntiles, int by_value)
+                                                              int mtiles, int ntiles)
 {
     constexpr int XC = 4 * TT, XST = 4096 * TT, WAVE = pfx_wave_bytes(TT); // 1 KB copies and bytes of an X stage
     __shared__ __attribute__((aligned(16))) uint8_t lds[8 * WAVE];
     __shared__ uint32_t tokmax[32 * TT]; // the tokens' largest |x| (bits)
+    __shared__ int tokinf[32 * TT];      // and their infinities
+    using Offset = std::conditional_t<FAR, size_t, uint32_t>;
+    auto copy16 = [](const uint8_t *base, Offset off, uint32_t dst) {
+        if constexpr (FAR)
+            lds_copy16(base + off, dst);
+        else
+            pf_copy16(base, off, dst);
+    };
 
     const int tiles = mtiles * ntiles;
     const int lin = prefill_lin((int)blockIdx.x, tiles, 1);
@@ -1182,18 +1240,22 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
     const size_t row_bytes = (size_t)nk * 144;
     const PrefillSplit ps = prefill_split_of(lin, mtiles, ntiles, nk, 1);
     const int m0 = ps.mt * (32 * TT), n0 = ps.nt * 64;
-    if (tid < 32 * TT)
+    if (tid < 32 * TT) {
         tokmax[tid] = 0u;
+        tokinf[tid] = 0;
+    }
     __syncthreads();
 
     float16v acc[TT][2];
     float big[TT];
-    int shift[TT];
-    const int nb = by_value ? 0 : (nk - half + 1) >> 1, ns = 2 * nb; // this wave's blocks and stages
-    auto product = [&](auto scaled) { // scaled: of the tokens times 2^shift
+    int shift[TT], infs[TT];
+    const int nb = (nk - half + 1) >> 1, ns = 2 * nb; // this wave's blocks and stages
+    auto product = [&](auto mode) { // scaled: of the tokens times 2^shift
+        constexpr bool SCALED = decltype(mode)::value == kSplitScaled, SIGNS = decltype(mode)::value == kSplitSigns;
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
             big[t] = 0.0f;
+            infs[t] = 0;
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -1203,19 +1265,19 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
             return;
         // copies: 8 tokens x 128 bytes each of an X stage, chunk c of token m
         // at place c ^ (m / 2 % 8) of its 128 bytes (the 16 lanes of a 128-bit
-        // read hit distinct banks), and 64 rows x 3 pieces of the blocks.  The
-        // offsets stay below 2^32: the launcher bounds K.  Rows past T or N
-        // re-read the last one, stages past the last repeat it.
-        uint32_t xo[XC], wo[3];
+        // read hit distinct banks), and 64 rows x 3 pieces of the blocks.  32-bit
+        // offsets suffice: the launcher bounds K.  Rows past T or N re-read the
+        // last one, stages past the last repeat it.
+        Offset xo[XC], wo[3];
 #pragma unroll
         for (int i = 0; i < XC; ++i) {
             const int m = 8 * i + (lane >> 3), c = (lane & 7) ^ ((m >> 1) & 7);
-            xo[i] = (uint32_t)min(m, T - 1 - m0) * ((uint32_t)K * 4u) + 16u * (uint32_t)c;
+            xo[i] = (Offset)min(m, T - 1 - m0) * ((Offset)K * 4u) + 16u * (uint32_t)c;
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
             const int q = 64 * i + lane, row = q / 3, piece = q - 3 * row;
-            wo[i] = (uint32_t)min(row, N - 1 - n0) * (uint32_t)row_bytes + (piece ? 32u * j + 16u * piece : 0u);
+            wo[i] = (Offset)min(row, N - 1 - n0) * (Offset)row_bytes + (piece ? 32u * j + 16u * piece : 0u);
         }
         const uint8_t *Xb = reinterpret_cast<const uint8_t *>(X + (size_t)m0 * K + 256 * half + 64 * j);
         const uint8_t *Wb = W + (size_t)n0 * row_bytes + 144 * half;
@@ -1227,13 +1289,13 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
             const uint8_t *b = Xb + (size_t)(st >> 1) * 2048 + 128 * (st & 1);
 #pragma unroll
             for (int i = 0; i < XC; ++i)
-                pf_copy16(b, xo[i], xdst + XST * (n & 1) + 1024 * i);
+                copy16(b, xo[i], xdst + XST * (n & 1) + 1024 * i);
         };
         auto issue_w = [&](int i) {
             const uint8_t *b = Wb + (size_t)min(i, nb - 1) * 288;
 #pragma unroll
             for (int k = 0; k < 3; ++k)
-                pf_copy16(b, wo[k], wdst + 1024 * k);
+                copy16(b, wo[k], wdst + 1024 * k);
         };
         const uint8_t *xl = mine + 128 * li, *wl = mine + 2 * XST + 48 * li;
         const int f = (li >> 1) & 7;
@@ -1241,6 +1303,7 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
         float4 xr[TT][2][2];
         uint2 qs[2][2];
         float ds[2][2], ndm[2], xsum[2][TT]; // [row tile or sub-block][..]
+        float m1[SIGNS ? 2 : 1][2];
         auto read_x = [&](int s) {
 #pragma unroll
             for (int t = 0; t < TT; ++t)
@@ -1257,16 +1320,31 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
             for (int u = 0; u < 2; ++u)
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    const uint2 b = qs[u][c];
-                    wq[u][c] = pfx_quants(s ? make_uint2(b.x >> 4, b.y >> 4) : b);
+                    const uint2 b = s ? make_uint2(qs[u][c].x >> 4, qs[u][c].y >> 4) : qs[u][c];
+                    if constexpr (SIGNS)
+                        wq[u][c] = pfx_signs(b, 2.0f * ds[u][s], m1[u][s]);
+                    else
+                        wq[u][c] = pfx_quants(b);
                 }
+            if constexpr (SIGNS) {
+#pragma unroll
+                for (int t = 0; t < TT; ++t)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const bf16x8 p = pfx_infinities(xr[t][c][0], xr[t][c][1], infs[t]);
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p, wq[u][c], acc[t][u], 0, 0, 0);
+                    }
+                return;
+            }
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
                 bf16x8 p[2][3];
                 xsum[s][t] = 0.0f;
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    if constexpr (decltype(scaled)::value) {
+                    if constexpr (SCALED) {
 #pragma unroll
                         for (int e = 0; e < 2; ++e) {
                             float4 &v = xr[t][c][e];
@@ -1324,6 +1402,10 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
                 ds[u][1] = 0.5f * d * scB;
                 // this lane half's sub-block of the pair
                 ndm[u] = fmaf(15.0f, h ? ds[u][1] : ds[u][0], -(dmin * (h ? mB : mA)));
+                if constexpr (SIGNS) {
+                    m1[u][0] = dmin * mA;
+                    m1[u][1] = dmin * mB;
+                }
             }
             stage(0);
             __builtin_amdgcn_s_waitcnt((XC + 3) | 0x0f70);
@@ -1333,6 +1415,8 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
             asm volatile("" ::: "memory");
             issue_x(2 * i + 3);
             stage(1);
+            if constexpr (SIGNS)
+                continue;
             // lane (li, h): token li's sum over the pair's sub-block h
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
@@ -1346,7 +1430,7 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
         }
         __builtin_amdgcn_s_waitcnt(0x0070); // the last (unused) copies have landed
     };
-    product(std::false_type{});
+    product(std::integral_constant<int, kSplitPlain>{});
 #pragma unroll
     for (int t = 0; t < TT; ++t)
         atomicMax(&tokmax[32 * t + li], __float_as_uint(big[t]));
@@ -1356,36 +1440,38 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
         const float b = __uint_as_float(tokmax[m]);
         return b > 0.0f && b < __builtin_inff() ? -__builtin_amdgcn_frexp_expf(b) : 0;
     };
-    bool out_of_range = false;
+    bool out_of_range = false, infinite = false;
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
         const float b = __uint_as_float(tokmax[32 * t + li]);
+        infinite |= b == __builtin_inff();
         out_of_range |= (b > 0.0f && b < kSplitMinX) || (b >= kSplitMaxX && b < __builtin_inff());
         shift[t] = shift_of(32 * t + li);
     }
     const bool again = __ballot(out_of_range) != 0; // the same in every wave
     if (again) {
-        product(std::true_type{});
+        product(std::integral_constant<int, kSplitScaled>{});
         __syncthreads();
     }
-    // lane (li, h), register r of acc[t][u]: token 32 t + 8 (r / 4) + 4 h + r % 4, row 32 u + li
+    // Y of the tokens with (inf) or without an infinity from the waves' partial
+    // tiles.  Lane (li, h), register r of acc[t][u]: token 32 t + 8 (r / 4) + 4 h
+    // + r % 4, row 32 u + li.
     float *const P = reinterpret_cast<float *>(lds);
+    auto write = [&](bool inf) {
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
+        for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+            for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                P[(32 * TT * wave + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3)) * PFX_LD + 32 * u + li] = acc[t][u][r];
-    __syncthreads();
+                for (int r = 0; r < 16; ++r)
+                    P[(32 * TT * wave + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3)) * PFX_LD + 32 * u + li] = acc[t][u][r];
+        __syncthreads();
 #pragma unroll
-    for (int p = 0; p < TT; ++p) {
-        const int ml = 32 * p + (tid >> 4), nl = 4 * (tid & 15), m = m0 + ml, n = n0 + nl;
-        if (m >= T || n >= N)
-            continue;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (!by_value && tokmax[ml] < 0x7f800000u) {
-            const int sm = again ? -shift_of(ml) : 0;
+        for (int p = 0; p < TT; ++p) {
+            const int ml = 32 * p + (tid >> 4), nl = 4 * (tid & 15), m = m0 + ml, n = n0 + nl;
+            if (m >= T || n >= N || (tokmax[ml] == 0x7f800000u) != inf)
+                continue;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int w = 0; w < 8; ++w) {
                 const float4 q = *reinterpret_cast<const float4 *>(P + (32 * TT * w + ml) * PFX_LD + nl);
@@ -1394,37 +1480,35 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
                 v.z += q.z;
                 v.w += q.w;
             }
-            v = make_float4(__builtin_ldexpf(v.x, sm), __builtin_ldexpf(v.y, sm), __builtin_ldexpf(v.z, sm),
-                            __builtin_ldexpf(v.w, sm));
-        } else {
-            // weight element 64 jj + 32 hh + l of a block is (d sc) q_l - dmin m
-            // with q_l the low (hh = 0) or high nibble of qs[32 jj + l]
-            // (src/Dequant.jl:364-371)
-            float a[4] = {0.f, 0.f, 0.f, 0.f};
-            for (int e = 0; e < 4 && n + e < N; ++e)
-                for (int kb = 0; kb < nk; ++kb) {
-                    const uint8_t *blk = W + (size_t)(n + e) * row_bytes + (size_t)kb * 144;
-                    const float *xv = X + (size_t)m * K + 256 * (size_t)kb;
-                    const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
-                    const float d = h2f(hd.x & 0xffffu), dmin = h2f(hd.x >> 16);
-                    for (int k = 0; k < 256; ++k) {
-                        uint32_t sc, mn;
-                        k_scale_min(hd.y, hd.z, hd.w, k >> 5, sc, mn);
-                        const uint32_t q = (blk[16 + 32 * (k >> 6) + (k & 31)] >> (4 * ((k >> 5) & 1))) & 15u;
-                        a[e] = fmaf(d * (float)sc * (float)q - dmin * (float)mn, xv[k], a[e]);
-                    }
-                }
-            v = make_float4(a[0], a[1], a[2], a[3]);
+            if (inf) {
+                const float k = (float)tokinf[ml];
+                auto sign = [&](float a) { return a == k ? __builtin_inff() : a == -k ? -__builtin_inff() : __builtin_nanf(""); };
+                v = make_float4(sign(v.x), sign(v.y), sign(v.z), sign(v.w));
+            } else {
+                const int sm = again ? -shift_of(ml) : 0;
+                v = make_float4(__builtin_ldexpf(v.x, sm), __builtin_ldexpf(v.y, sm), __builtin_ldexpf(v.z, sm),
+                                __builtin_ldexpf(v.w, sm));
+            }
+            float *y = Y + (size_t)m * (size_t)N + n;
+            if ((N & 3) == 0) {
+                *reinterpret_cast<float4 *>(y) = v;
+            } else {
+                y[0] = v.x;
+                if (n + 1 < N) y[1] = v.y;
+                if (n + 2 < N) y[2] = v.z;
+                if (n + 3 < N) y[3] = v.w;
+            }
         }
-        float *y = Y + (size_t)m * (size_t)N + n;
-        if ((N & 3) == 0) {
-            *reinterpret_cast<float4 *>(y) = v;
-        } else {
-            y[0] = v.x;
-            if (n + 1 < N) y[1] = v.y;
-            if (n + 2 < N) y[2] = v.z;
-            if (n + 3 < N) y[3] = v.w;
-        }
+    };
+    write(false);
+    if (__ballot(infinite) != 0) { // the same in every wave
+        __syncthreads();
+        product(std::integral_constant<int, kSplitSigns>{});
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+            atomicAdd(&tokinf[32 * t + li], infs[t]);
+        __syncthreads();
+        write(true);
     }
 }
 
@@ -1433,17 +1517,18 @@ hipError_t launch_prefill_q4k_f32(const void *w, const float *X, float *Y, int T
 {
     if (T <= 0 || outer <= 0 || inner <= 0 || inner % 256 || (int64_t)T * outer > (int64_t)INT32_MAX)
         return hipErrorInvalidValue;
-    const int tt = prefill_split_tokens(T, outer, device_cus()) / 32;
+    const int tt = inner > kPrefillSplitMaxK ? 1 : prefill_split_tokens(T, outer, device_cus()) / 32;
     const int mtiles = (T + 32 * tt - 1) / (32 * tt), ntiles = (outer + 63) / 64;
-    // 64 rows of X, and 64 rows of W, are addressed by 32-bit byte offsets
-    const int by_value = inner > kPrefillSplitMaxK;
     const dim3 grid(prefill_grid(mtiles * ntiles, 1)), block(512);
-    if (tt == 1)
-        hipLaunchKernelGGL(k_prefill_q4k_split<1>, grid, block, 0, s, (const uint8_t *)w, X, Y, T, inner, outer,
-                           mtiles, ntiles, by_value);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, (const uint8_t *)w, X, Y, T, inner, outer, mtiles, ntiles);
+    };
+    if (inner > kPrefillSplitMaxK)
+        launch(k_prefill_q4k_split<1, true>);
+    else if (tt == 1)
+        launch(k_prefill_q4k_split<1, false>);
     else
-        hipLaunchKernelGGL(k_prefill_q4k_split<2>, grid, block, 0, s, (const uint8_t *)w, X, Y, T, inner, outer,
-                           mtiles, ntiles, by_value);
+        launch(k_prefill_q4k_split<2, false>);
     return hipGetLastError();
 }
 

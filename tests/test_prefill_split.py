@@ -108,3 +108,73 @@ def test_terms_that_cancel_do_not_overflow(top):
     w = w.reshape(-1)
     X = (rng.uniform(0.5, 1, (T, inner)) * top).astype(np.float32)
     _check(w, X, outer, inner, f"cancelling terms, x to {top}")
+
+
+# a tile of 64 tokens, one of 32; K shared unevenly by the wave halves
+@pytest.mark.parametrize("T,outer,inner", [(600, 2050, 768), (70, 66, 2304), (5, 3, 256)])
+def test_infinities_in_many_tokens(T, outer, inner):
+    """Infinities of one sign, of both and beside a NaN, on weights of either
+    sign and of zero, in tokens of ordinary and of extreme size: every output is
+    what IEEE sums give."""
+    print(f"split prefill with infinities T={T} {outer}x{inner}", flush=True)
+    rng = synth.rng_for(0x5B1C + T)
+    w = synth.weight(rng, synth.Q4_K, outer, inner)
+    blocks = w.reshape(outer, inner // 256, 144)
+    zero = np.arange(outer) % 3 == 1
+    blocks[zero, 0, 4:16] = 0  # rows whose first block has scales and mins of zero
+    X = rng.standard_normal((T, inner)).astype(np.float32)
+    X[1::5] *= np.float32(2.0) ** rng.integers(-140, 120, X[1::5].shape[0])[:, None].astype(np.float32)
+    kinds = np.arange(T) % 5  # 0 finite, 1 one infinity, 2 several of one sign, 3 of both, 4 beside a NaN
+    for t in range(T):
+        n = (0, 1, 4, 4, 2)[kinds[t]]
+        at = rng.integers(0, inner, n)
+        X[t, at] = np.inf if t % 2 else -np.inf
+        if kinds[t] == 2:  # where a row's weights have one sign, it is the result's
+            X[t, at[1:]] = X[t, at[0]]
+        if kinds[t] == 3:
+            X[t, at[1::2]] = -X[t, at[0]]
+        if kinds[t] == 4:
+            X[t, (at[1] + 1) % inner] = np.nan
+    wf = oracle.dequant(synth.Q4_K, w, inner * outer).reshape(outer, inner).astype(np.float64)
+    got = _product(w, X, outer, inner)
+    seen = set()
+    with np.errstate(invalid="ignore"):
+        for t in range(T):
+            if kinds[t] == 0:
+                continue
+            bad = np.flatnonzero(~np.isfinite(X[t]))
+            want = (X[t, bad].astype(np.float64)[None, :] * wf[:, bad]).sum(axis=1)
+            assert np.array_equal(got[t], want, equal_nan=True), t
+            seen |= {str(v) for v in np.unique(want[np.isfinite(want) == 0])}
+    assert {"inf", "-inf", "nan"} <= seen
+    fin = kinds == 0
+    tol = 1e-5 * np.linalg.norm(wf, axis=1)[None, :] * np.linalg.norm(X[fin].astype(np.float64), axis=1)[:, None] + 2.0 ** -149
+    assert np.all(np.abs(got[fin] - X[fin].astype(np.float64) @ wf.T) <= tol)
+
+
+def test_rows_past_32_bit_offsets():
+    """Rows of 2^24 + 256 columns: tokens and weight rows addressed by 64 bits."""
+    rng = synth.rng_for(0x5B1D)
+    T, outer, inner = 33, 3, (1 << 24) + 256
+    print(f"split prefill T={T} {outer}x{inner}", flush=True)
+    row = synth.weight(rng, synth.Q4_K, outer, 4096).reshape(outer, 16, 144)
+    w = np.concatenate([np.tile(row, (1, inner // 4096, 1)), row[:, :1]], axis=1)  # 4097 x 16 + 1 blocks
+    x = rng.standard_normal(4096).astype(np.float32)
+    import torch
+    from inferno_hip import device as D
+    dw = D.DeviceWeight(torch.from_numpy(np.ascontiguousarray(w).reshape(-1)).cuda(), synth.Q4_K, inner, outer)
+    X = torch.zeros(T, inner, device="cuda")
+    xd = torch.from_numpy(x).cuda()
+    scales = 1.0 + torch.arange(T, device="cuda") / 8
+    X[:, : inner - 256].view(T, -1, 4096).copy_(xd * scales[:, None, None])
+    X[:, inner - 256:] = xd[:256] * scales[:, None]
+    got = D.prefill_q4_k_f32(dw, X).cpu().numpy().astype(np.float64)
+    wf = oracle.dequant(synth.Q4_K, row.reshape(-1), 4096 * outer).reshape(outer, 4096).astype(np.float64)
+    n = inner // 4096
+    x8 = (x[None, :] * scales.cpu().numpy()[:, None]).astype(np.float64)
+    want = n * (x8 @ wf.T) + x8[:, :256] @ wf[:, :256].T
+    norms = np.sqrt(n) * np.linalg.norm(wf, axis=1)[None, :] * np.sqrt(n) * np.linalg.norm(x8, axis=1)[:, None]
+    # the row bound: a wave adds 65538 sub-block sums in order, each rounding
+    # 2^-24 of a running sum of about a 64th of the norms' product (the cosine of
+    # 4096 random values): 6e-5 if every rounding went the same way
+    assert np.max(np.abs(got - want) / norms) <= 1e-4
