@@ -38,6 +38,7 @@
 #include <type_traits>
 #include "kq_common.h"
 #include "kq_launch.h"
+#include "kq_gemv_plan.h"
 #include "kq_sdig_plan.h"
 
 namespace ihip {
@@ -497,6 +498,19 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kwide(const uint8_t *__restri
 {
     kwide_body<FMT, R, GATEUP, GATEUP && EXT, !GATEUP && EXT, NWV>(W, W2, x, y, outer, nblk, nw, eps,
                                                                    resid, epi);
+}
+
+// y = W (rmsnorm(x) .* nw) for one weight: the gate/up pass's folded norm
+// (x .* nw staged, the row sums scaled by 1/sqrt(mean(x^2) + eps)) in front of
+// a plain GEMV, e.g. the grouped wq/wk/wv behind a layer's input norm
+// (src/ModelCPU.jl:903, 789-791), where norm_takes_wide says so.
+template <int FMT, int R, int NWV>
+__global__ __launch_bounds__(NWV * 64) void k_gemv_kwide_norm(const uint8_t *__restrict__ W,
+                                                              const float *__restrict__ x, float *y,
+                                                              int outer, int nblk,
+                                                              const float *__restrict__ nw, float eps)
+{
+    kwide_body<FMT, R, false, true, false, NWV>(W, nullptr, x, y, outer, nblk, nw, eps, nullptr, 0);
 }
 
 // ------------------------------------------------------------------------
@@ -1143,6 +1157,22 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kpers(const uint8_t *__restri
     __shared__ float ssw[NWV];
     kpers_run<FMT, R, GATEUP, GATEUP && EXT, !GATEUP && EXT, NWV, NB>(W, W2, x, y, outer, nblk, nw, eps,
                                                                       resid, epi, xbuf, xsum, xexp, ssw);
+}
+
+// The persistent kernel with the folded norm on a single weight (as
+// k_gemv_kwide_norm).
+template <int FMT, int R, int NWV, int NB>
+__global__ __launch_bounds__(NWV * 64) void k_gemv_kpers_norm(const uint8_t *__restrict__ W,
+                                                              const float *__restrict__ x, float *y,
+                                                              int outer, int nblk,
+                                                              const float *__restrict__ nw, float eps)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t xbuf[3 * kDigPlaneDw];
+    __shared__ __attribute__((aligned(16))) float xsum[128];
+    __shared__ __attribute__((aligned(8))) int xexp[128];
+    __shared__ float ssw[NWV];
+    kpers_run<FMT, R, false, true, false, NWV, NB>(W, nullptr, x, y, outer, nblk, nw, eps, nullptr, 0,
+                                                   xbuf, xsum, xexp, ssw);
 }
 
 // ------------------------------------------------------------------------
@@ -1843,13 +1873,6 @@ int device_cus()
     return ncu;
 }
 
-// Rows of at most 16 blocks with at least four 8-wave row groups per wave
-// over one workgroup per CU take the persistent kernel.
-static bool kwide_takes_kpers(int nblk, int outer) { return nblk <= 16 && outer >= 4 * 8 * 256; }
-
-// No more one-row workgroups of 8 waves than CUs: one row per wave.
-static bool kwide_one_row(int outer) { return (outer + 7) / 8 <= device_cus(); }
-
 // Rows of at most 16 steps of 1024 columns on the matrix cores: waves and ring
 // depth by the row's steps and the format's slot (3 to 5 KB a wave and slot,
 // beside 4 KB of digits a step).
@@ -1863,32 +1886,6 @@ constexpr MdPlan mdig_plan(int type, int nstep)
     if (type == kQ6_K && nstep <= 12)
         return {12, 2, 12};
     return type == kQ6_K || type == kQ8_0 ? MdPlan{8, 2, 16} : MdPlan{12, 2, 16};
-}
-// Which rows take it, by format, length and (gate/up) kind only: a row's sum is
-// the same whatever launch it is in, and the two kernels' differ.  The wide
-// kernels spread a row's blocks over 16 lane positions, this one over 4 a
-// step, and it starts later (x goes through LDS twice).  So the wide kernels
-// keep the Q4_K / Q5_K rows that fill their lanes, and the short Q4_K ones.
-// Measured on MI355X (us, graph replays over weights in HBM, wide / this):
-// Q4_K 2560 x 9728 8.6 / 6.3, 5120 x 5120 7.8 / 5.6, 4096 x 14336 10.6 / 9.9,
-// 4096 x 4096 4.1 / 4.6, 12288 x 4096 7.4 / 7.8, 3584 x 2560 3.45 / 3.73; Q5_K
-// 4096 x 2048 4.1 / 3.5, 9728 x 2560 7.4 / 6.5, 4096 x 4096 4.8 / 5.1; gate/up
-// Q4_K 6144 x 2048 7.2 / 5.7, 13824 x 5120 20.6 / 17.2, 10240 x 3584 11.0 / 10.5,
-// 12288 x 4096 12.8 / 13.0; Q5_K 9728 x 2560 12.3 / 9.7, 12288 x 4096 15.8 / 15.5;
-// the folded norm Q4_K 6144 x 4096 6.6 / 6.0.  Q6_K (streamed / this) 4096 x
-// 12288 12.4 / 11.7, 2560 x 9728 12.1 / 7.9, 5120 x 13824 26.9 / 15.9, 1024 x 4096
-// 4.9 / 3.6, 12288 x 4096 11.2 / 11.5; Q8_0 5003 x 2720 8.4 / 5.8, 2560 x 9728 11.2 /
-// 8.3; IQ4_NL 5120 x 5120 10.7 / 6.8, 5003 x 2720 8.8 / 5.1, 20000 x 6144 24.3 / 17.7.
-constexpr int kMdMaxSteps = 16, kMdMaxBlocks = 4 * kMdMaxSteps;
-constexpr bool mdig_takes(int type, int nblk, bool gateup)
-{
-    if (nblk > kMdMaxBlocks)
-        return false;
-    if (type == kQ6_K || nblk > 16)
-        return true;
-    if (gateup)
-        return type == kQ5_K || nblk <= 14;
-    return type == kQ5_K && nblk <= 12;
 }
 template <int FMT, bool GATEUP, bool NORM, bool RESID>
 static void launch_mdig(const uint8_t *W, const uint8_t *W2, const float *x, float *y, int nblk, int outer,
@@ -1961,7 +1958,7 @@ static hipError_t launch_kwide(const void *w, const void *w2, const float *x, fl
         else
             hipLaunchKernelGGL((k_gemv_kpers<FMT, 1, GATEUP, false, NWV, NB>), dim3(grid), dim3(NWV * 64),
                                0, s, W, W2, x, y, outer, nblk, nw, eps, resid, epi);
-    } else if (!GATEUP && kwide_one_row(outer)) {
+    } else if (!GATEUP && kwide_one_row(outer, device_cus())) {
         // no more one-row workgroups than CUs: one row per wave, all of them
         // at once (2048 x 2048 2.8-3.1 us against 3.5-3.6 with two rows per
         // wave; 3072 x 3072 keeps two rows: 1.5 one-row workgroups per CU
@@ -2091,15 +2088,34 @@ bool gemv_norm_fusable(int type, int inner, int)
     return (type == kQ4_K || type == kQ5_K) && inner % 256 == 0 && inner / 256 <= 16;
 }
 
+template <int FMT>
+static void launch_norm(const uint8_t *W, const float *x, const float *nw, float eps, float *y, int nblk,
+                        int outer, hipStream_t s)
+{
+    constexpr int NWV = 8;
+    if (!norm_takes_wide(FMT, nblk, outer, device_cus()))
+        launch_mdig<FMT, false, true, false>(W, nullptr, x, y, nblk, outer, nw, eps, nullptr, 0, s);
+    else if (kwide_takes_kpers(nblk, outer))
+        hipLaunchKernelGGL((k_gemv_kpers_norm<FMT, 1, NWV, 2>),
+                           dim3(std::max(1, std::min(device_cus(), (outer + NWV - 1) / NWV))),
+                           dim3(NWV * 64), 0, s, W, x, y, outer, nblk, nw, eps);
+    else if (kwide_one_row(outer, device_cus()))
+        hipLaunchKernelGGL((k_gemv_kwide_norm<FMT, 1, NWV>), dim3((outer + NWV - 1) / NWV), dim3(NWV * 64),
+                           0, s, W, x, y, outer, nblk, nw, eps);
+    else
+        hipLaunchKernelGGL((k_gemv_kwide_norm<FMT, 2, NWV>), dim3((outer + 2 * NWV - 1) / (2 * NWV)),
+                           dim3(NWV * 64), 0, s, W, x, y, outer, nblk, nw, eps);
+}
+
 hipError_t launch_gemv_norm(int type, const void *w, const float *x, const float *nw, float eps,
                             float *y, int inner, int outer, hipStream_t s)
 {
     if (!gemv_norm_fusable(type, inner, outer))
         return hipErrorNotSupported;
     if (type == kQ4_K)
-        launch_mdig<kQ4_K, false, true, false>((const uint8_t *)w, nullptr, x, y, inner / 256, outer, nw, eps, nullptr, 0, s);
+        launch_norm<kQ4_K>((const uint8_t *)w, x, nw, eps, y, inner / 256, outer, s);
     else
-        launch_mdig<kQ5_K, false, true, false>((const uint8_t *)w, nullptr, x, y, inner / 256, outer, nw, eps, nullptr, 0, s);
+        launch_norm<kQ5_K>((const uint8_t *)w, x, nw, eps, y, inner / 256, outer, s);
     return hipGetLastError();
 }
 

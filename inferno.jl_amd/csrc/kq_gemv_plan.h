@@ -1,0 +1,65 @@
+// kq_gemv_plan.h -- which GEMV kernel takes a weight, by its format, row length
+// and (where no other launch has to give the same bits) row count.  Shared by
+// the launchers (kq_gemv.hip) and the CPU tests (tests/native).
+#pragma once
+
+#include "kq_common.h"
+
+namespace ihip {
+
+// Rows of at most 16 blocks with at least four 8-wave row groups per wave
+// over one workgroup per CU take the wide kernels' persistent form.
+inline bool kwide_takes_kpers(int nblk, int outer) { return nblk <= 16 && outer >= 4 * 8 * 256; }
+
+// No more one-row workgroups of 8 waves than CUs: one row per wave.
+inline bool kwide_one_row(int outer, int ncu) { return (outer + 7) / 8 <= ncu; }
+
+// Which rows k_gemv_mdig takes, by format, length and (gate/up) kind only: a
+// row's sum is the same whatever launch it is in, and the two kernels' differ.
+// The wide kernels spread a row's blocks over 16 lane positions, this one over
+// 4 a step, and it starts later (x goes through LDS twice).  So the wide
+// kernels keep the Q4_K / Q5_K rows that fill their lanes, and the short Q4_K
+// ones.  Measured on MI355X (us, graph replays over weights in HBM, wide / this):
+// Q4_K 2560 x 9728 8.6 / 6.3, 5120 x 5120 7.8 / 5.6, 4096 x 14336 10.6 / 9.9,
+// 4096 x 4096 4.1 / 4.6, 12288 x 4096 7.4 / 7.8, 3584 x 2560 3.45 / 3.73; Q5_K
+// 4096 x 2048 4.1 / 3.5, 9728 x 2560 7.4 / 6.5, 4096 x 4096 4.8 / 5.1; gate/up
+// Q4_K 6144 x 2048 7.2 / 5.7, 13824 x 5120 20.6 / 17.2, 10240 x 3584 11.0 / 10.5,
+// 12288 x 4096 12.8 / 13.0; Q5_K 9728 x 2560 12.3 / 9.7, 12288 x 4096 15.8 / 15.5.
+// Q6_K (streamed / this) 4096 x 12288 12.4 / 11.7, 2560 x 9728 12.1 / 7.9, 5120 x
+// 13824 26.9 / 15.9, 1024 x 4096 4.9 / 3.6, 12288 x 4096 11.2 / 11.5; Q8_0 5003 x
+// 2720 8.4 / 5.8, 2560 x 9728 11.2 / 8.3; IQ4_NL 5120 x 5120 10.7 / 6.8, 5003 x 2720
+// 8.8 / 5.1, 20000 x 6144 24.3 / 17.7.
+constexpr int kMdMaxSteps = 16, kMdMaxBlocks = 4 * kMdMaxSteps;
+constexpr bool mdig_takes(int type, int nblk, bool gateup)
+{
+    if (nblk > kMdMaxBlocks)
+        return false;
+    if (type == kQ6_K || nblk > 16)
+        return true;
+    if (gateup)
+        return type == kQ5_K || nblk <= 14;
+    return type == kQ5_K && nblk <= 12;
+}
+
+// The folded norm on a single weight of at most 16 blocks a row: whether the
+// wide kernels take it.  By row count too (no other call promises these bits):
+// the wide kernels are ahead while one round of their workgroups holds the rows
+// (one row per wave up to 8 rows per CU, two up to 16) or where they run
+// persistent, and behind where a second round starts; longer rows fill their
+// lanes better.  Measured on MI355X (us, graph replays over weights in HBM, wide
+// / k_gemv_mdig): Q4_K 1024 x 1024 3.00 / 3.02, 1024 x 1536 3.06 / 3.28, 1024 x 2560
+// 3.04 / 3.37, 2048 x 4096 4.08 / 4.47, 4096 x 2048 3.91 / 3.80, 3072 x 2304 3.78 /
+// 4.12, 4096 x 4096 4.49 / 5.14, 6144 x 4096 6.45 / 5.80, 12288 x 3072 6.71 / 6.55,
+// 12288 x 3328 6.81 / 7.47, 12288 x 4096 7.22 / 8.12; Q5_K 1024 x 2048 3.27 / 3.28,
+// 1024 x 2304 3.23 / 3.48, 2048 x 4096 4.42 / 4.56, 4096 x 3072 5.00 / 4.64, 4096 x
+// 3328 4.93 / 5.22, 6144 x 4096 7.27 / 6.38, 12288 x 3072 8.02 / 7.69, 12288 x 4096
+// 8.76 / 9.33.
+inline bool norm_takes_wide(int type, int nblk, int outer, int ncu)
+{
+    const bool one = kwide_one_row(outer, ncu), two = (outer + 15) / 16 <= ncu;
+    if (type == kQ4_K)
+        return one ? nblk > 4 : two ? nblk > 8 : nblk > 12 && kwide_takes_kpers(nblk, outer);
+    return one ? nblk > 8 : nblk > 12 && (two || kwide_takes_kpers(nblk, outer));
+}
+
+} // namespace ihip

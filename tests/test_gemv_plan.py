@@ -1,0 +1,65 @@
+"""Which kernel takes a GEMV (kq_gemv_plan.h, through tests/native/
+gemv_plan_check.hip, on the CPU): the faster one at shapes where the two were
+timed 4 % apart or more, and on the GPU both kernels' results at the edges of
+the rules.
+"""
+import ctypes as C
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+import oracle
+from inferno_hip import synth
+
+LIB = Path(__file__).resolve().parent / "native" / "_build" / "libsdig_check.so"
+Q4_K, Q5_K = synth.Q4_K, synth.Q5_K
+
+
+@pytest.fixture(scope="module")
+def plan():
+    if not LIB.exists():
+        from inferno_hip import build
+        build.build_checks()
+    return C.CDLL(str(LIB))
+
+
+# (type, rows, columns, wide us, k_gemv_mdig us): graph replays, weights in HBM
+NORM_TIMES = (
+    (Q4_K, 256, 1536, 2.71, 3.01), (Q4_K, 1024, 2560, 3.04, 3.37), (Q4_K, 1024, 4096, 3.41, 3.82),
+    (Q4_K, 2048, 2048, 3.05, 3.34), (Q4_K, 2048, 4096, 4.08, 4.47), (Q4_K, 2304, 1024, 3.59, 3.20),
+    (Q4_K, 3072, 2304, 3.78, 4.12), (Q4_K, 4096, 3328, 4.34, 4.99), (Q4_K, 4096, 4096, 4.49, 5.14),
+    (Q4_K, 6144, 1536, 5.17, 4.14), (Q4_K, 6144, 4096, 6.45, 5.80), (Q4_K, 8192, 3584, 5.51, 6.25),
+    (Q4_K, 12288, 2560, 6.68, 6.20), (Q4_K, 12288, 4096, 7.22, 8.12), (Q4_K, 16384, 1024, 7.46, 4.74),
+    (Q5_K, 512, 3584, 3.54, 3.88), (Q5_K, 1024, 1024, 3.30, 3.10), (Q5_K, 1536, 2560, 3.46, 3.79),
+    (Q5_K, 1024, 4096, 3.78, 4.01), (Q5_K, 2304, 3072, 4.60, 4.33), (Q5_K, 4096, 3328, 4.93, 5.22),
+    (Q5_K, 6144, 4096, 7.27, 6.38), (Q5_K, 8192, 2304, 6.33, 5.72), (Q5_K, 12288, 3584, 8.29, 8.79),
+    (Q5_K, 16384, 4096, 10.71, 11.44))
+
+
+@pytest.mark.parametrize("t,outer,inner,wide,mdig", NORM_TIMES)
+def test_folded_norm_takes_the_faster_kernel(plan, t, outer, inner, wide, mdig):
+    assert bool(plan.norm_takes_wide_of(t, inner // 256, outer, 256)) == (wide < mdig)
+
+
+# either side of every line of the rule: 8 and 16 rows per CU, the persistent
+# form's 8192 rows, 4, 8 and 12 blocks
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", (Q4_K, Q5_K))
+@pytest.mark.parametrize("outer,inner", [(1, 1280), (7, 2304), (2047, 1024), (2048, 2304), (2049, 2048), (2049, 2304), (4096, 3328),
+                                         (4095, 3072), (4097, 4096), (8191, 3584), (8192, 3328), (8197, 3072), (8203, 4096)])
+def test_folded_norm_rows(t, outer, inner):
+    import torch
+    from inferno_hip import device as D
+    print(f"folded norm type {t} {outer}x{inner}", flush=True)
+    rng = synth.rng_for(0x6E0 + outer)
+    w, x = synth.weight(rng, t, outer, inner), synth.activations(rng, inner)
+    nw = rng.uniform(0.5, 1.5, inner).astype(np.float32)
+    y = D.gemv_norm(D.DeviceWeight(torch.from_numpy(w).cuda(), t, inner, outer), torch.from_numpy(nw).cuda(), 1e-6,
+                    torch.from_numpy(x).cuda()).cpu().numpy()
+    n = oracle.rmsnorm_f64(x, nw, 1e-6)
+    # the row bound, and the fp32 norm's few roundings
+    tol = 1.01e-4 * oracle.row_norms(t, w, inner, outer) * np.linalg.norm(n)
+    ratio = np.max(np.abs(y.astype(np.float64) - oracle.gemv_f64(t, w, n, inner, outer)) / tol)
+    print(f"max err/tol = {ratio:.3e}", flush=True)
+    assert ratio <= 1.0
