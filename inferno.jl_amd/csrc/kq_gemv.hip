@@ -548,7 +548,6 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kwide_norm(const uint8_t *__r
 // exponent A, exponent B} of the pair, Q6_K 2^(e - 22) of its four groups, Q8_0
 // and IQ4_NL 2^(e - 22) of its two blocks.
 constexpr int kMdPlaneDw = 65 * 4, kMdStepDw = 4 * kMdPlaneDw;
-constexpr int kMdUnits = 512; // units (four rows x one step) per workgroup
 // Bytes of a block and blocks of a step; 16-byte pieces of a row's step (PHASED:
 // from the 16-byte unit its first byte lies in, at an even phase of 0 .. 14);
 // pieces between two rows in a ring slot (one more: 13 of 16 lanes' 128-bit reads then hit
@@ -1873,38 +1872,29 @@ int device_cus()
     return ncu;
 }
 
-// Rows of at most 16 steps of 1024 columns on the matrix cores: waves and ring
-// depth by the row's steps and the format's slot (3 to 5 KB a wave and slot,
-// beside 4 KB of digits a step).
-struct MdPlan {
-    int nw, d, maxs;
-};
-constexpr MdPlan mdig_plan(int type, int nstep)
-{
-    if (nstep <= 4)
-        return {8, 3, 4};
-    if (type == kQ6_K && nstep <= 12)
-        return {12, 2, 12};
-    return type == kQ6_K || type == kQ8_0 ? MdPlan{8, 2, 16} : MdPlan{12, 2, 16};
-}
 template <int FMT, bool GATEUP, bool NORM, bool RESID>
 static void launch_mdig(const uint8_t *W, const uint8_t *W2, const float *x, float *y, int nblk, int outer,
                         const float *nw, float eps, const float *resid, int epi, hipStream_t s)
 {
     constexpr int BPS = MdFmt<FMT>::BLOCKS;
     const int nstep = (nblk + BPS - 1) / BPS, ngroups = (outer + 3) / 4;
-    const int gpw = std::min((ngroups + device_cus() - 1) / device_cus(), kMdUnits / (nstep * (GATEUP ? 2 : 1)));
+    const int gpw = mdig_groups(outer, nstep * (GATEUP ? 2 : 1), device_cus());
     const dim3 grid((ngroups + gpw - 1) / gpw);
     const uint32_t inv = (65536u + nstep - 1) / nstep;
-    constexpr MdPlan p16 = mdig_plan(FMT, 16), p12 = mdig_plan(FMT, 12);
     auto launch = [&](auto nwv, auto d, auto maxs) {
         hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, nwv.value, d.value, maxs.value>), grid,
                            dim3(nwv.value * 64), 0, s, W, W2, x, y, outer, nblk, gpw, inv, nw, eps, resid, epi);
     };
     using std::integral_constant;
-    const MdPlan p = mdig_plan(FMT, nstep);
-    if (p.maxs == 4)
-        launch(integral_constant<int, 8>{}, integral_constant<int, 3>{}, integral_constant<int, 4>{});
+    constexpr MdPlan p16 = mdig_plan(FMT, 16, 1), p12 = mdig_plan(FMT, 12, 1), p4 = mdig_plan(FMT, 4, 1),
+                     p4m = mdig_plan(FMT, 4, kMdManyGroups);
+    const MdPlan p = mdig_plan(FMT, nstep, gpw);
+    if (p.maxs == 4 && p.nw == p4.nw)
+        launch(integral_constant<int, p4.nw>{}, integral_constant<int, p4.d>{}, integral_constant<int, 4>{});
+    else if (p.maxs == 4)
+        launch(integral_constant<int, p4m.nw>{}, integral_constant<int, p4m.d>{}, integral_constant<int, 4>{});
+    else if constexpr (NORM && !GATEUP)
+        return; // the folded norm of a single weight is of rows of four steps at most
     else if (p.maxs == p12.maxs)
         launch(integral_constant<int, p12.nw>{}, integral_constant<int, p12.d>{}, integral_constant<int, p12.maxs>{});
     else

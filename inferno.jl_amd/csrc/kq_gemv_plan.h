@@ -3,6 +3,8 @@
 // the launchers (kq_gemv.hip) and the CPU tests (tests/native).
 #pragma once
 
+#include <algorithm>
+
 #include "kq_common.h"
 
 namespace ihip {
@@ -26,7 +28,7 @@ inline bool kwide_one_row(int outer, int ncu) { return (outer + 7) / 8 <= ncu; }
 // Q4_K 6144 x 2048 7.2 / 5.7, 13824 x 5120 20.6 / 17.2, 10240 x 3584 11.0 / 10.5,
 // 12288 x 4096 12.8 / 13.0; Q5_K 9728 x 2560 12.3 / 9.7, 12288 x 4096 15.8 / 15.5.
 // Q6_K (streamed / this) 4096 x 12288 12.4 / 11.7, 2560 x 9728 12.1 / 7.9, 5120 x
-// 13824 26.9 / 15.9, 1024 x 4096 4.9 / 3.6, 12288 x 4096 11.2 / 11.5; Q8_0 5003 x
+// 13824 26.9 / 15.9, 1024 x 4096 4.9 / 3.6, 12288 x 4096 10.8 / 10.8; Q8_0 5003 x
 // 2720 8.4 / 5.8, 2560 x 9728 11.2 / 8.3; IQ4_NL 5120 x 5120 10.7 / 6.8, 5003 x 2720
 // 8.8 / 5.1, 20000 x 6144 24.3 / 17.7.
 constexpr int kMdMaxSteps = 16, kMdMaxBlocks = 4 * kMdMaxSteps;
@@ -39,6 +41,38 @@ constexpr bool mdig_takes(int type, int nblk, bool gateup)
     if (gateup)
         return type == kQ5_K || nblk <= 14;
     return type == kQ5_K && nblk <= 12;
+}
+
+// k_gemv_mdig's launch: groups of four rows per workgroup (`steps` of 1024
+// columns a group, gate and up together), one workgroup per CU where the units
+// it can hold allow.
+constexpr int kMdUnits = 512; // units (four rows x one step) per workgroup
+inline int mdig_groups(int outer, int steps, int ncu)
+{
+    const int ngroups = (outer + 3) / 4;
+    return std::min((ngroups + ncu - 1) / ncu, kMdUnits / steps);
+}
+// Waves, ring slots per wave and the most steps the instantiation takes, by the
+// row's steps and the format's slot (3 to 5 KB a wave and slot, beside 4 KB of
+// digits a step).  Q6_K rows of four steps, four groups or more per workgroup,
+// run on 12 waves: measured on MI355X (us, graph replays over weights in HBM, 8
+// waves x 3 slots / 12 x 2) 12288 x 4096 11.25 / 10.8 (the streamed kernel 10.8),
+// 4096 x 4096 6.2 / 5.5, 8192 x 3328 7.85 / 7.36; 10 and 11 waves x 3 slots 11.6
+// and 11.8 at 12288 x 4096, 16 x 2 11.5.  Fewer steps or groups leave the added
+// waves idle: 4096 x 2560 4.64 / 4.84, 2048 x 4096 4.33 / 4.63.
+struct MdPlan {
+    int nw, d, maxs;
+};
+constexpr int kMdManyGroups = 4;
+constexpr MdPlan mdig_plan(int type, int nstep, int groups)
+{
+    if (type == kQ6_K && nstep == 4 && groups >= kMdManyGroups)
+        return {12, 2, 4};
+    if (nstep <= 4)
+        return {8, 3, 4};
+    if (type == kQ6_K && nstep <= 12)
+        return {12, 2, 12};
+    return type == kQ6_K || type == kQ8_0 ? MdPlan{8, 2, 16} : MdPlan{12, 2, 16};
 }
 
 // The folded norm on a single weight of at most 16 blocks a row: whether the

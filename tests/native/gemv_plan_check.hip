@@ -7,3 +7,14 @@ extern "C" int norm_takes_wide_of(int type, int nblk, int outer, int ncu)
 {
     return ihip::norm_takes_wide(type, nblk, outer, ncu);
 }
+
+// waves, ring slots and steps of k_gemv_mdig's instantiation, and its groups
+extern "C" void mdig_plan_of(int type, int outer, int nstep, int ncu, int *out)
+{
+    const int groups = ihip::mdig_groups(outer, nstep, ncu);
+    const ihip::MdPlan p = ihip::mdig_plan(type, nstep, groups);
+    out[0] = p.nw;
+    out[1] = p.d;
+    out[2] = p.maxs;
+    out[3] = groups;
+}

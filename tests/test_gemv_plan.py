@@ -13,7 +13,7 @@ import oracle
 from inferno_hip import synth
 
 LIB = Path(__file__).resolve().parent / "native" / "_build" / "libsdig_check.so"
-Q4_K, Q5_K = synth.Q4_K, synth.Q5_K
+Q4_K, Q5_K, Q6_K = synth.Q4_K, synth.Q5_K, synth.Q6_K
 
 
 @pytest.fixture(scope="module")
@@ -63,3 +63,32 @@ def test_folded_norm_rows(t, outer, inner):
     ratio = np.max(np.abs(y.astype(np.float64) - oracle.gemv_f64(t, w, n, inner, outer)) / tol)
     print(f"max err/tol = {ratio:.3e}", flush=True)
     assert ratio <= 1.0
+
+
+# (rows, columns, waves): timed with 8 and with 12
+@pytest.mark.parametrize("outer,inner,waves", [(12288, 4096, 12), (4096, 4096, 12), (8192, 3328, 12), (32768, 3840, 12),
+                                               (2048, 4096, 8), (1024, 4096, 8), (4096, 2560, 8), (512, 3328, 8)])
+def test_q6_k_rows_of_four_steps(plan, outer, inner, waves):
+    out = (C.c_int * 4)()
+    plan.mdig_plan_of(Q6_K, outer, -(-inner // 1024), 256, out)
+    assert out[0] == waves
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("outer,inner", [(3073, 4096), (3072, 3328), (4099, 3840), (12301, 4096), (32771, 3328)])
+def test_q6_k_rows_on_twelve_waves(outer, inner):
+    """Against float64, and the bits of the same rows in a launch of 8 waves."""
+    import torch
+    from inferno_hip import device as D
+    print(f"Q6_K {outer}x{inner}", flush=True)
+    rng = synth.rng_for(0x6E1 + outer)
+    w, x = synth.weight(rng, Q6_K, outer, inner), synth.activations(rng, inner)
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    y = D.gemv(D.DeviceWeight(wd, Q6_K, inner, outer), xd).cpu().numpy()
+    tol = oracle.tolerance(oracle.row_norms(Q6_K, w, inner, outer), x)
+    ratio = np.max(np.abs(y.astype(np.float64) - oracle.gemv_f64(Q6_K, w, x, inner, outer)) / tol)
+    print(f"max err/tol = {ratio:.3e}", flush=True)
+    assert ratio <= 1.0
+    k = 1021
+    few = D.gemv(D.DeviceWeight(wd[: k * (len(w) // outer)], Q6_K, inner, k), xd).cpu().numpy()
+    assert np.array_equal(few.view(np.uint32), y[:k].view(np.uint32))
