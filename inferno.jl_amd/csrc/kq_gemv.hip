@@ -1929,7 +1929,7 @@ static hipError_t launch_kwide(const void *w, const void *w2, const float *x, fl
     const bool ext = GATEUP ? nw != nullptr : resid != nullptr;
     const uint8_t *W = (const uint8_t *)w, *W2 = (const uint8_t *)w2;
     if constexpr (FMT == kQ4_K || FMT == kQ5_K) {
-        if (mdig_takes(FMT, nblk, GATEUP)) {
+        if (GATEUP ? !gate_up_takes_wide(FMT, nblk, outer, device_cus()) : mdig_takes(FMT, nblk, false)) {
             if (ext)
                 launch_mdig<FMT, GATEUP, GATEUP, !GATEUP>(W, W2, x, y, nblk, outer, nw, eps, resid, epi, s);
             else
@@ -1937,7 +1937,7 @@ static hipError_t launch_kwide(const void *w, const void *w2, const float *x, fl
             return hipGetLastError();
         }
     }
-    constexpr bool kPers = !(GATEUP && FMT == kQ5_K); // those rows are all taken above
+    constexpr bool kPers = !(GATEUP && FMT == kQ5_K); // so many of those rows are taken above
     if (kPers && kwide_takes_kpers(nblk, outer)) {
         const int grid = std::max(1, std::min(device_cus(), (outer + NWV - 1) / NWV));
         if constexpr (!kPers)

@@ -96,4 +96,22 @@ inline bool norm_takes_wide(int type, int nblk, int outer, int ncu)
     return one ? nblk > 8 : nblk > 12 && (two || kwide_takes_kpers(nblk, outer));
 }
 
+// Gate/up (one wide workgroup has eight rows of each): whether the wide kernels
+// take it although mdig_takes does, by row count as above: while one round of
+// their workgroups holds the rows and, but for the longest Q4_K ones, a
+// workgroup of k_gemv_mdig has more than one group of four.  Measured likewise:
+// Q4_K 1536 x 2048 3.41 / 3.42, 1024 x 2816 3.69 / 3.45, 1536 x 2304 3.63 / 3.91, 2048 x
+// 2816 3.82 / 4.02, 1024 x 3328 3.61 / 3.95, 1536 x 3584 3.90 / 4.62, 2304 x 2560 5.07 /
+// 4.53, 4096 x 3584 5.93 / 6.05; Q5_K 1024 x 3584 4.37 / 4.09, 1536 x 3328 4.49 / 4.91,
+// 2048 x 4096 5.05 / 5.27, 1536 x 3072 4.50 / 4.26, 2304 x 4096 6.84 / 6.02.
+inline bool gate_up_takes_wide(int type, int nblk, int outer, int ncu)
+{
+    if (!mdig_takes(type, nblk, true))
+        return true;
+    if (nblk > 16 || !kwide_one_row(outer, ncu))
+        return false;
+    const bool groups = outer > 4 * ncu;
+    return type == kQ4_K ? nblk > 12 || (nblk > 8 && groups) : nblk > 12 && groups;
+}
+
 } // namespace ihip

@@ -18,3 +18,8 @@ extern "C" void mdig_plan_of(int type, int outer, int nstep, int ncu, int *out)
     out[2] = p.maxs;
     out[3] = groups;
 }
+
+extern "C" int gate_up_takes_wide_of(int type, int nblk, int outer, int ncu)
+{
+    return ihip::gate_up_takes_wide(type, nblk, outer, ncu);
+}

@@ -92,3 +92,49 @@ def test_q6_k_rows_on_twelve_waves(outer, inner):
     k = 1021
     few = D.gemv(D.DeviceWeight(wd[: k * (len(w) // outer)], Q6_K, inner, k), xd).cpu().numpy()
     assert np.array_equal(few.view(np.uint32), y[:k].view(np.uint32))
+
+
+GATE_UP_TIMES = (
+    (Q4_K, 1024, 3328, 3.61, 3.95), (Q4_K, 1024, 2048, 3.46, 3.25), (Q4_K, 1024, 2816, 3.69, 3.45), (Q4_K, 1536, 2304, 3.61, 3.91), (Q4_K, 2048, 2816, 3.83, 4.14),
+    (Q4_K, 1536, 3584, 3.90, 4.65), (Q4_K, 2304, 2560, 5.09, 4.56), (Q4_K, 9728, 3584, 10.62, 9.88), (Q4_K, 1408, 5120, 5.38, 4.86),
+    (Q5_K, 512, 2560, 4.01, 3.70), (Q5_K, 1024, 3584, 4.40, 4.01), (Q5_K, 1536, 3328, 4.54, 4.85), (Q5_K, 2048, 3584, 4.85, 5.11),
+    (Q5_K, 1408, 4096, 4.64, 4.83), (Q5_K, 1536, 3072, 4.52, 4.31), (Q5_K, 2304, 4096, 6.84, 5.98), (Q5_K, 14336, 4096, 18.28, 17.58))
+
+
+@pytest.mark.parametrize("t,outer,inner,wide,mdig", GATE_UP_TIMES)
+def test_gate_up_takes_the_faster_kernel(plan, t, outer, inner, wide, mdig):
+    assert bool(plan.gate_up_takes_wide_of(t, inner // 256, outer, 256)) == (wide < mdig)
+
+
+# either side of every line of the rule, with the folded norm and without
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", (Q4_K, Q5_K))
+@pytest.mark.parametrize("outer,inner", [(1, 2304), (2047, 2048), (2048, 2304), (2049, 2304), (1024, 2560), (1025, 2560), (1024, 3328), (1025, 3328),
+                                         (2041, 4096), (2049, 3584), (1025, 3072)])
+def test_gate_up_rows(t, outer, inner):
+    import torch
+    from inferno_hip import device as D
+    print(f"gate/up type {t} {outer}x{inner}", flush=True)
+    rng = synth.rng_for(0x6E2 + outer + inner)
+    ws = [synth.weight(rng, t, outer, inner) for _ in range(2)]
+    x, nw = synth.activations(rng, inner), rng.uniform(0.5, 1.5, inner).astype(np.float32)
+    dws = [D.DeviceWeight(torch.from_numpy(w).cuda(), t, inner, outer) for w in ws]
+    xd = torch.from_numpy(x).cuda()
+    mats = [oracle.dequant(t, w, outer * inner).reshape(outer, inner).astype(np.float64) for w in ws]
+
+    def check(h, n, what):
+        g, u = (m @ n for m in mats)
+        ng, nu = (np.linalg.norm(m, axis=1) * 1.01e-4 * np.linalg.norm(n) for m in mats)
+        with np.errstate(over="ignore"):
+            s = 1 / (1 + np.exp(-g))
+        # silu's slope is below 1.1; fp32 roundings of the last two products
+        tol = 1.1 * ng * (np.abs(u) + nu) + np.abs(g * s) * nu + 1e-6 * np.abs(g * s * u)
+        assert np.all(np.abs(h - g * s * u) <= tol), what
+
+    check(D.gate_up_swiglu(*dws, xd).cpu().numpy().astype(np.float64), x.astype(np.float64), "plain")
+    wd = synth.weight(rng, Q4_K, inner, 256 * -(-outer // 256))
+    if outer % 256 == 0:  # the norm's form is the FFN block's
+        h = torch.empty(outer + inner, device="cuda")
+        D.ffn_block(*dws, D.DeviceWeight(torch.from_numpy(wd).cuda(), Q4_K, outer, inner), torch.from_numpy(nw).cuda(),
+                    1e-6, xd, h)
+        check(h[:outer].cpu().numpy().astype(np.float64), oracle.rmsnorm_f64(x, nw, 1e-6), "norm")
