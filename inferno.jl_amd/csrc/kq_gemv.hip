@@ -2053,18 +2053,13 @@ hipError_t launch_gemv(int type, const void *w, const float *x, float *y, int in
         }
         return launch_sdig<kQ6_K, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     case kQ8_0:
-        // rows of one pass (at most 4096 columns in whole 256-column units) on
-        // the wide lane layout: 4096 x 4096 5.9 us against k_gemv_mdig's 6.1,
-        // 2048 x 2048 3.0 / 3.3, 9728 x 2560 8.0 / 7.6
-        if (inner % 256 == 0 && inner <= 4096)
+        if (b32_takes_wide(type, inner))
             return launch_kwide<kQ8_0, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi);
         if (inner <= 1024 * kMdMaxSteps)
             return launch_mdig_b32<kQ8_0>(w, x, y, inner, outer, resid, epi, s);
         return launch_sdig<kQ8_0, false>(w, x, y, inner, outer, nullptr, s, resid, epi);
     case kIQ4_NL:
-        // the wide lane layout where it is all but full (4096 x 4096 5.0 us
-        // against k_gemv_mdig's 5.4), and for rows too long for the others
-        if (inner % 256 == 0 && ((inner > 3584 && inner <= 4096) || inner > 1024 * kMdMaxSteps))
+        if (b32_takes_wide(type, inner))
             return launch_kwide<kIQ4_NL, false>(w, nullptr, x, y, inner, outer, s, nullptr, 0.0f, resid, epi);
         if (inner <= 1024 * kMdMaxSteps)
             return launch_mdig_b32<kIQ4_NL>(w, x, y, inner, outer, resid, epi, s);

@@ -43,6 +43,22 @@ constexpr bool mdig_takes(int type, int nblk, bool gateup)
     return type == kQ5_K && nblk <= 12;
 }
 
+// Q8_0 and IQ4_NL rows of whole 256-column units on the wide lane layout, by
+// length only (as mdig_takes).  Measured on MI355X (us, graph replays over weights
+// in HBM, wide / k_gemv_mdig): Q8_0 4096 x 4096 5.9 / 6.1, 2048 x 2048 3.0 / 3.3, 9728 x
+// 2560 8.0 / 7.6 (the one length lost); IQ4_NL 4096 x 4096 5.0 / 5.4, 1024 x 3584 3.18 /
+// 3.52, 4096 x 3328 4.81 / 5.21, 12288 x 3328 9.80 / 9.37, and where k_gemv_mdig has it
+// 1024 x 2560 3.21 / 3.35, 2048 x 3072 3.64 / 3.76, 4096 x 3072 4.72 / 4.44, 12288 x 2560
+// 9.50 / 7.54.  IQ4_NL rows too long for the others too (4096 x 20480).
+inline bool b32_takes_wide(int type, int inner)
+{
+    if (inner % 256)
+        return false;
+    if (type == kQ8_0)
+        return inner <= 4096;
+    return (inner > 3072 && inner <= 4096) || inner > 1024 * kMdMaxSteps;
+}
+
 // k_gemv_mdig's launch: groups of four rows per workgroup (`steps` of 1024
 // columns a group, gate and up together), one workgroup per CU where the units
 // it can hold allow.

@@ -23,3 +23,8 @@ extern "C" int gate_up_takes_wide_of(int type, int nblk, int outer, int ncu)
 {
     return ihip::gate_up_takes_wide(type, nblk, outer, ncu);
 }
+
+extern "C" int b32_takes_wide_of(int type, int inner)
+{
+    return ihip::b32_takes_wide(type, inner);
+}

@@ -138,3 +138,25 @@ def test_gate_up_rows(t, outer, inner):
         D.ffn_block(*dws, D.DeviceWeight(torch.from_numpy(wd).cuda(), Q4_K, outer, inner), torch.from_numpy(nw).cuda(),
                     1e-6, xd, h)
         check(h[:outer].cpu().numpy().astype(np.float64), oracle.rmsnorm_f64(x, nw, 1e-6), "norm")
+
+
+# by length only: the rows of an engine's projections decide
+@pytest.mark.parametrize("inner,wide,mdig", [(3328, 4.81, 5.21), (3584, 4.86, 5.25), (4096, 5.0, 5.4), (3072, 4.72, 4.44),
+                                             (2560, 4.61, 4.34), (5120, 7.39, 5.62)])
+def test_iq4_nl_of_4096_rows_takes_the_faster_kernel(plan, inner, wide, mdig):
+    assert bool(plan.b32_takes_wide_of(synth.IQ4_NL, inner)) == (wide < mdig)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("outer,inner", [(1, 3328), (2049, 3328), (515, 3584), (8195, 3328), (9, 3360), (30, 3072)])
+def test_iq4_nl_rows(outer, inner):
+    import torch
+    from inferno_hip import device as D
+    print(f"IQ4_NL {outer}x{inner}", flush=True)
+    rng = synth.rng_for(0x6E3 + outer)
+    w, x = synth.weight(rng, synth.IQ4_NL, outer, inner), synth.activations(rng, inner)
+    y = D.gemv(D.DeviceWeight(torch.from_numpy(w).cuda(), synth.IQ4_NL, inner, outer), torch.from_numpy(x).cuda()).cpu().numpy()
+    tol = oracle.tolerance(oracle.row_norms(synth.IQ4_NL, w, inner, outer), x)
+    ratio = np.max(np.abs(y.astype(np.float64) - oracle.gemv_f64(synth.IQ4_NL, w, x, inner, outer)) / tol)
+    print(f"max err/tol = {ratio:.3e}", flush=True)
+    assert ratio <= 1.0
