@@ -14,8 +14,6 @@
 // lanes run the eight fp32 chains in block order and lane 0 adds them up in
 // the horizontal-sum order.  Q4_K keeps four more chains for the dmin terms
 // (accm, :262-270), Q5_K one (summs, :352-360).
-#include <algorithm>
-
 #include "kq_common.h"
 #include "kq_launch.h"
 
@@ -448,23 +446,24 @@ static bool q8kw_ok(int type, const void *w, int nb)
            ((uintptr_t)w & 15u) == 0;
 }
 
-// Q6_K rows of at most kQ86MaxBlocks blocks in the same numerics, streamed: one
-// row per wave at a time, eight blocks an item (1680 bytes from the 16-byte
-// unit of their first byte, at the row's even phase), through a private ring
-// of D slots of LDS filled by direct-to-LDS 128-bit copies.  Lane (block s,
-// integer lane t) forms sumi[t] of its block as q8k_item does, from dword reads
-// of LDS.  16 waves share x as Q8_K blocks, quantized by the workgroup itself
-// (QX, through the ring's last slots) or read from q8; the grid is one
-// workgroup per CU and walks the rows, TW waves to a row (wave rank of a team
-// takes items rank, rank + TW, ..), as q86_team picks.  The row's terms wait in
-// LDS for its fp32 chains, eight lanes, block by block in order.
+// Q6_K rows of at most kQ86MaxBlocks blocks in the same numerics, streamed: a
+// row for each team of TW waves, eight blocks an item (1680 bytes from the
+// 16-byte unit of their first byte, at the row's even phase), wave `rank` of the
+// team taking items rank, rank + TW, .., each in a slot of LDS of its own filled
+// by direct-to-LDS 128-bit copies.  Lane (block s, integer lane t) forms
+// sumi[t] of its block as q8k_item does, from dword reads of LDS.  16 waves
+// share x as Q8_K blocks, quantized by the workgroup itself (QX, through the
+// slots past the first) or read from q8; the grid has a team for every row
+// (q86_team).  The row's terms meet in LDS for its fp32 chains, eight lanes,
+// block by block in order.
 //
 // k_gemv_q8k reads a block as 2-byte pieces straight from memory, eight lanes
 // a block (ten cache-line lookups per 42 bytes), and quantizes x in a launch
-// of its own.  Measured on MI355X (us, quantizing included, streamed launches,
-// that / this): 512 x 1024 8.2 / 5.2, 1024 x 4096 8.2 / 5.2, 777 x 5120 8.3 / 5.7,
-// 4096 x 4096 8.0 / 6.7; with the weights in HBM 4096 x 4096 9.2 / 7.2.
-constexpr int kQ86MaxBlocks = 24, kQ86Waves = 16, kQ86Depth = 3, kQ86Slot = 2048;
+// of its own.  Measured on MI355X (us, quantizing included, graph replays over
+// weights in HBM, that / this): 256 x 256 4.30 / 3.18, 512 x 1024 4.64 / 3.50, 1024 x
+// 4096 6.26 / 5.17, 1024 x 5120 7.31 / 5.66, 4096 x 4096 8.83 / 6.81 (held in the
+// memory-side cache 9.07 / 7.46).
+constexpr int kQ86MaxBlocks = 24, kQ86Waves = 16, kQ86Items = (kQ86MaxBlocks + 7) / 8, kQ86Slot = 2048;
 template <bool QX, int TW>
 __global__ __launch_bounds__(64 * kQ86Waves) void k_gemv_q8k6(const uint8_t *__restrict__ W,
                                                               const float *__restrict__ x,
@@ -472,25 +471,22 @@ __global__ __launch_bounds__(64 * kQ86Waves) void k_gemv_q8k6(const uint8_t *__r
                                                               uint8_t *__restrict__ q8out,
                                                               float *__restrict__ out, int outer, int nb)
 {
-    constexpr int NWV = kQ86Waves, D = kQ86Depth, SLOT = kQ86Slot, MB = kQ86MaxBlocks;
-    __shared__ __attribute__((aligned(16))) uint8_t ring[NWV * D * SLOT];
+    constexpr int NWV = kQ86Waves, SLOT = kQ86Slot, MB = kQ86MaxBlocks, TEAMS = NWV / TW;
+    __shared__ __attribute__((aligned(16))) uint8_t slots[NWV * kQ86Items * SLOT];
     __shared__ __attribute__((aligned(16))) uint32_t s_qs[MB * 64];
     __shared__ float s_yd[MB];
-    // float(sumi[0..7]), d; a team of several waves uses its places in turn
-    __shared__ float s_st[NWV][MB][9];
-    static_assert((MB + NWV - 1) / NWV * 1024 <= (D - 1) * SLOT, "a wave's blocks of x fit its last slots");
+    __shared__ float s_st[TEAMS][MB][9]; // float(sumi[0..7]), d
+    static_assert((MB + NWV - 1) / NWV * 1024 <= (kQ86Items - 1) * SLOT, "a wave's blocks of x fit its last slots");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int s = lane >> 3, t = lane & 7;
     const uint32_t row_bytes = (uint32_t)nb * 210u;
-    constexpr int TEAMS = NWV / TW;
     const int team = w / TW, rank = w % TW;
-    const int ni = (nb + 7) >> 3, stride = (int)gridDim.x * TEAMS, row0 = (int)blockIdx.x * TEAMS;
-    const int first = row0 + team, rounds = (outer - row0 - 1) / stride + 1; // the workgroup's
-    const int nrows = first < outer ? (outer - first - 1) / stride + 1 : 0;
-    const int n = nrows * ((ni - rank + TW - 1) / TW); // this wave's items
-    uint8_t *const mine = ring + w * (D * SLOT);
+    const int row = (int)blockIdx.x * TEAMS + team;
+    const int ni = (nb + 7) >> 3;
+    const int n = row < outer ? (ni - rank + TW - 1) / TW : 0; // this wave's items, at most kQ86Items
+    uint8_t *const mine = slots + w * (kQ86Items * SLOT);
     const uint32_t mine_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mine;
 
     // x of this wave's blocks w, w + NWV, .. into the slots past the first
@@ -498,24 +494,18 @@ __global__ __launch_bounds__(64 * kQ86Waves) void k_gemv_q8k6(const uint8_t *__r
         for (int k = 0; w + NWV * k < nb; ++k)
             lds_copy16_at(x + (size_t)(w + NWV * k) * 256, 16u * lane, mine_lds + SLOT + 1024 * k);
     }
-    int ir = first, ii = rank, islot = 0; // the next item to copy: row, item of it, slot
-    auto issue = [&]() {
-        const uint8_t *base = W + (size_t)ir * row_bytes + (size_t)ii * 1680u;
+    auto issue = [&](int i) {
+        const int it = rank + TW * i;
+        const uint8_t *base = W + (size_t)row * row_bytes + (size_t)it * 1680u;
         const uint32_t phase = (uint32_t)(uintptr_t)base & 15u;
         // pieces past the item's last byte: the last one again
-        const uint32_t last = (phase + (uint32_t)min(8, nb - 8 * ii) * 210u - 1u) & ~15u;
+        const uint32_t last = (phase + (uint32_t)min(8, nb - 8 * it) * 210u - 1u) & ~15u;
         base -= phase;
-        lds_copy16_at(base, min(16u * lane, last), mine_lds + SLOT * islot);
-        lds_copy16_at(base, min(1024u + 16u * lane, last), mine_lds + SLOT * islot + 1024);
-        islot = islot == D - 1 ? 0 : islot + 1;
-        ii += TW;
-        if (ii >= ni) {
-            ii = rank;
-            ir += stride;
-        }
+        lds_copy16_at(base, min(16u * lane, last), mine_lds + SLOT * i);
+        lds_copy16_at(base, min(1024u + 16u * lane, last), mine_lds + SLOT * i + 1024);
     };
     if (n > 0)
-        issue();
+        issue(0);
     if constexpr (QX) {
         if (n > 0)
             __builtin_amdgcn_s_waitcnt(2 | 0x0f70);
@@ -544,97 +534,90 @@ __global__ __launch_bounds__(64 * kQ86Waves) void k_gemv_q8k6(const uint8_t *__r
     }
     __builtin_amdgcn_s_waitcnt(0xc07f); // the raw values are read, the blocks written
     asm volatile("" ::: "memory");
-    for (int i = 1; i < min(n, D); ++i)
-        issue();
+    for (int i = 1; i < n; ++i)
+        issue(i);
     lds_barrier();
 
-    int slot = 0, i = 0;
-    for (int round = 0; round < rounds; ++round) {
-        const int row = first + round * stride;
-        float (*const st)[9] = s_st[TW == 1 ? w : team * TW + (round & 1)];
-        for (int it = row < outer ? rank : ni; it < ni; it += TW, ++i) {
-            // stores to q8out count too: then this waits for more than it needs
-            const int later = min(D, n - i) - 1;
-            if (later >= 2)
-                __builtin_amdgcn_s_waitcnt(4 | 0x0f70);
-            else if (later == 1)
-                __builtin_amdgcn_s_waitcnt(2 | 0x0f70);
-            else
-                __builtin_amdgcn_s_waitcnt(0x0f70);
-            asm volatile("" ::: "memory");
-            const int blk = 8 * it + s;
-            const uint32_t at = (uint32_t)(uintptr_t)W + (uint32_t)row * row_bytes; // phase of the row (1680 is 105 units)
-            const uint32_t byte = (at & 15u) + 210u * (uint32_t)s;
-            const uint32_t *p = reinterpret_cast<const uint32_t *>(mine + SLOT * slot + (byte & ~3u));
-            const uint32_t sh = byte & 2u;
-            auto dword = [&](int k) { return __builtin_amdgcn_alignbyte(p[k + 1], p[k], sh); };
-            uint32_t sc[4];
+    float (*const st)[9] = s_st[team];
+    for (int i = 0; i < n; ++i) {
+        // stores to q8out count too: then this waits for more than it needs
+        const int later = n - 1 - i;
+        if (later >= 2)
+            __builtin_amdgcn_s_waitcnt(4 | 0x0f70);
+        else if (later == 1)
+            __builtin_amdgcn_s_waitcnt(2 | 0x0f70);
+        else
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+        asm volatile("" ::: "memory");
+        const int blk = 8 * (rank + TW * i) + s;
+        const uint32_t at = (uint32_t)(uintptr_t)W + (uint32_t)row * row_bytes; // phase of the row (1680 is 105 units)
+        const uint32_t byte = (at & 15u) + 210u * (uint32_t)s;
+        const uint32_t *p = reinterpret_cast<const uint32_t *>(mine + SLOT * i + (byte & ~3u));
+        const uint32_t sh = byte & 2u;
+        auto dword = [&](int k) { return __builtin_amdgcn_alignbyte(p[k + 1], p[k], sh); };
+        uint32_t sc[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) sc[k] = dword(48 + k) >> (t >= 4 ? 8 : 0);
-            const uint32_t dw = p[52];
-            const uint32_t *qx = s_qs + min(blk, nb - 1) * 64 + t;
-            int sumi = 0;
+        for (int k = 0; k < 4; ++k) sc[k] = dword(48 + k) >> (t >= 4 ? 8 : 0);
+        const uint32_t dw = p[52];
+        const uint32_t *qx = s_qs + min(blk, nb - 1) * 64 + t;
+        int sumi = 0;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint32_t hq = dword(32 + 8 * j + t);
-                const uint32_t lb[2] = {dword(16 * j + t), dword(16 * j + 8 + t)};
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t hq = dword(32 + 8 * j + t);
+            const uint32_t lb[2] = {dword(16 * j + t), dword(16 * j + 8 + t)};
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t lo = k < 2 ? (lb[k & 1] & 0x0f0f0f0fu) : ((lb[k & 1] >> 4) & 0x0f0f0f0fu);
-                    const uint32_t q = lo | (((hq >> (2 * k)) & 0x03030303u) << 4);
-                    // q - 32 as a signed byte: (q + 96) with the top bit flipped
-                    const int pr = sdot4((q + 0x60606060u) ^ 0x80808080u, (int)qx[32 * j + 8 * k], 0);
-                    sumi += (int)(int8_t)(sc[2 * j + (k >> 1)] >> (16 * (k & 1))) * pr;
-                }
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t lo = k < 2 ? (lb[k & 1] & 0x0f0f0f0fu) : ((lb[k & 1] >> 4) & 0x0f0f0f0fu);
+                const uint32_t q = lo | (((hq >> (2 * k)) & 0x03030303u) << 4);
+                // q - 32 as a signed byte: (q + 96) with the top bit flipped
+                const int pr = sdot4((q + 0x60606060u) ^ 0x80808080u, (int)qx[32 * j + 8 * k], 0);
+                sumi += (int)(int8_t)(sc[2 * j + (k >> 1)] >> (16 * (k & 1))) * pr;
             }
-            if (blk < nb) {
-                st[blk][t] = (float)sumi;
-                if (t == 0)
-                    st[blk][8] = s_yd[blk] * h2f(sh ? dw >> 16 : dw & 0xffffu);
-            }
-            __builtin_amdgcn_s_waitcnt(0xc07f); // the slot is read, the terms written
-            asm volatile("" ::: "memory");
-            if (i + D < n)
-                issue();
-            slot = slot == D - 1 ? 0 : slot + 1;
         }
-        if constexpr (TW > 1)
-            lds_barrier(); // every wave's terms of the round; the next round's go to the team's other place
-        if (rank == 0 && row < outer) { // the row's chains
-            float acc = 0.0f;
-            for (int b0 = 0; b0 < nb; b0 += 8) {
-                float dv[8], sv[8];
-#pragma unroll
-                for (int b = 0; b < 8; ++b) {
-                    dv[b] = st[min(b0 + b, nb - 1)][8];
-                    sv[b] = st[min(b0 + b, nb - 1)][t];
-                }
-#pragma unroll
-                for (int b = 0; b < 8; ++b)
-                    if (b0 + b < nb)
-                        acc = fmaf(dv[b], sv[b], acc);
-            }
-            __builtin_amdgcn_s_waitcnt(0xc07f); // read before later terms are written
-            asm volatile("" ::: "memory");
-            float a[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) a[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), k));
-            // AVX2 horizontal sums (quant_kernels.c:91-98)
-            const float s0 = a[0] + a[4], s1 = a[1] + a[5], s2 = a[2] + a[6], s3 = a[3] + a[7];
-            if (lane == 0)
-                out[row] = (s0 + s2) + (s1 + s3);
+        if (blk < nb) {
+            st[blk][t] = (float)sumi;
+            if (t == 0)
+                st[blk][8] = s_yd[blk] * h2f(sh ? dw >> 16 : dw & 0xffffu);
         }
     }
+    __builtin_amdgcn_s_waitcnt(0xc07f); // the terms are written
+    asm volatile("" ::: "memory");
+    if constexpr (TW > 1)
+        lds_barrier(); // by every wave of the team
+    if (rank != 0 || row >= outer)
+        return; // wave-uniform
+    float acc = 0.0f; // the row's chains
+    for (int b0 = 0; b0 < nb; b0 += 8) {
+        float dv[8], sv[8];
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            dv[b] = st[min(b0 + b, nb - 1)][8];
+            sv[b] = st[min(b0 + b, nb - 1)][t];
+        }
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+            if (b0 + b < nb)
+                acc = fmaf(dv[b], sv[b], acc);
+    }
+    float a[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), k));
+    // AVX2 horizontal sums (quant_kernels.c:91-98)
+    const float s0 = a[0] + a[4], s1 = a[1] + a[5], s2 = a[2] + a[6], s3 = a[3] + a[7];
+    if (lane == 0)
+        out[row] = (s0 + s2) + (s1 + s3);
 }
 
-// Waves to a row: as many (of 1, 2, 4) as one round of the chip's waves has for
-// every row and the row has items for.  Measured on MI355X (us, quantizing
-// included, graph replays, 1 wave a row / as chosen): 777 x 5120 7.6 / 5.7, 1024
-// x 4096 6.1 / 5.4.
+// Waves to a row: as many of 1, 2 (from 5 blocks on) and 4 (from 17) as one
+// round of the chip's waves has for every row.  (Two waves of a row of at most
+// eight blocks are one at work, in twice the workgroups.)  Measured on MI355X
+// (us, quantizing included, graph replays over weights in HBM, fewer / more
+// waves): 256 x 256 3.18 / 3.72, 256 x 512 3.21 / 3.34, 512 x 1024 3.50 / 3.56; 512 x 1280
+// 3.56 / 3.68, 512 x 2048 3.77 / 3.71; 512 x 5120 6.29 / 5.20, 1024 x 6144 6.75 / 5.76.
 static int q86_team(int nb, int outer, int ncu)
 {
     int tw = 1;
-    while (tw < 4 && (int64_t)outer * 2 * tw <= (int64_t)ncu * kQ86Waves && 2 * tw <= (nb + 7) / 8 + 1)
+    while (tw < 4 && (int64_t)outer * 2 * tw <= (int64_t)ncu * kQ86Waves && nb > (tw == 1 ? 4 : 16))
         tw *= 2;
     return tw;
 }
@@ -644,7 +627,7 @@ static hipError_t launch_q8k6(const void *w, const float *x, const void *q8, voi
                               int outer, hipStream_t s)
 {
     const int tw = q86_team(nb, outer, device_cus()), teams = kQ86Waves / tw;
-    const dim3 grid((unsigned)std::min((outer + teams - 1) / teams, device_cus())), block(64 * kQ86Waves);
+    const dim3 grid((unsigned)((outer + teams - 1) / teams)), block(64 * kQ86Waves);
     const uint8_t *W = (const uint8_t *)w, *Q = (const uint8_t *)q8;
     if (tw == 1)
         hipLaunchKernelGGL((k_gemv_q8k6<QX, 1>), grid, block, 0, s, W, x, Q, (uint8_t *)q8out, out, outer, nb);
@@ -656,10 +639,11 @@ static hipError_t launch_q8k6(const void *w, const float *x, const void *q8, voi
 }
 
 // Rows of up to kQ86MaxBlocks blocks of a 16-byte aligned W, one round of the
-// chip's waves at most.  There the launch and the latency are the cost.  Past
-// it k_gemv_q8k is as fast or faster on weights that the memory-side cache
-// holds (us there, streamed launches, that / this: 4096 x 12288 13.6 / 13.7, 2560
-// x 9728 10.4 / 11.4, 14336 x 4096 14.3 / 16.3).
+// chip's waves at most: there the launch and the latency are the cost.  Forms of
+// this kernel for longer rows and more of them were slower than k_gemv_q8k on
+// weights that the memory-side cache holds (us there, streamed launches, that /
+// this: 4096 x 12288 13.6 / 13.7, 2560 x 9728 10.4 / 11.4, 14336 x 4096 14.3 / 16.3) and
+// 10-24 % faster on weights in HBM; the line follows the first.
 static bool q8k6_ok(int type, const void *w, int nb, int outer)
 {
     return type == kQ6_K && nb >= 1 && nb <= kQ86MaxBlocks && ((uintptr_t)w & 15u) == 0 &&
