@@ -514,7 +514,7 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kwide_norm(const uint8_t *__r
 }
 
 // ------------------------------------------------------------------------
-// Q4_K / Q5_K on the matrix cores (k_gemv_mdig)
+// Four rows at a time on the matrix cores (k_gemv_mdig), every format
 // ------------------------------------------------------------------------
 
 // v_mfma_i32_4x4x4_16b_i8 forms sixteen independent 4 x 4 products over four
@@ -1666,7 +1666,7 @@ __device__ __forceinline__ void sxd_load(SXD &X, const uint32_t (*d)[64][4], int
 
 // The walk itself over LDS the caller declares (ring: NW * D * sdig_slot
 // bytes, 16-byte aligned; digs: the staged digits of sdig_share_cap(NW)
-// segments unless ARGMAX; part: kSdigMaxRows x NW; wkey / wflag: NW each).
+// segments (ARGMAX); part: kSdigMaxRows x NW; wkey / wflag: NW each).
 // PH: rows that are not 16-byte multiples (segments at a byte phase in their
 // slots); without it every phase is 0 and the lane offsets are fixed.
 template <int FMT, int NW, int D, bool ARGMAX, bool RESID, bool PH>
@@ -1688,7 +1688,8 @@ __device__ __forceinline__ void sdig_run(const uint8_t *__restrict__ W, const fl
                   "segment geometry");
     static_assert(SLOT >= F::SEG_BYTES + 16, "Q8_0 / IQ4_NL read one dword past a segment");
     // segments whose digits can be staged in LDS for the segment's other waves
-    constexpr int SHC = sdig_share_cap(NW);
+    // (rows without the argmax have nine or more: one wave each at most)
+    constexpr int SHC = ARGMAX ? sdig_share_cap(NW) : 0;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1842,7 +1843,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemv_sdig(const uint8_t *__restrict
                                                        int rpc, ArgPart *__restrict__ parts,
                                                        const float *resid, int epi)
 {
-    constexpr int SHC = sdig_share_cap(NW);
+    constexpr int SHC = ARGMAX ? sdig_share_cap(NW) : 0;
     __shared__ __attribute__((aligned(16))) uint8_t ring[NW * D * sdig_slot(FMT)];
     __shared__ __attribute__((aligned(16))) uint32_t digs[SHC > 0 ? SHC : 1][kDigQuads][64][4];
     __shared__ float part[kSdigMaxRows][NW]; // one column per segment (nseg <= NW)

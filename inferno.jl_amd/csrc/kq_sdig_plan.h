@@ -1,6 +1,7 @@
 // kq_sdig_plan.h -- launch plan and index arithmetic of the streamed digit
-// GEMV (k_gemv_sdig, kq_gemv.hip): Q6_K / Q8_0 / IQ4_NL rows, the lm_head with
-// the fused argmax, the FFN down projection.
+// GEMV (k_gemv_sdig, kq_gemv.hip): the Q6_K / Q8_0 lm_head with the fused argmax
+// (rows of 1 to 16 segments), and Q6_K / Q8_0 / IQ4_NL rows of more than 16384
+// columns (9 to 16 segments; shorter ones run in k_gemv_mdig).
 //
 // The kernel forms every global address, LDS offset, wait count and row index
 // through these functions, and the host-side bounds check
@@ -264,21 +265,21 @@ struct SdigPlan {
 
 // Waves per workgroup, rows per chunk and workgroups per CU by segment count,
 // measured on MI355X (us per GEMV in sweeps of HBM-resident copies; the
-// previous plan in parentheses where it differed):
-//   1 segment     8 waves, 2 per CU (LDS), 32 rows for the 151936 x 2048
-//                 Q6_K lm_head (53-55 us), by size for plain rows (sdig_plan).
-//                 Rows finish inside their wave.
+// previous plan in parentheses where it differed).  Rows of 2 to 8 segments were
+// timed plain; only the lm_head's come here.
+//   1 segment     8 waves, 2 per CU (LDS), 32 rows: the 151936 x 2048 Q6_K
+//                 lm_head 53-55 us.  Rows finish inside their wave.
 //   2..6          12 waves, 16 rows, 1 per CU (all of 113-137 KB of LDS a CU
 //                 holds; 4 per CU queued three more in rounds: 12288 x 4096
-//                 Q6_K 11.2 us against 15.6): 4096 x 4096 Q8_0 6.47, Q6_K 6.48,
-//                 IQ4_NL 6.23 (8 waves: 6.95+); 4096 x 6144 Q6_K 8.17;
-//                 4096 x 8192 Q8_0 9.67 (16.0); 4096 x 10240 Q8_0 12.70
-//                 (18.7); 4096 x 12288 Q6_K 12.3-12.4 (6 waves: 14.3).
-//                 Two or more waves per segment share its staged digits.
+//                 Q6_K 11.2 us against 15.6): 4096 x 4096 Q8_0 6.47, Q6_K 6.48;
+//                 4096 x 6144 Q6_K 8.17; 4096 x 8192 Q8_0 9.67 (16.0); 4096 x
+//                 10240 Q8_0 12.70 (18.7); 4096 x 12288 Q6_K 12.3-12.4 (6
+//                 waves: 14.3).  Two or more waves per segment share its
+//                 staged digits.
 //   7..8          16 waves, 16 rows, 2 per CU: 4096 x 14336 Q6_K 15.1-15.5
-//                 (18.2), IQ4_NL 16.1-16.3 (19.8); 4096 x 16384 Q6_K 15.7
-//                 (18.9).  Q8_0, whose 16-wave workgroup takes 104 KB of
-//                 LDS: 8 waves, 16 rows, 4 per CU (4096 x 16384 17.0; 21.8).
+//                 (18.2); 4096 x 16384 Q6_K 15.7 (18.9).  Q8_0, whose 16-wave
+//                 workgroup takes 104 KB of LDS: 8 waves, 16 rows, 4 per CU
+//                 (4096 x 16384 17.0; 21.8).
 //   9..12         12 waves, 16 rows, 1 per CU: 4096 x 24576 Q6_K 20.6 (16
 //                 waves 21.3), 4096 x 20480 Q8_0 21.9 (23.0).
 //   13..16        16 waves, 16 rows, 1 per CU: 8192 x 28672 Q6_K 42.6 (2 per
@@ -316,15 +317,10 @@ inline SdigPlan sdig_plan(int fmt, int nblk, int outer, bool argmax, int ncu)
     const int ncu1 = sd_max(1, ncu);
     int per_cu = sdig_wg_per_cu(fmt, p.nseg);
     // One-segment rows: the staged digits put a workgroup at 56-72 KB of LDS,
-    // two per CU.  With the argmax (the lm_head) 32 rows per chunk (151936 x
-    // 2048 Q6_K 53.3-54.6 us against 55.3-57.2 with one x load per wave and
-    // three workgroups per CU); plain, rows per chunk by matrix size (151936 x
-    // 2048 52.1 us against 61.0 with 3 per CU and 32 rows; 4096 x 2048 Q8_0
-    // 4.72 against 6.30; 2048 x 2048 Q6_K with 8-row chunks 4.39 against 6.12).
+    // two per CU, 32 rows per chunk (151936 x 2048 Q6_K 53.3-54.6 us against
+    // 55.3-57.2 with one x load per wave and three workgroups per CU).
     if (p.nseg == 1) {
         per_cu = 2;
-        if (!argmax)
-            p.rpc = outer >= 64 * ncu1 ? 32 : outer >= 16 * ncu1 ? 16 : 8;
         // a third ring slot per wave where two workgroups still fit a CU
         // (Q6_K / IQ4_NL: 2 x 71 KB; Q8_0's 3 KB slots would not): 151936 x
         // 2048 Q6_K 49.4 us against 52.1 with two slots (four: 58.1, one

@@ -147,20 +147,20 @@ GEMV_CASES = [
     (synth.Q6_K, 151936, 2048),   # the lm_head shape as a plain GEMV (one segment, staged digits)
     (synth.Q6_K, 7, 768),         # rows of 630 bytes: segments at byte phases (streamed kernel)
     (synth.Q8_0, 4096, 4096),
-    (synth.Q8_0, 11, 2304),       # partial 64-block segment
+    (synth.Q8_0, 11, 2304),       # 72 blocks: the wide lane layout, the pass partly idle
     (synth.Q8_0, 6, 96),          # 3 blocks a row, at byte phases
     (synth.IQ4_NL, 2048, 1024),   # an SSM-projection-sized IQ4_NL matrix
-    (synth.IQ4_NL, 1000, 4096),   # two 64-block segments per row
-    (synth.IQ4_NL, 13, 2304),     # partial segment (72 blocks)
+    (synth.IQ4_NL, 1000, 4096),   # 128 blocks a row: the wide lane layout, one row per wave
+    (synth.IQ4_NL, 13, 2304),     # 72 blocks: two steps of 32 and a partial one
     (synth.IQ4_NL, 5, 96),        # 3 blocks a row, at byte phases
     (synth.Q4_K, 1536, 4096),     # one GPU's gate/up rows of the FFN over 8 GPUs
     (synth.Q6_K, 4096, 1536),     # one GPU's down-projection columns (6 blocks a row)
-    (synth.Q4_K, 300, 5120),      # 16 + 4 blocks: persistent multi-pass kernel, 2-pass capacity
-    (synth.Q5_K, 77, 11008),      # 43 blocks: 3 passes, the last partial (4-pass capacity)
-    (synth.Q4_K, 2000, 13824),    # 54 blocks, many row groups per wave
-    (synth.Q4_K, 64, 28672),      # 112 blocks: 7 passes (8-pass capacity)
-    (synth.Q4_K, 10, 33024),      # 129 blocks: past the persistent kernel, serial passes
-    (synth.Q4_K, 4096, 5120),     # 256 workgroups over 256 CUs: serial passes, the last partial
+    (synth.Q4_K, 300, 5120),      # 20 blocks: five steps of four in the matrix-core kernel
+    (synth.Q5_K, 77, 11008),      # 43 blocks: eleven steps, the last partial
+    (synth.Q4_K, 2000, 13824),    # 54 blocks, two groups of rows per workgroup
+    (synth.Q4_K, 64, 28672),      # 112 blocks: the wide kernel, 7 passes in turn
+    (synth.Q4_K, 10, 33024),      # 129 blocks: 9 passes, the last of one block
+    (synth.Q4_K, 4096, 5120),     # five steps, four groups of rows per workgroup
     (synth.IQ4_NL, 8200, 2048),   # IQ4_NL in the persistent wide kernel
     (synth.IQ4_NL, 4096, 4096),   # IQ4_NL in the wide kernel, one workgroup per CU
     (synth.Q8_0, 8200, 2048),     # Q8_0 in the persistent wide kernel
@@ -208,17 +208,20 @@ def test_gemv_host_mirror_and_weight_cache(t):
 
 
 # Shapes that reach every launch the host makes (one instantiation each):
-#   Q4_K / Q5_K wide kernel, two rows per wave: ragged row counts, 1..9
-#     passes of 4096 columns, the last one partial;
-#   the persistent wide kernel: >= 8192 rows of at most 4096 columns;
-#   the streamed digit kernel: 8 waves for one segment of 2048 columns and
-#     for 7..8 Q8_0 segments, 12 waves for 2..6 (staged digits shared by two
-#     or more waves of a segment) and 9..12, 16 waves for 7..8 Q6_K / IQ4_NL
-#     segments and 13..16 (waves past the segments idle), partial last
-#     segments, chunks that end inside a workgroup's last round;
-#   rows that are not 16-byte multiples (Q6_K rows of any block count, Q8_0 and
-#     IQ4_NL rows of any multiple of 32 columns): segments copied from the
-#     unit below them, at byte phases 2..14, 1 to 16 segments;
+#   the wide kernels (Q4_K of at most 16 blocks, Q5_K of 13 to 16, Q8_0 and
+#     IQ4_NL rows that fill their lanes, Q4_K / Q5_K rows of more than 64 blocks):
+#     one and two rows per wave, ragged row counts, 1 to 9 passes of 4096
+#     columns, the last one partial; persistent from 8192 rows of at most 4096
+#     columns on;
+#   the matrix-core kernel (other rows of at most 16384 columns), four rows and
+#     1024 columns a step: 1 to 4, 5 to 12 and 13 to 16 steps, partial last
+#     steps and row groups, one and several groups per workgroup, rows at byte
+#     phases 2..14 (Q6_K rows of any block count, Q8_0 and IQ4_NL rows of any
+#     multiple of 32 columns);
+#   the streamed digit kernel (Q6_K / Q8_0 / IQ4_NL rows past 16384 columns): 12
+#     waves for 9..12 segments of 2048 columns, 16 for 13..16 (waves past the
+#     segments idle), partial last segments, phased and not, chunks that end
+#     inside a workgroup's last round;
 #   rows past 16 segments: the byte-granular kernel.
 LAUNCH_SHAPES = [
     (synth.Q4_K, 1037, 4096), (synth.Q5_K, 515, 4608), (synth.Q4_K, 9, 8448),
@@ -235,7 +238,10 @@ LAUNCH_SHAPES = [
     (synth.Q6_K, 33, 2304), (synth.Q8_0, 13, 896), (synth.Q8_0, 1000, 2336), (synth.IQ4_NL, 9, 2336),
     (synth.IQ4_NL, 517, 4640), (synth.Q6_K, 1031, 32512), (synth.Q8_0, 3, 32),
     (synth.Q8_0, 5, 34816),
-    (synth.Q5_K, 100, 5120),    # persistent multi-pass kernel, 2-pass capacity
+    (synth.Q5_K, 100, 5120),
+    (synth.Q5_K, 8199, 3328), (synth.Q5_K, 8203, 3840),  # persistent, the pass partly idle
+    (synth.Q8_0, 8197, 3840), (synth.Q8_0, 8193, 4096), (synth.IQ4_NL, 8201, 3840), (synth.IQ4_NL, 8194, 4096),
+    (synth.IQ4_NL, 31, 18464), (synth.Q8_0, 260, 26656), (synth.Q6_K, 260, 17152),  # streamed, phased
 ]
 
 
@@ -271,15 +277,16 @@ def test_gemv_every_launch(t, outer, inner):
 
 @pytest.mark.parametrize("hidden,inter", [
     (4096, 1030),   # wide kernel, one gate and one up row per wave
-    (8448, 515),    # three passes, the last partial (one row pair per wave: serial)
-    (14336, 300),   # four passes, serial
-    (5120, 600),    # two passes, serial
-    (5120, 2056),   # persistent multi-pass kernel, 2-pass capacity
-    (8448, 2100),   # persistent multi-pass kernel, 4-pass capacity, the last pass partial
-    (5120, 2048),   # 256 workgroups over 256 CUs: serial passes
-    (20480, 64),    # 80 blocks: past the persistent kernel, serial passes
-    (4096, 8195),   # persistent kernel
-    (2560, 8200),   # persistent kernel, partial pass
+    (8448, 515),    # the matrix-core kernel: 33 blocks in nine steps, the last partial
+    (14336, 300),   # fourteen steps
+    (5120, 600),    # five steps, one group of rows per workgroup
+    (5120, 2056),   # three groups
+    (8448, 2100),   # three groups, partial last step
+    (5120, 2048),   # two groups
+    (20480, 64),    # 80 blocks: the wide kernel, five passes in turn
+    (4096, 8195),   # Q4_K: persistent
+    (3840, 8195),   # Q4_K: persistent, the pass partly idle
+    (2560, 8200),   # three steps, the last partial, nine groups
 ])
 @pytest.mark.parametrize("t", [synth.Q4_K, synth.Q5_K])
 def test_gate_up_every_launch(t, hidden, inter):

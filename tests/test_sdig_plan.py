@@ -1,7 +1,7 @@
 """CPU check of the streamed digit GEMV's launch arithmetic (no GPU).
 
-k_gemv_sdig (Q6_K / Q8_0 / IQ4_NL GEMV, the lm_head with the fused argmax,
-the FFN down projection) forms every address, LDS offset, wait count and row
+k_gemv_sdig (the lm_head with the fused argmax, Q6_K / Q8_0 / IQ4_NL rows past
+16384 columns) forms every address, LDS offset, wait count and row
 index through inferno.jl_amd/csrc/kq_sdig_plan.h.  tests/native/sdig_check.hip
 includes the same header and walks a whole launch -- every workgroup, wave,
 item, copy and lane -- asserting that global reads and writes stay inside W,
@@ -9,9 +9,10 @@ x, y and the argmax partials, copies land in the wave's own LDS ring, ring
 reads stay inside a slot, each vmcnt wait covers the item it guards, every
 wave meets the same barriers and every row is produced exactly once.
 
-The launches checked are the ones the GPU tests and the benchmark make, the
-151936 x 2048 plain Q6_K GEMV, rows of every segment count the kernel takes
-(1..16), and CU counts that push the grid to its limits.
+The launches checked are the ones the GPU tests and the benchmark make, rows
+of every segment count the kernel takes (1..16; plain rows of up to 8 segments
+run in another kernel, but the arithmetic covers them), and CU counts that
+push the grid to its limits.
 """
 import ctypes as C
 from pathlib import Path
@@ -41,7 +42,7 @@ def chk():
     return run
 
 
-# (type, outer, inner) the GPU tests run through the streamed kernel
+# (type, outer, inner), plain and with the argmax
 STREAM_SHAPES = ((Q6_K, 1029, 12288), (Q6_K, 77, 6144), (Q6_K, 300, 24576), (Q6_K, 33, 10240),
                  (Q6_K, 65, 16384), (Q8_0, 1031, 4096), (Q8_0, 45, 2304), (Q8_0, 19, 256),
                  (IQ4_NL, 517, 4608), (Q8_0, 300, 14336), (Q8_0, 129, 18688), (Q6_K, 40, 32768),
@@ -95,7 +96,7 @@ def test_every_segment_count(chk, t):
     """Rows of 1..16 segments (full and partial last segments): 8 waves for
     one segment, 12 for 2..6 and 9..12, 16 for 7..8 (Q8_0: 8) and 13..16; three
     ring slots for one segment where two workgroups still fit a CU (not Q8_0's
-    3 KB slots), else two; 16 rows per chunk (at 4096 rows)."""
+    3 KB slots), else two; 16 rows per chunk, 32 for one segment (at 4096 rows)."""
     unit = 2048 if t == Q6_K else 256  # the host's row-alignment unit
     for nseg in range(1, 17):
         for inner in {2048 * nseg, 2048 * nseg - (2048 - unit)}:
@@ -104,7 +105,7 @@ def test_every_segment_count(chk, t):
                     else 12 if nseg <= 12 else 16)
             depth = 3 if nseg == 1 and t != Q8_0 else 2
             assert (st[1], st[2], st[4]) == (want, depth, nseg), (inner, st)
-            assert st[3] == 16, (inner, st)  # one segment: 16 rows per chunk at 4096 plain rows
+            assert st[3] == (32 if nseg == 1 else 16), (inner, st)
     n, msg, _ = chk(t, 2048 * 16 + unit, 7)
     assert n > 0 and "does not take" in msg  # 17 segments: the byte-granular kernel's
     for nseg in range(1, 17):  # ragged row counts
