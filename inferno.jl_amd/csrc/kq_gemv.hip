@@ -548,38 +548,6 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_kwide_norm(const uint8_t *__r
 // exponent A, exponent B} of the pair, Q6_K 2^(e - 22) of its four groups, Q8_0
 // and IQ4_NL 2^(e - 22) of its two blocks.
 constexpr int kMdPlaneDw = 65 * 4, kMdStepDw = 4 * kMdPlaneDw;
-// Bytes of a block and blocks of a step; 16-byte pieces of a row's step (PHASED:
-// from the 16-byte unit its first byte lies in, at an even phase of 0 .. 14);
-// pieces between two rows in a ring slot (one more: 13 of 16 lanes' 128-bit reads then hit
-// distinct banks, 8 without); 1 KB copies of a slot.
-template <int FMT>
-struct MdFmt;
-template <>
-struct MdFmt<kQ4_K> {
-    static constexpr int BYTES = 144, BLOCKS = 4, PIECES = 36, PITCH = 37, COPIES = 3;
-    static constexpr bool PHASED = false;
-};
-template <>
-struct MdFmt<kQ5_K> {
-    static constexpr int BYTES = 176, BLOCKS = 4, PIECES = 44, PITCH = 45, COPIES = 3;
-    static constexpr bool PHASED = false;
-};
-template <>
-struct MdFmt<kQ6_K> {
-    static constexpr int BYTES = 210, BLOCKS = 4, PIECES = 54, PITCH = 55, COPIES = 4;
-    static constexpr bool PHASED = true;
-};
-template <>
-struct MdFmt<kQ8_0> {
-    static constexpr int BYTES = 34, BLOCKS = 32, PIECES = 69, PITCH = 70, COPIES = 5;
-    static constexpr bool PHASED = true;
-};
-template <>
-struct MdFmt<kIQ4_NL> {
-    static constexpr int BYTES = 18, BLOCKS = 32, PIECES = 37, PITCH = 38, COPIES = 3;
-    static constexpr bool PHASED = true;
-};
-
 // Digits of one float4 of x (number f of the row); 8 consecutive threads hold
 // one sub-block of 32 elements.
 template <int FMT>
@@ -776,7 +744,7 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
     constexpr int SLOT = 1024 * NC;
     constexpr int NX = (MAXS * 256 + NT - 1) / NT; // float4 of x per thread
     // float4 of x per thread that the ring holds at a time (with nw: both)
-    constexpr int XC = NX < D * NC / (NORM ? 2 : 1) ? NX : D * NC / (NORM ? 2 : 1);
+    constexpr int XC = md_x_chunk(NX, D, NC, NORM);
     static_assert(4 * LP <= 64 * NC && D <= 3, "a unit is NC copies");
     __shared__ __attribute__((aligned(16))) uint8_t ring[NWV * D * SLOT];
     __shared__ __attribute__((aligned(16))) uint32_t dig[MAXS * kMdStepDw];
@@ -794,10 +762,8 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
     const int ngroups = (outer + 3) >> 2;
     const int G0 = (int)blockIdx.x * gpw, ng = min(gpw, ngroups - G0);
     const int units = ng * NM * nstep;
-    const int n = wave < units ? (units - wave - 1) / NWV + 1 : 0; // this wave's
-    // quotients by nstep of numbers up to 16: inv = ceil(65536 / nstep)
-    auto div_steps = [&](int a) { return (int)(((uint32_t)a * inv) >> 16); };
-    const int qn = div_steps(NWV), rn = NWV - qn * nstep;
+    const int n = md_wave_units(units, wave, NWV);
+    const int qn = md_div(NWV, inv), rn = NWV - qn * nstep;
 
     // the residual of the thread's first row, ahead of everything else
     float rv = 0.0f;
@@ -809,16 +775,15 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
 
     // x, then nw: a wave copies what its own threads convert, 1 KB a copy, at
     // most XC copies of each at a time
-    const int nx = (inner / 4 - 64 * wave + NT - 1) / NT; // its copies of x
-    const int xc = min(nx, XC), raw_slots = ((NORM ? 2 : 1) * xc + NC - 1) / NC;
+    const int nx = md_x_copies(inner, wave, NT); // its copies of x
+    const int xc = min(nx, XC), raw_slots = md_raw_slots(xc, NORM, NC);
     const int pre = max(0, min(n, D - raw_slots)); // units issued before x is there
     const uint32_t raw = (uint32_t)(D - raw_slots) * SLOT;
     auto issue_x = [&](int k0) {
 #pragma unroll
         for (int k = 0; k < XC; ++k)
             if (k0 + k < nx) {
-                // threads past the row (rows of no whole 256 columns) copy its end
-                const uint32_t o = (uint32_t)min(16 * tid, 4 * inner - 16 - 16 * NT * (k0 + k));
+                const uint32_t o = md_x_off(inner, tid, NT, k0 + k);
                 lds_copy16_at(x + 4 * NT * (k0 + k), o, mine_lds + raw + 1024 * k);
                 if constexpr (NORM)
                     lds_copy16_at(nw + 4 * NT * (k0 + k), o, mine_lds + raw + 1024 * (xc + k));
@@ -831,7 +796,7 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
     struct Cur {
         int vg, s;
     };
-    const int g0 = div_steps(wave);
+    const int g0 = md_div(wave, inv);
     Cur lc = {g0, wave - g0 * nstep}, uc = lc;
     auto advance = [&](Cur &c) {
         c.vg += qn;
@@ -844,9 +809,9 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
     uint32_t ro[NC], po[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-        const int q = 64 * i + lane, row = min(q / LP, 3);
+        const int q = 64 * i + lane, row = md_piece_row(q, LP);
         ro[i] = __umul24((uint32_t)row, row_bytes);
-        po[i] = 16u * (uint32_t)min(q - row * LP, PP - 1);
+        po[i] = md_piece_off(q, row, LP, PP);
     }
     int islot = 0;
     auto issue = [&]() {
@@ -859,14 +824,8 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mdig(const uint8_t *__restric
         base -= phase;
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
-            uint32_t o = min(ro[i], rmax);
-            if constexpr (F::PHASED) { // from the 16-byte unit of the row's first byte
-                o += phase;
-                o = (o & ~15u) + min(po[i], ((o & 15u) + nbytes - 1u) & ~15u);
-            } else {
-                o += min(po[i], nbytes - 16u);
-            }
-            lds_copy16_at(base, o, mine_lds + SLOT * islot + 1024 * i);
+            lds_copy16_at(base, md_copy_off<F::PHASED>(min(ro[i], rmax), po[i], nbytes, phase),
+                          mine_lds + SLOT * islot + 1024 * i);
         }
         islot = islot == D - 1 ? 0 : islot + 1;
         advance(lc);
@@ -1881,7 +1840,7 @@ static void launch_mdig(const uint8_t *W, const uint8_t *W2, const float *x, flo
     const int nstep = (nblk + BPS - 1) / BPS, ngroups = (outer + 3) / 4;
     const int gpw = mdig_groups(outer, nstep * (GATEUP ? 2 : 1), device_cus());
     const dim3 grid((ngroups + gpw - 1) / gpw);
-    const uint32_t inv = (65536u + nstep - 1) / nstep;
+    const uint32_t inv = md_inv(nstep);
     auto launch = [&](auto nwv, auto d, auto maxs) {
         hipLaunchKernelGGL((k_gemv_mdig<FMT, GATEUP, NORM, RESID, nwv.value, d.value, maxs.value>), grid,
                            dim3(nwv.value * 64), 0, s, W, W2, x, y, outer, nblk, gpw, inv, nw, eps, resid, epi);

@@ -91,6 +91,91 @@ constexpr MdPlan mdig_plan(int type, int nstep, int groups)
     return type == kQ6_K || type == kQ8_0 ? MdPlan{8, 2, 16} : MdPlan{12, 2, 16};
 }
 
+// ---- k_gemv_mdig's index arithmetic, which tests/native/mdig_check.hip walks ----
+// Bytes of a block and blocks of a step; 16-byte pieces of a row's step (PHASED:
+// from the 16-byte unit its first byte lies in, at an even phase of 0 .. 14);
+// pieces between two rows in a ring slot (one more: 13 of 16 lanes' 128-bit reads then hit
+// distinct banks, 8 without); 1 KB copies of a slot.
+template <int FMT>
+struct MdFmt;
+template <>
+struct MdFmt<kQ4_K> {
+    static constexpr int BYTES = 144, BLOCKS = 4, PIECES = 36, PITCH = 37, COPIES = 3;
+    static constexpr bool PHASED = false;
+};
+template <>
+struct MdFmt<kQ5_K> {
+    static constexpr int BYTES = 176, BLOCKS = 4, PIECES = 44, PITCH = 45, COPIES = 3;
+    static constexpr bool PHASED = false;
+};
+template <>
+struct MdFmt<kQ6_K> {
+    static constexpr int BYTES = 210, BLOCKS = 4, PIECES = 54, PITCH = 55, COPIES = 4;
+    static constexpr bool PHASED = true;
+};
+template <>
+struct MdFmt<kQ8_0> {
+    static constexpr int BYTES = 34, BLOCKS = 32, PIECES = 69, PITCH = 70, COPIES = 5;
+    static constexpr bool PHASED = true;
+};
+template <>
+struct MdFmt<kIQ4_NL> {
+    static constexpr int BYTES = 18, BLOCKS = 32, PIECES = 37, PITCH = 38, COPIES = 3;
+    static constexpr bool PHASED = true;
+};
+
+// A unit is one step of a group of four rows (of its gate or of its up rows);
+// wave w of nwv takes units w, w + nwv, ...
+__host__ __device__ inline int md_wave_units(int units, int wave, int nwv)
+{
+    return wave < units ? (units - wave - 1) / nwv + 1 : 0;
+}
+// Quotients by nstep of numbers up to 16: inv = ceil(65536 / nstep).
+__host__ __device__ inline uint32_t md_inv(int nstep) { return (65536u + (uint32_t)nstep - 1) / (uint32_t)nstep; }
+__host__ __device__ inline int md_div(int a, uint32_t inv) { return (int)(((uint32_t)a * inv) >> 16); }
+
+// x (and, NORM, the norm's weights) in 1 KB copies, a wave those that its own
+// threads convert: how many, how many of each the ring's last slots hold at a
+// time, the slots that takes, and a thread's byte offset in its copy k (threads
+// past the row, in rows of no whole 256 columns, copy its end).
+__host__ __device__ inline int md_x_copies(int inner, int wave, int nt)
+{
+    return (inner / 4 - 64 * wave + nt - 1) / nt;
+}
+__host__ __device__ constexpr int md_x_chunk(int nx, int d, int copies, bool norm)
+{
+    return nx < d * copies / (norm ? 2 : 1) ? nx : d * copies / (norm ? 2 : 1);
+}
+__host__ __device__ inline int md_raw_slots(int xc, bool norm, int copies)
+{
+    return ((norm ? 2 : 1) * xc + copies - 1) / copies;
+}
+__host__ __device__ inline uint32_t md_x_off(int inner, int tid, int nt, int k)
+{
+    return (uint32_t)min(16 * tid, 4 * inner - 16 - 16 * nt * k);
+}
+
+// Piece q of a slot (copy q / 64, lane q % 64): its row of the group and its
+// byte offset in that row's step.
+__host__ __device__ inline int md_piece_row(int q, int pitch) { return min(q / pitch, 3); }
+__host__ __device__ inline uint32_t md_piece_off(int q, int row, int pitch, int pieces)
+{
+    return 16u * (uint32_t)min(q - row * pitch, pieces - 1);
+}
+// Byte offset, from the group's first row's step (PHASED: from the 16-byte unit
+// `phase` bytes below it), of the piece at `piece` of the row `row` bytes
+// further: the row's nbytes, the last piece of them again past their end.
+template <bool PHASED>
+__host__ __device__ inline uint32_t md_copy_off(uint32_t row, uint32_t piece, uint32_t nbytes, uint32_t phase)
+{
+    if constexpr (PHASED) { // from the 16-byte unit of the row's first byte
+        const uint32_t o = row + phase;
+        return (o & ~15u) + min(piece, ((o & 15u) + nbytes - 1u) & ~15u);
+    } else {
+        return row + min(piece, nbytes - 16u);
+    }
+}
+
 // The folded norm on a single weight of at most 16 blocks a row: whether the
 // wide kernels take it.  By row count too (no other call promises these bits):
 // the wide kernels are ahead while one round of their workgroups holds the rows

@@ -1,7 +1,8 @@
 """Which kernel takes a GEMV (kq_gemv_plan.h, through tests/native/
 gemv_plan_check.hip, on the CPU): the faster one at shapes where the two were
 timed 4 % apart or more, and on the GPU both kernels' results at the edges of
-the rules.
+the rules.  And every copy, slot and wait of k_gemv_mdig's launches, walked on
+the CPU through the kernel's own index functions (tests/native/mdig_check.hip).
 """
 import ctypes as C
 from pathlib import Path
@@ -160,3 +161,42 @@ def test_iq4_nl_rows(outer, inner):
     ratio = np.max(np.abs(y.astype(np.float64) - oracle.gemv_f64(synth.IQ4_NL, w, x, inner, outer)) / tol)
     print(f"max err/tol = {ratio:.3e}", flush=True)
     assert ratio <= 1.0
+
+
+def _mdig_walk(plan, t, outer, inner, gateup=False, norm=False, ncu=256):
+    msg, st = C.create_string_buffer(512), (C.c_longlong * 8)()
+    plan.mdig_check.restype = C.c_longlong
+    n = plan.mdig_check(t, inner // (256 if t in (Q4_K, Q5_K, Q6_K) else 32), outer, int(gateup), int(norm), ncu, msg, 512, st)
+    assert n == 0, f"type {t} {outer}x{inner} gate/up {gateup} norm {norm}: {n} violations, first: {msg.value.decode()}"
+    return list(st)
+
+
+# every number of steps, whole and partial last steps, ragged row groups
+@pytest.mark.parametrize("t", (Q4_K, Q5_K, Q6_K, synth.Q8_0, synth.IQ4_NL))
+def test_matrix_core_launches_stay_in_bounds(plan, t):
+    unit = 256 if t in (Q4_K, Q5_K, Q6_K) else 32
+    for nstep in range(1, 17):
+        for inner in sorted({1024 * nstep, 1024 * nstep - unit, 1024 * (nstep - 1) + unit}):
+            for outer in (1, 6, 1027, 4100):
+                _mdig_walk(plan, t, outer, inner)
+    for outer, inner in ((12288, 4096), (151936, 2560), (32771, 3328), (5, 16384)):
+        _mdig_walk(plan, t, outer, inner)
+
+
+@pytest.mark.parametrize("t", (Q4_K, Q5_K))
+def test_matrix_core_gate_up_and_norm_launches_stay_in_bounds(plan, t):
+    for nstep in range(1, 17):
+        for inner in (1024 * nstep, 1024 * nstep - 768):
+            for outer in (3, 1030, 2049):
+                for norm in (False, True):
+                    _mdig_walk(plan, t, outer, inner, gateup=True, norm=norm)
+                if nstep <= 4:
+                    _mdig_walk(plan, t, outer, inner, norm=True)
+    _mdig_walk(plan, t, 13824, 5120, gateup=True, norm=True)
+
+
+@pytest.mark.parametrize("ncu", (1, 7, 80, 304))
+def test_matrix_core_launches_on_other_devices(plan, ncu):
+    for t, outer, inner in ((Q6_K, 4099, 3840), (synth.Q8_0, 1031, 16352), (Q4_K, 2050, 8448), (Q5_K, 31, 256)):
+        st = _mdig_walk(plan, t, outer, inner, ncu=ncu)
+        assert st[1] * (-(-inner // 1024)) <= 512
