@@ -239,12 +239,67 @@ inline int prefill_split_tokens(int T, int outer, int ncu)
     const int64_t r32 = (((int64_t)T + 31) / 32 * nt + cus - 1) / cus, r64 = (((int64_t)T + 63) / 64 * nt + cus - 1) / cus;
     return 10 * r32 <= 17 * r64 ? 32 : 64;
 }
+// ---- copies and LDS reads of k_prefill_q4k_wide, _thin and _split, which
+// tests/native/prefill_copy_check.hip walks ----
+// A block's 32 chunks of 8 values in a row of Xh: chunk 16 h + 4 g + c at place
+// 8 g + 4 h + c.
+__host__ __device__ constexpr int pf_chunk_place(int chunk)
+{
+    return 8 * ((chunk >> 2) & 3) + 4 * (chunk >> 4) + (chunk & 3);
+}
+// An X stage is 128 bytes (eight 16-byte chunks) of each token, eight tokens a
+// copy: lane l of copy i brings token 8 i + l / 8, and its place l % 8 holds chunk
+// (l % 8) ^ (token / 2 % 8), so that the 16 lanes of a 128-bit read, one chunk of
+// consecutive tokens, hit distinct banks.
+__host__ __device__ inline int pf_copy_token(int i, int lane) { return 8 * i + (lane >> 3); }
+__host__ __device__ inline int pf_copy_chunk(int token, int lane) { return (lane & 7) ^ ((token >> 1) & 7); }
+// Byte of chunk c of token m in a stage of LDS.
+__host__ __device__ inline uint32_t pf_stage_at(int m, int c) { return 128u * (uint32_t)m + 16u * (uint32_t)(c ^ ((m >> 1) & 7)); }
+// Weight pieces of 16 bytes: whole blocks of `rows` rows (the last piece again
+// past them), or the header and 32 quant bytes (pair j) of each.
+struct PfPiece {
+    int row;
+    uint32_t off; // in the row's block
+};
+__host__ __device__ inline PfPiece pf_block_piece(int i, int lane, int rows)
+{
+    const int q = min(64 * i + lane, rows * 9 - 1);
+    return {q / 9, 16u * (uint32_t)(q - 9 * (q / 9))};
+}
+__host__ __device__ inline PfPiece pf_pair_piece(int i, int lane, int j)
+{
+    const int q = 64 * i + lane, row = q / 3, piece = q - 3 * row;
+    return {row, piece ? 32u * (uint32_t)j + 16u * (uint32_t)piece : 0u};
+}
+
 // The same product on fp32 operands (k_prefill_q4k_split), any inner; needs
 // T * outer <= INT32_MAX.
 hipError_t launch_prefill_q4k_f32(const void *w, const float *X, float *Y, int T, int inner,
                                   int outer, hipStream_t s);
 
 // kq_q8k.hip
+// k_gemv_q8k6: rows of at most kQ86MaxBlocks Q6_K blocks, eight (1680 bytes) an
+// item, copied from the 16-byte unit of the item's first byte (phase bytes below
+// it) in two copies of 64 lanes; pieces past the item's last byte are the last one
+// again.
+constexpr int kQ86MaxBlocks = 24, kQ86Waves = 16, kQ86Items = (kQ86MaxBlocks + 7) / 8, kQ86Slot = 2048;
+__host__ __device__ inline uint32_t q86_copy_off(int i, int lane, uint32_t phase, int blocks)
+{
+    return min(1024u * (uint32_t)i + 16u * (uint32_t)lane, (phase + (uint32_t)blocks * 210u - 1u) & ~15u);
+}
+// Waves to a row: as many of 1, 2 (from 5 blocks on) and 4 (from 17) as one
+// round of the chip's waves has for every row.  (Two waves of a row of at most
+// eight blocks are one at work, in twice the workgroups.)  Measured on MI355X
+// (us, quantizing included, graph replays over weights in HBM, fewer / more
+// waves): 256 x 256 3.18 / 3.72, 256 x 512 3.21 / 3.34, 512 x 1024 3.50 / 3.56; 512 x 1280
+// 3.56 / 3.68, 512 x 2048 3.77 / 3.71; 512 x 5120 6.29 / 5.20, 1024 x 6144 6.75 / 5.76.
+inline int q86_team(int nb, int outer, int ncu)
+{
+    int tw = 1;
+    while (tw < 4 && (int64_t)outer * 2 * tw <= (int64_t)ncu * kQ86Waves && nb > (tw == 1 ? 4 : 16))
+        tw *= 2;
+    return tw;
+}
 hipError_t launch_quantize_q8k(const float *x, void *y, int64_t k, hipStream_t s);
 hipError_t launch_gemv_q8k(int type, const void *w, const void *q8, float *out, int inner,
                            int outer, hipStream_t s);

@@ -57,10 +57,6 @@ constexpr int PF_BM = kPrefillBM, PF_BN = kPrefillBN; // workgroup tile: tokens 
 // c at place 8 g + 4 h + c.  The wide kernel below multiplies a block in four
 // stages, lane half h of its matrix products covering columns 128 h + 32 g +
 // 8 c ..: with this order a stage of a token row is 128 contiguous bytes.
-__host__ __device__ constexpr int pf_chunk_place(int chunk)
-{
-    return 8 * ((chunk >> 2) & 3) + 4 * (chunk >> 4) + (chunk & 3);
-}
 // element i (a multiple of 8) of a row -> its element offset in Xh's row
 __device__ __forceinline__ int pf_x_place(int i) { return (i & ~255) + 8 * pf_chunk_place((i & 255) >> 3); }
 constexpr int PF_CVT_REG = 4; // 8-value steps a thread holds: 256 x 8 x 4 = 8192 values
@@ -622,22 +618,18 @@ __global__ __launch_bounds__(256, RU == 2 ? 2 : 3) void k_prefill_q4k_wide(
     const int m0 = ps.mt * PFW_BM, n0 = ps.nt * (128 * RU) + 32 * RU * wave; // this wave's first row
 
     // byte offsets of this wave's copies from Xh / W (stage 0, column 0):
-    // tokens 32 wave .. +31 of the X stage (8 a copy; chunk c of token m at
-    // place c ^ (m / 2 % 8) of its 128 bytes, so that the 16 lanes of a
-    // 128-bit read, one chunk of consecutive tokens, hit distinct banks) and
-    // the wave's own weight rows.  Rows past T or N re-read the last one.
+    // tokens 32 wave .. +31 of the X stage and the wave's own weight rows.
+    // Rows past T or N re-read the last one.
     uint32_t xo[4], wo[WB];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int m = 32 * wave + 8 * i + (lane >> 3);
-        const int c = (lane & 7) ^ ((m >> 1) & 7);
-        xo[i] = 2u * (uint32_t)min(m0 + m, T - 1) * (uint32_t)K + 16u * (uint32_t)c;
+        const int m = 32 * wave + pf_copy_token(i, lane);
+        xo[i] = 2u * (uint32_t)min(m0 + m, T - 1) * (uint32_t)K + 16u * (uint32_t)pf_copy_chunk(m, lane);
     }
 #pragma unroll
     for (int i = 0; i < WB; ++i) {
-        const int q = min(64 * i + lane, 32 * RU * 9 - 1);
-        const int row = q / 9, piece = q - 9 * row;
-        wo[i] = (uint32_t)min(n0 + row, N - 1) * row_bytes + 16u * (uint32_t)piece;
+        const PfPiece q = pf_block_piece(i, lane, 32 * RU);
+        wo[i] = (uint32_t)min(n0 + q.row, N - 1) * row_bytes + q.off;
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     const uint32_t xdst = lds0 + 4096u * wave, wdst = lds0 + 2 * PFW_XSTAGE + (uint32_t)WREG * wave;
@@ -664,11 +656,10 @@ __global__ __launch_bounds__(256, RU == 2 ? 2 : 3) void k_prefill_q4k_wide(
             for (int r = 0; r < 16; ++r) acc[u][t][r] = 0.0f;
 
     const uint8_t *wl = lds + 2 * PFW_XSTAGE + WREG * wave + 144 * li;
-    const int f = (li >> 1) & 7;
     const uint8_t *xl[4]; // the lane's chunk of K step c in buffer 0, token li
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-        xl[c] = lds + 128 * li + 16 * ((4 * h + c) ^ f);
+        xl[c] = lds + pf_stage_at(li, 4 * h + c);
 
     // lane (li, h): rows 32 u + li, columns 128 h .. 128 h + 127 of the block (qs
     // bytes 64 h ..): stage g is sub-block 4 h + g, K step c its bytes 8 c ..
@@ -871,20 +862,20 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_thin(const uint8_t *__re
 
     const int nb = (nk - half + 1) >> 1; // this wave's steps
     if (nb > 0) {
-        // copies: 8 tokens x 8 chunks each of the pair's 64 columns (chunk e of
-        // token m at place e ^ (m / 2 % 8) of its 128 bytes, for the banks),
-        // and header and 32 quant bytes of every row.  Rows past T or N re-read
-        // the last one, steps past the last repeat it.
+        // copies: the pair's 64 columns of X, and header and 32 quant bytes of
+        // every row.  Rows past T or N re-read the last one, steps past the
+        // last repeat it.
         uint32_t xo[XC], wo[WC];
 #pragma unroll
         for (int i = 0; i < XC; ++i) {
-            const int m = 8 * i + (lane >> 3), e = (lane & 7) ^ ((m >> 1) & 7);
-            xo[i] = 2u * (uint32_t)min(m0 + m, T - 1) * (uint32_t)K + 16u * (uint32_t)pf_chunk_place(8 * j + e);
+            const int m = pf_copy_token(i, lane);
+            xo[i] = 2u * (uint32_t)min(m0 + m, T - 1) * (uint32_t)K +
+                    16u * (uint32_t)pf_chunk_place(8 * j + pf_copy_chunk(m, lane));
         }
 #pragma unroll
         for (int i = 0; i < WC; ++i) {
-            const int q = 64 * i + lane, row = q / 3, piece = q - 3 * row;
-            wo[i] = (uint32_t)min(n0 + row, N - 1) * row_bytes + (piece ? 32u * j + 16u * piece : 0u);
+            const PfPiece q = pf_pair_piece(i, lane, j);
+            wo[i] = (uint32_t)min(n0 + q.row, N - 1) * row_bytes + q.off;
         }
         uint8_t *const mine = lds + PFT_WAVE * wave;
         const uint32_t xdst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mine;
@@ -899,8 +890,7 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_thin(const uint8_t *__re
             for (int k = 0; k < XC; ++k)
                 pf_copy16(x, xo[k], xdst + 1024 * k);
         };
-        const uint8_t *xl = mine + 128 * li, *wl = mine + PFT_X + 48 * li;
-        const int f = (li >> 1) & 7;
+        const uint8_t *wl = mine + PFT_X + 48 * li;
         issue(0);
         for (int i = 0; i < nb; ++i) {
             __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0): this step's copies
@@ -918,7 +908,7 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_thin(const uint8_t *__re
                     q[u][c] = *reinterpret_cast<const uint2 *>(wl + 32 * 48 * u + 16 + 16 * c + 8 * h);
 #pragma unroll
             for (int s = 0; s < 4; ++s)
-                x[s] = *reinterpret_cast<const half8 *>(xl + 16 * ((2 * s + h) ^ f));
+                x[s] = *reinterpret_cast<const half8 *>(mine + pf_stage_at(li, 2 * s + h));
             __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): in registers
             asm volatile("" ::: "memory");
             issue(i + 1);
@@ -1263,21 +1253,19 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
         }
         if (nb <= 0)
             return;
-        // copies: 8 tokens x 128 bytes each of an X stage, chunk c of token m
-        // at place c ^ (m / 2 % 8) of its 128 bytes (the 16 lanes of a 128-bit
-        // read hit distinct banks), and 64 rows x 3 pieces of the blocks.  32-bit
-        // offsets suffice: the launcher bounds K.  Rows past T or N re-read the
-        // last one, stages past the last repeat it.
+        // copies: 32 columns of X a stage, and 64 rows x 3 pieces of the blocks.
+        // 32-bit offsets suffice: the launcher bounds K.  Rows past T or N
+        // re-read the last one, stages past the last repeat it.
         Offset xo[XC], wo[3];
 #pragma unroll
         for (int i = 0; i < XC; ++i) {
-            const int m = 8 * i + (lane >> 3), c = (lane & 7) ^ ((m >> 1) & 7);
-            xo[i] = (Offset)min(m, T - 1 - m0) * ((Offset)K * 4u) + 16u * (uint32_t)c;
+            const int m = pf_copy_token(i, lane);
+            xo[i] = (Offset)min(m, T - 1 - m0) * ((Offset)K * 4u) + 16u * (uint32_t)pf_copy_chunk(m, lane);
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const int q = 64 * i + lane, row = q / 3, piece = q - 3 * row;
-            wo[i] = (Offset)min(row, N - 1 - n0) * (Offset)row_bytes + (piece ? 32u * j + 16u * piece : 0u);
+            const PfPiece q = pf_pair_piece(i, lane, j);
+            wo[i] = (Offset)min(q.row, N - 1 - n0) * (Offset)row_bytes + q.off;
         }
         const uint8_t *Xb = reinterpret_cast<const uint8_t *>(X + (size_t)m0 * K + 256 * half + 64 * j);
         const uint8_t *Wb = W + (size_t)n0 * row_bytes + 144 * half;
@@ -1297,8 +1285,7 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
             for (int k = 0; k < 3; ++k)
                 copy16(b, wo[k], wdst + 1024 * k);
         };
-        const uint8_t *xl = mine + 128 * li, *wl = mine + 2 * XST + 48 * li;
-        const int f = (li >> 1) & 7;
+        const uint8_t *wl = mine + 2 * XST + 48 * li;
 
         float4 xr[TT][2][2];
         uint2 qs[2][2];
@@ -1311,8 +1298,8 @@ __global__ __launch_bounds__(512, 2) void k_prefill_q4k_split(const uint8_t *__r
                 for (int c = 0; c < 2; ++c)
 #pragma unroll
                     for (int e = 0; e < 2; ++e)
-                        xr[t][c][e] = *reinterpret_cast<const float4 *>(xl + XST * s + 4096 * t +
-                                                                       16 * ((4 * c + 2 * h + e) ^ f));
+                        xr[t][c][e] = *reinterpret_cast<const float4 *>(mine + XST * s + 4096 * t +
+                                                                       pf_stage_at(li, 4 * c + 2 * h + e));
         };
         auto stage = [&](int s) {
             bf16x8 wq[2][2];

@@ -463,7 +463,6 @@ static bool q8kw_ok(int type, const void *w, int nb)
 // weights in HBM, that / this): 256 x 256 4.30 / 3.18, 512 x 1024 4.64 / 3.50, 1024 x
 // 4096 6.26 / 5.17, 1024 x 5120 7.31 / 5.66, 4096 x 4096 8.83 / 6.81 (held in the
 // memory-side cache 9.07 / 7.46).
-constexpr int kQ86MaxBlocks = 24, kQ86Waves = 16, kQ86Items = (kQ86MaxBlocks + 7) / 8, kQ86Slot = 2048;
 template <bool QX, int TW>
 __global__ __launch_bounds__(64 * kQ86Waves) void k_gemv_q8k6(const uint8_t *__restrict__ W,
                                                               const float *__restrict__ x,
@@ -498,11 +497,10 @@ __global__ __launch_bounds__(64 * kQ86Waves) void k_gemv_q8k6(const uint8_t *__r
         const int it = rank + TW * i;
         const uint8_t *base = W + (size_t)row * row_bytes + (size_t)it * 1680u;
         const uint32_t phase = (uint32_t)(uintptr_t)base & 15u;
-        // pieces past the item's last byte: the last one again
-        const uint32_t last = (phase + (uint32_t)min(8, nb - 8 * it) * 210u - 1u) & ~15u;
+        const int blocks = min(8, nb - 8 * it);
         base -= phase;
-        lds_copy16_at(base, min(16u * lane, last), mine_lds + SLOT * i);
-        lds_copy16_at(base, min(1024u + 16u * lane, last), mine_lds + SLOT * i + 1024);
+        lds_copy16_at(base, q86_copy_off(0, lane, phase, blocks), mine_lds + SLOT * i);
+        lds_copy16_at(base, q86_copy_off(1, lane, phase, blocks), mine_lds + SLOT * i + 1024);
     };
     if (n > 0)
         issue(0);
@@ -606,20 +604,6 @@ __global__ __launch_bounds__(64 * kQ86Waves) void k_gemv_q8k6(const uint8_t *__r
     const float s0 = a[0] + a[4], s1 = a[1] + a[5], s2 = a[2] + a[6], s3 = a[3] + a[7];
     if (lane == 0)
         out[row] = (s0 + s2) + (s1 + s3);
-}
-
-// Waves to a row: as many of 1, 2 (from 5 blocks on) and 4 (from 17) as one
-// round of the chip's waves has for every row.  (Two waves of a row of at most
-// eight blocks are one at work, in twice the workgroups.)  Measured on MI355X
-// (us, quantizing included, graph replays over weights in HBM, fewer / more
-// waves): 256 x 256 3.18 / 3.72, 256 x 512 3.21 / 3.34, 512 x 1024 3.50 / 3.56; 512 x 1280
-// 3.56 / 3.68, 512 x 2048 3.77 / 3.71; 512 x 5120 6.29 / 5.20, 1024 x 6144 6.75 / 5.76.
-static int q86_team(int nb, int outer, int ncu)
-{
-    int tw = 1;
-    while (tw < 4 && (int64_t)outer * 2 * tw <= (int64_t)ncu * kQ86Waves && nb > (tw == 1 ? 4 : 16))
-        tw *= 2;
-    return tw;
 }
 
 template <bool QX>

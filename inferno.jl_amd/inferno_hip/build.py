@@ -109,7 +109,8 @@ def build_checks(verbose: bool = False) -> Path:
     include the headers the kernels form their indices with and run on the CPU."""
     return _hipcc(CHECK_LIB, [CHECKS / "sdig_check.hip", CHECKS / "prefill_check.hip",
                               CHECKS / "prefill_plan_check.hip",
-                              CHECKS / "gemv_plan_check.hip", CHECKS / "mdig_check.hip"], verbose)
+                              CHECKS / "gemv_plan_check.hip", CHECKS / "mdig_check.hip",
+                              CHECKS / "prefill_copy_check.hip"], verbose)
 
 
 if __name__ == "__main__":

@@ -20,6 +20,7 @@
 // Built by inferno_hip.build into tests/native/_build/libsdig_check.so; called
 // from tests/test_gemv_plan.py through ctypes.
 #include "kq_gemv_plan.h"
+#include "kq_launch.h"
 
 #include <cstdarg>
 #include <cstdio>
@@ -198,5 +199,57 @@ extern "C" long long mdig_check(int type, int nblk, int outer, int gateup, int n
     case kIQ4_NL: walk<kIQ4_NL>(R, nblk, outer, gateup, norm, ncu, at, stats); break;
     default: R.fail("unknown type %d", type);
     }
+    return R.n;
+}
+
+// k_gemv_q8k6 (kq_q8k.hip): every row has a team and every item of a row one of
+// its waves, the copies read whole units inside W or the unit holding its last
+// byte, the bytes of each block lie in the slot where the lanes read them, and a
+// lane's dwords past its block stay in the slot.
+extern "C" long long q8k6_check(int nb, int outer, int ncu, char *msg, int cap)
+{
+    MReport R{msg, cap};
+    if (msg && cap > 0)
+        msg[0] = 0;
+    const int tw = q86_team(nb, outer, ncu), teams = kQ86Waves / tw, grid = (outer + teams - 1) / teams, ni = (nb + 7) / 8;
+    if (nb < 1 || nb > kQ86MaxBlocks || outer < 1 || outer > ncu * kQ86Waves || grid > ncu)
+        R.fail("%d rows of %d blocks: %d workgroups", outer, nb, grid);
+    std::vector<int> items((size_t)ni, 0);
+    for (int rank = 0; rank < tw; ++rank) {
+        const int n = (ni - rank + tw - 1) / tw;
+        if (n > kQ86Items)
+            R.fail("%d items for a wave", n);
+        for (int i = 0; i < n; ++i)
+            if (rank + tw * i >= ni)
+                R.fail("item %d of %d", rank + tw * i, ni);
+            else
+                items[(size_t)(rank + tw * i)]++;
+    }
+    for (int i = 0; i < ni; ++i)
+        if (items[(size_t)i] != 1)
+            R.fail("item %d is computed %d times", i, items[(size_t)i]);
+    const int64_t row_bytes = (int64_t)nb * 210, w_end = ((int64_t)outer * row_bytes + 15) / 16 * 16;
+    for (int row = 0; row < outer && R.n < 20; ++row)
+        for (int it = 0; it < ni; ++it) {
+            const int64_t at = row * row_bytes + it * 1680; // W itself is 16-byte aligned
+            const uint32_t phase = (uint32_t)(at & 15);
+            const int blocks = std::min(8, nb - 8 * it);
+            if (phase != (uint32_t)(row * row_bytes & 15))
+                R.fail("row %d item %d: not at its row's phase", row, it);
+            std::vector<int64_t> image(kQ86Slot, -1);
+            for (int i = 0; i < 2; ++i)
+                for (int l = 0; l < 64; ++l) {
+                    const int64_t src = at - phase + q86_copy_off(i, l, phase, blocks);
+                    if (src < 0 || src % 16 || src + 16 > w_end)
+                        R.fail("row %d item %d: bytes %lld.. of %lld", row, it, (long long)src, (long long)w_end);
+                    for (int b = 0; b < 16; ++b) image[(size_t)(1024 * i + 16 * l + b)] = src + b;
+                }
+            if (phase + 7 * 210 + 4 * 54 > (uint32_t)kQ86Slot)
+                R.fail("the last block's dwords leave the slot");
+            for (int s = 0; s < blocks; ++s)
+                for (int b = 0; b < 210; ++b)
+                    if (image[phase + 210u * (uint32_t)s + (uint32_t)b] != at + 210 * s + b)
+                        R.fail("row %d item %d block %d byte %d: not in the slot", row, it, s, b);
+        }
     return R.n;
 }

@@ -200,3 +200,12 @@ def test_matrix_core_launches_on_other_devices(plan, ncu):
     for t, outer, inner in ((Q6_K, 4099, 3840), (synth.Q8_0, 1031, 16352), (Q4_K, 2050, 8448), (Q5_K, 31, 256)):
         st = _mdig_walk(plan, t, outer, inner, ncu=ncu)
         assert st[1] * (-(-inner // 1024)) <= 512
+
+
+@pytest.mark.parametrize("nb", range(1, 25))
+def test_int8_q6_k_launches_stay_in_bounds(plan, nb):
+    plan.q8k6_check.restype = C.c_longlong
+    msg = C.create_string_buffer(512)
+    for outer in (1, 15, 17, 257, 1030):
+        for ncu in (80, 256):
+            assert plan.q8k6_check(nb, outer, ncu, msg, 512) == 0, f"{outer} rows: {msg.value.decode()}"

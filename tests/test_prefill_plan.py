@@ -63,3 +63,23 @@ def test_sweep(chk, ncu):
         for outer in (1, 64, 129, 512, 1000, 4096, 14336):
             for inner in (256, 1792, 2048, 2816, 4096, 8192, 16384):
                 chk(T, inner, outer, ncu)
+
+
+# the copies of the 128-token, the 32-token and the fp32-operand kernels through
+# the kernels' own functions (tests/native/prefill_copy_check.hip): kind, size
+@pytest.mark.parametrize("kind,size", [(0, 1), (0, 2), (1, 0), (2, 1), (2, 2)])
+@pytest.mark.parametrize("T,outer,inner", [(1, 1, 768), (31, 63, 1024), (33, 65, 1280), (127, 255, 768), (129, 257, 2304),
+                                           (2048, 12288, 4096), (257, 4100, 2560), (77, 9728, 2560), (509, 2047, 14336)])
+def test_copies_stay_in_bounds(chk, kind, size, T, outer, inner):
+    L, msg = C.CDLL(str(LIB)), C.create_string_buffer(512)
+    L.prefill_copy_check.restype = C.c_longlong
+    n = L.prefill_copy_check(kind, size, T, inner, outer, msg, 512)
+    assert n == 0, f"kind {kind} {T}x{inner}x{outer}: {n} violations, first: {msg.value.decode()}"
+
+
+@pytest.mark.parametrize("size", (1, 2))
+def test_copies_of_short_rows_stay_in_bounds(chk, size):
+    L, msg = C.CDLL(str(LIB)), C.create_string_buffer(512)
+    L.prefill_copy_check.restype = C.c_longlong
+    for T, outer, inner in ((1, 1, 256), (70, 130, 512)):  # one and two block columns: a wave half without any
+        assert L.prefill_copy_check(2, size, T, inner, outer, msg, 512) == 0, msg.value.decode()
