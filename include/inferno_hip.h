@@ -319,15 +319,17 @@ int ihip_prefill_convert_dev(const float *X, void *xh, int T, int inner, ihip_st
 int ihip_prefill_q4_k_xh_dev(const void *w, void *xh, float *Y, int T, int inner, int outer,
                              ihip_stream stream);
 /* The per-token prefill loop (src/ModelCPU.jl:1001-1017 over
- * mul_quant_mat_vec, :285-307) on fp32 operands: the weights dequantized to
- * fp32 exactly and X as given, multiplied on the fp32 matrix cores.  The
- * error is fp32 rounding, within 1e-4 * ||w_row|| * ||x|| for any finite X;
+ * mul_quant_mat_vec, :285-307) on fp32 operands: X as given and the exact
+ * weights, both in bf16 parts that hold every bit, multiplied on the bf16
+ * matrix cores and summed in fp32.  The error is fp32 rounding, within 1e-4 *
+ * ||w_row|| * ||x|| for any finite X (rows whose weights all but vanish beside
+ * their block scales excepted: their error is relative to the scales);
  * ihip_prefill_q4_k_dev (which takes this path for rows of at most 512
  * columns) rounds both operands of longer rows to fp16, which meets that
  * bound for the benchmark's data but not for every X (a token equal to a
  * weight row reaches 2-3x it) and needs every dequantized weight below
- * 65504 in magnitude.  Several times slower than the fp16 path on long rows;
- * no scratch.  w, X and Y are 16-byte aligned; T * outer < 2^31. */
+ * 65504 in magnitude.  Up to three times the time of the fp16 path on long
+ * rows; no scratch.  w, X and Y are 16-byte aligned; T * outer < 2^31. */
 int ihip_prefill_q4_k_f32_dev(const void *w, const float *X, float *Y, int T, int inner,
                               int outer, ihip_stream stream);
 

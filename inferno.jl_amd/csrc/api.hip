@@ -372,9 +372,10 @@ int resolve_locked(const void *host, int type, int inner, int outer, const void 
 }
 
 // Fast kernels need 16-byte aligned weights and x.  Rows of any whole number
-// of blocks qualify: the streamed Q6_K / Q8_0 / IQ4_NL kernel copies rows
-// that are not 16-byte multiples from the unit below each segment (which may
-// read up to 14 bytes past the weight's last byte, inside its 16-byte unit).
+// of blocks qualify: the kernels that stream Q6_K / Q8_0 / IQ4_NL rows through
+// LDS copy rows that are not 16-byte multiples from the unit below each piece
+// (which may read up to 14 bytes past the weight's last byte, inside its
+// 16-byte unit).
 bool fast_ok(int, const void *w, const float *x, int)
 {
     return al16(w) && al16(x);

@@ -30,7 +30,8 @@ inline bool kwide_one_row(int outer, int ncu) { return (outer + 7) / 8 <= ncu; }
 // Q6_K (streamed / this) 4096 x 12288 12.4 / 11.7, 2560 x 9728 12.1 / 7.9, 5120 x
 // 13824 26.9 / 15.9, 1024 x 4096 4.9 / 3.6, 12288 x 4096 10.8 / 10.8; Q8_0 5003 x
 // 2720 8.4 / 5.8, 2560 x 9728 11.2 / 8.3; IQ4_NL 5120 x 5120 10.7 / 6.8, 5003 x 2720
-// 8.8 / 5.1, 20000 x 6144 24.3 / 17.7.
+// 8.8 / 5.1, 20000 x 6144 24.3 / 17.7.  What going by length costs: few rows of Q5_K
+// (1024 x 2560 2.90 / 3.17, 1024 x 3072 2.92 / 3.17, 1024 x 1024 2.87 / 2.81).
 constexpr int kMdMaxSteps = 16, kMdMaxBlocks = 4 * kMdMaxSteps;
 constexpr bool mdig_takes(int type, int nblk, bool gateup)
 {

@@ -205,7 +205,13 @@ inline int prefill_wide_rows(int T, int inner, int outer, int ncu)
 // (k_prefill_q4k_thin): by the same estimate, fitted to 105 shapes of 8 to 1024
 // tokens timed in graph replays (relative rms 9 %; the split 64 x 128 tile 5 %).
 // Over them the choice is never over 2 % slower than without this kernel,
-// 1.13 times as fast on average and 0.2 % from the faster of the two.
+// 1.13 times as fast on average and 0.2 % from the faster of the two.  That is
+// on weights that the memory-side cache holds.  From HBM its gain is smaller,
+// and at 1 to 32 tokens some shapes lose (us, the product alone, 64 x 128 / thin;
+// held in the cache): 1 x 4096 x 4096 11.1 / 12.1 (11.9 / 11.0), 32 x 3584 x 3584 12.5
+// / 15.5 (12.5 / 11.7), 32 x 4096 x 6144 13.9 / 16.1 (14.0 / 12.5), 77 x 2560 x 9728
+// 16.3 / 17.4 (16.5 / 15.5); 32 x 2048 x 5632 11.7 / 9.8 (11.7 / 8.4), 128 x 4096 x 4096
+// 18.9 / 14.3 (17.8 / 12.4).
 constexpr int kPrefillThinBM = 32, kPrefillThinBN = 64;
 inline bool prefill_thin(int T, int inner, int outer, int ncu)
 {
