@@ -46,11 +46,13 @@ constexpr bool mdig_takes(int type, int nblk, bool gateup)
 
 // Q8_0 and IQ4_NL rows of whole 256-column units on the wide lane layout, by
 // length only (as mdig_takes).  Measured on MI355X (us, graph replays over weights
-// in HBM, wide / k_gemv_mdig): Q8_0 4096 x 4096 5.9 / 6.1, 2048 x 2048 3.0 / 3.3, 9728 x
-// 2560 8.0 / 7.6 (the one length lost); IQ4_NL 4096 x 4096 5.0 / 5.4, 1024 x 3584 3.18 /
-// 3.52, 4096 x 3328 4.81 / 5.21, 12288 x 3328 9.80 / 9.37, and where k_gemv_mdig has it
-// 1024 x 2560 3.21 / 3.35, 2048 x 3072 3.64 / 3.76, 4096 x 3072 4.72 / 4.44, 12288 x 2560
-// 9.50 / 7.54.  IQ4_NL rows too long for the others too (4096 x 20480).
+// in HBM, wide / k_gemv_mdig): Q8_0 1024 x 4096 3.41 / 3.63, 4096 x 4096 5.97 / 6.10,
+// 12288 x 4096 11.45 / 12.01, 2048 x 2560 3.41 / 3.79, 8192 x 2560 6.93 / 6.96, 2048 x
+// 2048 3.37 / 3.65, 12288 x 2048 7.66 / 7.59, 1024 x 1024 2.90 / 2.94, and many rows of
+// 1024 columns the other way (12288 6.98 / 5.08); IQ4_NL 4096 x 4096 5.0 / 5.4, 1024 x
+// 3584 3.18 / 3.52, 4096 x 3328 4.81 / 5.21, 12288 x 3328 9.80 / 9.37, and where
+// k_gemv_mdig has it 1024 x 2560 3.21 / 3.35, 2048 x 3072 3.64 / 3.76, 4096 x 3072 4.72 /
+// 4.44, 12288 x 2560 9.50 / 7.54.  IQ4_NL rows too long for the others too (4096 x 20480).
 inline bool b32_takes_wide(int type, int inner)
 {
     if (inner % 256)
