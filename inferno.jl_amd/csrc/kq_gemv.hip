@@ -16,9 +16,10 @@
 // `dmin*m` term of Q4_K/Q5_K and the weight offsets of Q6_K / Q8_0 / IQ4_NL
 // are taken off through per-sub-block sums of x that all rows share.
 //
-//   * Q4_K / Q5_K rows that fill 16 blocks ("wide" kernels, k_gemv_kwide /
-//     k_gemv_kpers): blocks are 16-byte multiples, so lanes load straight from
-//     HBM with 128-bit loads.  A wave covers 16 blocks (4096 columns) of R rows
+//   * Q4_K rows of at most 16 blocks, the longer Q5_K ones of them, and Q8_0 /
+//     IQ4_NL rows in their lane layout ("wide" kernels, k_gemv_kwide /
+//     k_gemv_kpers; the lines stand in kq_gemv_plan.h): blocks are 16-byte
+//     multiples, so lanes load straight from HBM with 128-bit loads.  A wave covers 16 blocks (4096 columns) of R rows
 //     per pass: lane = (block, sub-block pair), 64 weights per lane per row.
 //   * All other rows of at most 16384 columns (k_gemv_mdig): four rows x 1024
 //     columns a step through a private LDS ring per wave, filled by gfx950's
